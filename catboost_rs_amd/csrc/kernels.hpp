@@ -250,8 +250,10 @@ static __global__ __launch_bounds__(256) void prepare_kernel(
     double* __restrict__ sstat /* [n][K+1] */, int newton,
     unsigned long long* __restrict__ partials /* [gridDim.x][kPartials] */,
     const double* __restrict__ ext_der /* nullable [2][n]: der1, der2 of a pair loss */,
-    const double* __restrict__ score_w /* nullable [n]: histogram weight (pairwise weights) */) {
+    const double* __restrict__ score_w /* nullable [n]: histogram weight (pairwise weights) */,
+    uint32_t* __restrict__ gcnt /* the partition's group counts, cleared for the tree */, uint32_t n_gcnt) {
     constexpr int C = K + 1;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_gcnt; i += gridDim.x * blockDim.x) gcnt[i] = 0;
     __shared__ unsigned long long red[4][kPartials];
     unsigned long long acc[kPartials] = {0, 0, 0, 0, 0, 0, 0, 0};
     const double bscale = (double)(1 << kBoundShift);
@@ -2754,17 +2756,19 @@ __global__ __launch_bounds__(512) void score_chain_kernel(
     }
 }
 
-// Level argmax over features in enumeration order (floats ascending, then one-hot
-// columns ascending); strict first-wins.  One workgroup of 1024 threads.
-static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __restrict__ best_score,
-                                                      const uint32_t* __restrict__ best_bin,
-                                                      const uint8_t* __restrict__ one_hot,
-                                                      uint32_t F, SplitRec* __restrict__ out) {
-    __shared__ double rs[16];
-    __shared__ uint32_t rk[16];
+// Level argmax over features in enumeration order (floats ascending, then one-hot columns
+// ascending); strict first-wins.  Every thread of the workgroup calls it (one barrier); the
+// result is returned to every thread.
+template <uint32_t NT>
+__device__ __forceinline__ SplitRec block_argmax(const double* __restrict__ best_score,
+                                                 const uint32_t* __restrict__ best_bin,
+                                                 const uint8_t* __restrict__ one_hot, uint32_t F) {
+    constexpr uint32_t NW = NT / 64;
+    __shared__ double rs[NW];
+    __shared__ uint32_t rk[NW];
     double s = -INFINITY;
     uint32_t key = 0xFFFFFFFFu;
-    for (uint32_t f = threadIdx.x; f < F; f += blockDim.x) {
+    for (uint32_t f = threadIdx.x; f < F; f += NT) {
         const double v = best_score[f];
         const uint32_t k = f + ((one_hot && one_hot[f]) ? F : 0u);
         if (v > s || (v == s && k < key)) {
@@ -2786,36 +2790,61 @@ static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __res
         rk[wave] = key;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t nw = (blockDim.x + 63) / 64;
-        for (uint32_t k = 1; k < nw; ++k)
-            if (rs[k] > s || (rs[k] == s && rk[k] < key)) {
-                s = rs[k];
-                key = rk[k];
-            }
-        SplitRec r;
-        r.valid = (s > -INFINITY) ? 1u : 0u;
-        r.feature = key == 0xFFFFFFFFu ? 0u : (key >= F ? key - F : key);
-        r.one_hot = (key != 0xFFFFFFFFu && key >= F) ? 1u : 0u;
-        r.bin = r.valid ? best_bin[r.feature] : 0u;
-        r.score = s;
-        *out = r;
-    }
+    s = rs[0];
+    key = rk[0];
+#pragma unroll
+    for (uint32_t k = 1; k < NW; ++k)
+        if (rs[k] > s || (rs[k] == s && rk[k] < key)) {
+            s = rs[k];
+            key = rk[k];
+        }
+    SplitRec r;
+    r.valid = (s > -INFINITY) ? 1u : 0u;
+    r.feature = key == 0xFFFFFFFFu ? 0u : (key >= F ? key - F : key);
+    r.one_hot = (key != 0xFFFFFFFFu && key >= F) ? 1u : 0u;
+    r.bin = r.valid ? best_bin[r.feature] : 0u;
+    r.score = s;
+    return r;
+}
+
+// The argmax as a launch of its own: for tables wider than kArgmaxFuse features.
+static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __restrict__ best_score,
+                                                             const uint32_t* __restrict__ best_bin,
+                                                             const uint8_t* __restrict__ one_hot, uint32_t F,
+                                                             SplitRec* __restrict__ out) {
+    const SplitRec r = block_argmax<1024>(best_score, best_bin, one_hot, F);
+    if (threadIdx.x == 0) *out = r;
 }
 
 // ---------------------------------------------------------------------------------
 // Stable partition by leaf.
-//   split_count: leaf |= pass << level for every row; per-block counts of sampled rows
-//                per new leaf -> cnt[leaf][block]
-//   plan_scan:   per leaf, exclusive scan over blocks (in place) + total
-//   compact:     the plan (smaller child per parent, ties -> the TRUE child, tree.rs:1109,
-//                and the segment offsets of the next fill) from the totals, then the rows
-//                of the built children written in ascending row order per segment;
-//                inside a block, ranks come from wave ballots (match on the key bits) and
-//                mbcnt, across waves from per-wave counts in LDS.
+//   split_count: the level's argmax, then leaf |= pass << level for every row; counts of sampled
+//                rows per new leaf of every wave (cnt[wave][leaf]) and of every group of
+//                kGroupBlocks workgroups (gcnt[group][leaf], added atomically)
+//   compact:     leaf totals and the rows before this workgroup from the group counts and its
+//                own group's wave counts; the plan (smaller child per parent, ties -> the TRUE
+//                child, tree.rs:1109, and the segment offsets of the next fill) from the totals;
+//                then the rows of the built children written in ascending row order per
+//                segment; inside a block, ranks come from wave ballots (match on the key bits)
+//                and mbcnt, across waves from per-wave counts in LDS.
+// A dependent launch costs 4.6-5.7 us whatever it does, so the argmax (a workgroup over F scores)
+// and the scan of the counts ride in the kernels that need their results: each workgroup of
+// split_count repeats the argmax, each workgroup of compact sums the counts before it.
 // ---------------------------------------------------------------------------------
 constexpr uint32_t kPartRows = 4096;   // rows per partition block (4 waves)
 constexpr uint32_t kPartWaveRows = kPartRows / 4;
+// Workgroups a group of the counts covers: compact reads groups + 4 kGroupBlocks counts per leaf
+// (10M rows: 153 + 64), and a group count takes kGroupBlocks atomics on one address (about 66 ns
+// each, one after another, 1 us in all).
+constexpr uint32_t kGroupBlocks = 16;
+__host__ __device__ inline uint32_t part_groups(uint32_t n_blocks) { return (n_blocks + kGroupBlocks - 1) / kGroupBlocks; }
+// Group counts of level l of a tree: [group][2 << l], the levels one after another.
+__host__ __device__ inline size_t group_count_off(uint32_t groups, uint32_t level) {
+    return (size_t)groups * ((2u << level) - 2u);
+}
+// Features up to which split_count's workgroups repeat the argmax (256 threads over F scores, at
+// most 16 each); wider tables launch argmax_kernel.
+constexpr uint32_t kArgmaxFuse = 4096;
 
 // Lanes of this wave whose key equals mine (valid lanes only): one ballot per key bit.
 __device__ __forceinline__ uint64_t wave_peers(uint32_t key, bool valid, uint32_t nbits) {
@@ -2827,22 +2856,23 @@ __device__ __forceinline__ uint64_t wave_peers(uint32_t key, bool valid, uint32_
     return mask;
 }
 
-// Leaf update of one level and the per-wave row counts of every new leaf.  Each wave owns
-// kPartWaveRows consecutive rows; its counts go to cnt[leaf][wave].  Up to 4 new leaves a
+// Leaf update of one level and the row counts of every new leaf.  Each wave owns kPartWaveRows
+// consecutive rows; its counts go to cnt[wave][leaf].  Up to 4 new leaves a
 // leader per distinct leaf adds the popcount of its peers (one ballot per key bit, so no LDS
 // cell takes more than one add per 64 rows); with more leaves every row adds 1 to its leaf's
 // LDS counter (few lanes share a counter, and the ballots would grow with the level).
+// kArgmax: the level's split is the argmax of the features' best candidates, taken by every
+// workgroup while its rows' leaves load (workgroup 0 stores it); else it is read from *split.
+template <bool kArgmax>
 static __global__ __launch_bounds__(256) void split_count_kernel(
-    const uint8_t* __restrict__ cols, uint64_t n, const SplitRec* __restrict__ split,
-    uint32_t level, uint16_t* __restrict__ leaf, uint32_t* __restrict__ cnt, uint32_t n_waves,
-    int write_counts) {
+    const uint8_t* __restrict__ cols, uint64_t n, SplitRec* __restrict__ split,
+    const double* __restrict__ best_score, const uint32_t* __restrict__ best_bin,
+    const uint8_t* __restrict__ one_hot, uint32_t F, uint32_t level, uint16_t* __restrict__ leaf,
+    uint32_t* __restrict__ cnt, uint32_t* __restrict__ gcnt /* nullable: no counts */) {
     __shared__ uint32_t c[4][kMaxLeaves];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t n_new = 2u << level;
     for (uint32_t k = lane; k < n_new; k += 64) c[wave][k] = 0;
-    __syncthreads();
-    const SplitRec s = *split;
-    const uint8_t* col = cols + (size_t)s.feature * n;
     const uint64_t wid = (uint64_t)blockIdx.x * 4 + wave;
     const uint64_t beg = wid * kPartWaveRows;
     const uint64_t end = min(beg + kPartWaveRows, n);
@@ -2853,8 +2883,21 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint64_t i = beg + (uint64_t)u * 64 + lane;
-        bin[u] = i < end ? col[i] : 0u;
         lf[u] = i < end ? leaf[i] : 0x8000u;
+    }
+    SplitRec s;
+    if (kArgmax) {
+        s = block_argmax<256>(best_score, best_bin, one_hot, F);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *split = s;
+    } else {
+        s = *split;
+    }
+    __syncthreads();
+    const uint8_t* col = cols + (size_t)s.feature * n;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint64_t i = beg + (uint64_t)u * 64 + lane;
+        bin[u] = i < end ? col[i] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -2863,7 +2906,7 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
         const bool pass = s.one_hot ? bin[u] == s.bin : bin[u] > s.bin;
         lf[u] |= (uint32_t)pass << level;
         if (in) leaf[i] = (uint16_t)lf[u];
-        if (write_counts) {
+        if (gcnt) {
             const bool valid = in && !(lf[u] & 0x8000u);
             if (level >= 2) {   // uniform
                 if (valid) atomicAdd(&c[wave][lf[u]], 1u);
@@ -2873,69 +2916,14 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
             }
         }
     }
-    if (!write_counts) return;
-    for (uint32_t k = lane; k < n_new; k += 64) cnt[(size_t)k * n_waves + wid] = c[wave][k];
-}
-
-static __global__ __launch_bounds__(1024) void plan_scan_kernel(uint32_t* __restrict__ cnt,
-                                                         uint32_t n_blocks,
-                                                         uint32_t* __restrict__ totals) {
-    __shared__ uint32_t sh[128];   // [0, 16): wave totals, [64, 80): their exclusive prefix
-    uint32_t* row = cnt + (size_t)blockIdx.x * n_blocks;
-    const uint32_t per = (n_blocks + blockDim.x - 1) / blockDim.x;
-    const uint32_t b0 = threadIdx.x * per;
-    uint32_t local = 0;
-    constexpr uint32_t kBatch = 8;   // loads in flight per thread
-    for (uint32_t k0 = 0; k0 < per; k0 += kBatch) {
-        uint32_t v[kBatch];
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; ++q) {
-            const uint32_t k = k0 + q;
-            v[q] = (k < per && b0 + k < n_blocks) ? row[b0 + k] : 0u;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; ++q) local += v[q];
-    }
-    // inclusive scan of the threads' sums: within each wave by shuffles, then over the wave
-    // totals by wave 0 (two barriers)
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
-    uint32_t inc = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(inc, o, 64);
-        if (lane >= (uint32_t)o) inc += u;
-    }
-    if (lane == 63) sh[wave] = inc;
+    if (!gcnt) return;
+    for (uint32_t k = lane; k < n_new; k += 64) cnt[wid * n_new + k] = c[wave][k];
     __syncthreads();
-    if (wave == 0) {
-        const uint32_t t = lane < n_waves ? sh[lane] : 0u;
-        uint32_t wi = t;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(wi, o, 64);
-            if (lane >= (uint32_t)o) wi += u;
-        }
-        if (lane < n_waves) sh[64 + lane] = wi - t;   // exclusive prefix of the wave totals
+    uint32_t* g = gcnt + (size_t)(blockIdx.x / kGroupBlocks) * n_new;
+    for (uint32_t k = threadIdx.x; k < n_new; k += 256) {
+        const uint32_t t = c[0][k] + c[1][k] + c[2][k] + c[3][k];
+        if (t) atomicAdd(g + k, t);
     }
-    __syncthreads();
-    uint32_t run = sh[64 + wave] + inc - local;  // exclusive prefix of this thread's range
-    for (uint32_t k0 = 0; k0 < per; k0 += kBatch) {
-        uint32_t v[kBatch];
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; ++q) {
-            const uint32_t k = k0 + q;
-            v[q] = (k < per && b0 + k < n_blocks) ? row[b0 + k] : 0u;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kBatch; ++q) {
-            const uint32_t k = k0 + q;
-            if (k < per && b0 + k < n_blocks) {
-                row[b0 + k] = run;
-                run += v[q];
-            }
-        }
-    }
-    if (threadIdx.x == blockDim.x - 1) totals[blockIdx.x] = sh[64 + wave] + inc;
 }
 
 // Stable compaction of the rows of every directly built child into idx (grouped by parent in
@@ -2948,11 +2936,13 @@ static __global__ __launch_bounds__(1024) void plan_scan_kernel(uint32_t* __rest
 // of its rows in order instead of gathering them.
 // The level's plan (the smaller child of every parent, ties to the TRUE child, tree.rs:1109, and
 // the segment offsets of the next fill) comes from the children's totals: every block derives it
-// (at most 128 parents, one wave) and block 0 stores it for the kernels after.
+// (at most 128 parents, one wave) and block 0 stores it for the kernels after.  The totals and
+// the rows before a block are sums of the groups' counts and of its own group's wave counts
+// (integers: the order does not matter), read while the block's leaf ids load.
 template <int SPW>
 static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __restrict__ leaf, uint64_t n,
                                                       uint32_t level, const uint32_t* __restrict__ cnt,
-                                                      uint32_t n_waves, const uint32_t* __restrict__ totals,
+                                                      const uint32_t* __restrict__ gcnt, uint32_t n_groups,
                                                       LevelPlan* __restrict__ plan,
                                                       uint32_t* __restrict__ idx,
                                                       const unsigned long long* __restrict__ sp_in,
@@ -2960,9 +2950,50 @@ static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __r
     __shared__ uint32_t run[4][kMaxLeaves / 2];
     __shared__ uint32_t built[kMaxLeaves / 2];
     __shared__ uint32_t segb[kMaxLeaves / 2];
+    __shared__ uint32_t tot[kMaxLeaves], pre[kMaxLeaves];   // rows of a new leaf; those before this block
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t n_parent = 1u << level;
+    const uint32_t n_parent = 1u << level, n_new = 2u << level;
     const uint64_t wid = (uint64_t)blockIdx.x * 4 + wave;
+    const uint64_t beg = wid * kPartWaveRows;
+    const uint64_t end = min(beg + kPartWaveRows, n);
+    constexpr int U = kPartWaveRows / 64;
+    uint32_t lfs[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {   // all loads in flight before the first use
+        const uint64_t i = beg + (uint64_t)u * 64 + lane;
+        lfs[u] = i < end ? leaf[i] : 0x8000u;
+    }
+    static_assert(kMaxLeaves == 256, "a thread's counts are all of one leaf (n_new divides 256)");
+    if (threadIdx.x < n_new) {
+        tot[threadIdx.x] = 0;
+        pre[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    {
+        const uint32_t group = blockIdx.x / kGroupBlocks;
+        const uint32_t w0 = group * kGroupBlocks * 4, w1 = blockIdx.x * 4;   // its group's waves before this block
+        uint32_t t = 0, p = 0;
+        const uint32_t cells = n_groups * n_new, before = group * n_new;
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < cells; i += 256) {
+            const uint32_t v = gcnt[i];
+            t += v;
+            p += i < before ? v : 0u;
+        }
+        const uint32_t* own = cnt + (size_t)w0 * n_new;
+        const uint32_t own_cells = (w1 - w0) * n_new;
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < own_cells; i += 256) p += own[i];
+        for (uint32_t o = n_new; o < 64; o <<= 1) {   // a wave's lanes of one leaf
+            t += __shfl_xor(t, o, 64);
+            p += __shfl_xor(p, o, 64);
+        }
+        if (lane < n_new) {
+            atomicAdd(&tot[threadIdx.x & (n_new - 1u)], t);
+            atomicAdd(&pre[threadIdx.x & (n_new - 1u)], p);
+        }
+    }
+    __syncthreads();
     static_assert(kMaxLeaves / 2 <= 128, "two parents per lane of one wave");
     if (wave == 0) {
         uint32_t sz[2], inc[2];
@@ -2971,7 +3002,7 @@ static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __r
             const uint32_t p = lane + 64u * q;
             sz[q] = 0;
             if (p < n_parent) {
-                const uint32_t nf = totals[p], nt = totals[p + n_parent];
+                const uint32_t nf = tot[p], nt = tot[p + n_parent];
                 const bool true_smaller = nt <= nf;
                 built[p] = true_smaller ? p + n_parent : p;
                 sz[q] = true_smaller ? nt : nf;
@@ -3003,18 +3034,13 @@ static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __r
         }
     }
     __syncthreads();
-    for (uint32_t p = lane; p < n_parent; p += 64)
-        run[wave][p] = segb[p] + cnt[(size_t)built[p] * n_waves + wid];
-    __syncthreads();
-    const uint64_t beg = wid * kPartWaveRows;
-    const uint64_t end = min(beg + kPartWaveRows, n);
-    constexpr int U = kPartWaveRows / 64;
-    uint32_t lfs[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {   // all loads in flight before the first use
-        const uint64_t i = beg + (uint64_t)u * 64 + lane;
-        lfs[u] = i < end ? leaf[i] : 0x8000u;
+    for (uint32_t p = lane; p < n_parent; p += 64) {
+        const uint32_t lf = built[p];
+        uint32_t r = segb[p] + pre[lf];
+        for (uint32_t w = 0; w < wave; ++w) r += cnt[(size_t)(blockIdx.x * 4 + w) * n_new + lf];
+        run[wave][p] = r;
     }
+    __syncthreads();
     // listed rows: key = parent, valid = the row lies in its parent's directly built child
     uint32_t vmask = 0;   // validity bit per u
     uint32_t key_of[U];

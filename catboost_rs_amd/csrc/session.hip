@@ -130,9 +130,9 @@ struct cbh_session {
     uint32_t* idx = nullptr;
     long long* hist[2] = {nullptr, nullptr};
     size_t hist_cells_max = 0;
-    uint32_t* cnt = nullptr;
-    uint32_t* totals = nullptr;
-    uint32_t n_part_blocks = 0;
+    uint32_t* cnt = nullptr;         // partition: row counts [wave][leaf] of the level
+    uint32_t* gcnt = nullptr;        // [level][group][leaf], cleared once per tree
+    uint32_t n_part_blocks = 0, n_groups_part = 0;
     LevelPlan* plans = nullptr;   // [depth]
     SplitRec* splits = nullptr;   // [depth]
     double* best_score = nullptr;
@@ -295,7 +295,7 @@ struct cbh_session {
     void release() {
         dfree(rows); dfree(cols); dfree(weight); dfree(target); dfree(approx); dfree(sstat);
         dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(cnt);
-        dfree(totals); dfree(best_score);
+        dfree(gcnt); dfree(best_score);
         dfree(best_bin); dfree(n_cand); dfree(one_hot); dfree(scales);
         dfree(leaf_sums); dfree(leaf_scaled); dfree(jump);
         dfree(out_dev);
@@ -424,8 +424,11 @@ int session_alloc(cbh_session* s) {
     CHECK(dalloc(&s->hist[0], s->hist_cells_max));
     CHECK(dalloc(&s->hist[1], s->hist_cells_max));
     s->n_part_blocks = (uint32_t)((n + kPartRows - 1) / kPartRows);
-    CHECK(dalloc(&s->cnt, ((size_t)s->n_part_blocks * 4) << s->depth));   // [leaf][wave]
-    CHECK(dalloc(&s->totals, (size_t)1 << s->depth));
+    // per level of up to 2^(depth - 1) new leaves: counts [wave][leaf], and per group of
+    // workgroups [level][group][leaf]
+    CHECK(dalloc(&s->cnt, ((size_t)s->n_part_blocks * 4) << (s->depth - 1)));
+    s->n_groups_part = part_groups(s->n_part_blocks);
+    CHECK(dalloc(&s->gcnt, group_count_off(s->n_groups_part, s->depth - 1) + 1));
     {   // one block for the per-tree results, sections 256-byte aligned
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         const size_t o_plans = up(sizeof(SplitRec) * s->depth);
@@ -1440,8 +1443,6 @@ int pairwise_level(cbh_session* s, const long long* cur, uint32_t level) {
     }
     pairwise_best_kernel<<<F, 256, 0, st>>>(s->cand_scores, s->n_cand, B, s->best_score, s->best_bin);
     HIP_TRY(hipGetLastError());
-    argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, nullptr, F, s->splits + level);
-    HIP_TRY(hipGetLastError());
     return CBH_OK;
 }
 
@@ -1595,7 +1596,8 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         n, loss, s->approx, s->target, s->weight, s->leaf,
         apply_prev && !s->ranking ? s->leaf_scaled : nullptr,   // a pair loss applied them above
         s->smp_dev, s->jt(), use_host_sample ? s->host_sample : nullptr, s->sstat, newton, s->partials,
-        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr);
+        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, s->gcnt,
+        (uint32_t)group_count_off(s->n_groups_part, s->depth - 1));
     HIP_TRY(hipGetLastError());
     scales_kernel<<<1, 256, 0, st>>>(s->partials, pgrid, s->bounds, s->scales,
                                      (s->packed || s->pkk) ? s->pack_bits : 0, s->count ? 1 : 0);
@@ -1828,29 +1830,32 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                                                     s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
         HIP_TRY(hipGetLastError());
-        if (!s->pairwise) {
-            argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, s->one_hot, s->F, s->splits + level);
+        const bool fuse_argmax = s->F <= kArgmaxFuse;
+        if (!fuse_argmax) {
+            argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F,
+                                              s->splits + level);
             HIP_TRY(hipGetLastError());
         }
         CHECK(s->stage_end());
         // ---- partition ----
         CHECK(s->stage_begin(kStPartition));
         const bool last = level + 1 == s->depth;
-        split_count_kernel<<<NB, 256, 0, st>>>(s->cols, n, s->splits + level, level, s->leaf, s->cnt,
-                                               4 * NB, last ? 0 : 1);
+        uint32_t* gcnt = last ? nullptr : s->gcnt + group_count_off(s->n_groups_part, level);
+        (fuse_argmax ? split_count_kernel<true> : split_count_kernel<false>)<<<NB, 256, 0, st>>>(
+            s->cols, n, s->splits + level, s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F, level,
+            s->leaf, s->cnt, gcnt);
         HIP_TRY(hipGetLastError());
         if (!last) {
-            plan_scan_kernel<<<2u << level, 1024, 0, st>>>(s->cnt, 4 * NB, s->totals);
-            HIP_TRY(hipGetLastError());
+            const uint32_t ng = s->n_groups_part;
             if (s->packed || s->count)   // the listed rows' packed statistic
-                compact_kernel<1><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, 4 * NB, s->totals, s->plans + level,
-                                                      s->idx, s->spack, s->sseq);
+                compact_kernel<1><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
+                                                      s->spack, s->sseq);
             else if (s->tiled && s->sseq)   // both f64 score channels of the listed rows
-                compact_kernel<2><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, 4 * NB, s->totals, s->plans + level,
-                                                      s->idx, (const unsigned long long*)s->sstat, s->sseq);
+                compact_kernel<2><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
+                                                      (const unsigned long long*)s->sstat, s->sseq);
             else
-                compact_kernel<0><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, 4 * NB, s->totals, s->plans + level,
-                                                      s->idx, nullptr, nullptr);
+                compact_kernel<0><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
+                                                      nullptr, nullptr);
             HIP_TRY(hipGetLastError());
         }
         CHECK(s->stage_end());
@@ -2229,7 +2234,7 @@ int cbh_session_read_approx(cbh_session* s, double* approx_out, uint64_t n_times
             prepare_kernel<K><<<grid_for(s->n, 256, kPrepBlocks), 256, 0, s->stream>>>(
                 s->n, s->cfg.loss == CBH_LOSS_RMSE ? 0 : 1, s->approx, s->target, s->weight, s->leaf,
                 s->leaf_scaled, s->smp_dev + 1, s->jt(), nullptr, s->sstat, 0, s->partials, nullptr,
-                nullptr);
+                nullptr, nullptr, 0u);
             HIP_TRY(hipGetLastError());
             return CBH_OK;
         });
