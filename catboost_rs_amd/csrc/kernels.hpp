@@ -644,7 +644,7 @@ static __global__ __launch_bounds__(1024) void fill_kernel(
     while (pos < re) {
         const uint32_t seg_end = (idx && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
         const uint32_t end = min(re, seg_end);
-        const uint32_t slot = idx ? plan->built[seg] : 0u;
+        const uint32_t slot = seg;
         if (end > pos) {
             fill_range<C, kSkip, CU>(rows, stride, idx, sfix, pos, end, w0, TW, plane, (unsigned long long*)lds, fl);
             __syncthreads();
@@ -1131,7 +1131,7 @@ static __global__ __launch_bounds__(kPackThreads) void fill_packed_kernel(
     while (pos < re) {
         const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
         const uint32_t end = min(re, seg_end);
-        const uint32_t slot = kGather ? plan->built[seg] : 0u;
+        const uint32_t slot = seg;
         if (end > pos) {
             if (kGather || !narrow)
                 packed_range<kGather, kCount>(pk, rbase, sh, wl4, wl, ibase, sbase, pos, end, (uint32_t)n, r0, off8,
@@ -1540,7 +1540,7 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
     while (pos < re) {
         const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
         const uint32_t end = min(re, seg_end);
-        const uint32_t slot = kGather ? plan->built[seg] : 0u;
+        const uint32_t slot = seg;
         if (end > pos) {
             if (!narrow && sets == 4)
                 exact_range<kGather, 4>(ex, rbase, sh, wl4, 8u * (l >> 3), l, ibase, sbase, seq, pos, end,
@@ -1678,7 +1678,7 @@ static __global__ __launch_bounds__(kPkkThreads) void fill_pkk_kernel(
         const uint32_t seg_lo = kGather ? plan->seg_begin[seg] : 0u;
         const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
         const uint32_t end = min(re, seg_end);
-        const uint32_t slot = kGather ? plan->built[seg] : 0u;
+        const uint32_t slot = seg;
         if (end > pos) {
             // blocks of 128 rows (one per row slot), two register sets SA and SB in flight: the
             // words and statistics of a block are loaded two blocks ahead, gathered row indices
@@ -1899,7 +1899,7 @@ static __global__ __launch_bounds__(kPkkThreads) void fill_pks_kernel(
         const uint32_t seg_lo = kGather ? plan->seg_begin[seg] : 0u;
         const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
         const uint32_t end = min(re, seg_end);
-        const uint32_t slot = kGather ? plan->built[seg] : 0u;
+        const uint32_t slot = seg;
         if (end > pos) {
             // blocks of 64 rows (one per DPP row); lane j < NP of a DPP row loads plane j of the
             // row's statistics
@@ -2075,59 +2075,74 @@ static __global__ void pack_stats_count_kernel(const double* __restrict__ sstat,
 
 // Histograms are kept in PREFIX form over bins (cell b holds the sum of bins 0..b): the
 // split scorer then reads FALSE = prefix[b], TRUE = prefix[B-1] - prefix[b] directly, and
-// the sibling subtraction stays valid because the prefix is linear.  This pass turns the
-// directly built children of a level (raw sums from the fill) into prefix form: one wave per
-// (child, channel, feature) row, each lane scanning up to 4 consecutive bins.
-// With `parent` given (levels >= 1) the same wave then writes the sibling row, parent - built,
-// both in prefix form (the subtraction is linear), so no separate derive pass is needed.
-static __global__ __launch_bounds__(256) void hist_prefix_kernel(long long* __restrict__ hist,
-                                                                 const LevelPlan* __restrict__ plan,
-                                                                 uint32_t n_built, uint32_t C, uint32_t F,
-                                                                 uint32_t B,
-                                                                 const long long* __restrict__ parent,
-                                                                 const uint32_t* __restrict__ skip_bin,
-                                                                 const long long* __restrict__ seg_tot) {
+// the sibling subtraction stays valid because the prefix is linear.  The fill adds the raw sums of
+// the directly built children into a buffer of their own, raw[segment][ch][f][bin], which is
+// zero outside a level's fill and its finishing: whoever reads a cell clears it, so no launch
+// or pass zeroes histograms.  The finishing turns a raw row into the prefix row of its child
+// and, with `parent` given (levels >= 1), writes the sibling's row, parent - built, both in
+// prefix form.  One wave per (child, channel, feature) row, each lane scanning up to 4
+// consecutive bins.
+struct PrefixRow {
+    long long v[4];
+    // the raw bins of this lane, cleared
+    __device__ __forceinline__ void take(long long* __restrict__ raw, uint32_t b0, uint32_t E, uint32_t B) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            const uint32_t b = b0 + e;
+            const bool in = e < E && b < B;
+            v[e] = in ? raw[b] : 0;
+            if (in) raw[b] = 0;
+        }
+    }
+    // inclusive prefix over the wave's bins; a dominant bin d the fill left out (its cell still 0)
+    // is rebuilt as the segment's channel total minus the other bins, i.e. every prefix from that
+    // bin on grows by it
+    __device__ __forceinline__ void scan(uint32_t lane, uint32_t b0, uint32_t d, uint32_t B, const long long* tot) {
+#pragma unroll
+        for (uint32_t e = 1; e < 4; ++e) v[e] += v[e - 1];
+        const long long run = v[3];
+        long long incl = run;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const long long u = __shfl_up(incl, o, 64);
+            if (lane >= (uint32_t)o) incl += u;
+        }
+        const long long off = incl - run;
+        long long dv = 0;
+        if (d < B) dv = *tot - __shfl(incl, 63, 64);   // d: the same in every lane
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) v[e] += off + (b0 + e >= d ? dv : 0);
+    }
+};
+
+static __global__ __launch_bounds__(256) void hist_prefix_kernel(
+    long long* __restrict__ raw, long long* __restrict__ hist, const LevelPlan* __restrict__ plan, uint32_t n_built,
+    uint32_t C, uint32_t CU /* channels finished, 0 .. CU-1 */, uint32_t F, uint32_t B,
+    const long long* __restrict__ parent, const uint32_t* __restrict__ skip_bin,
+    const long long* __restrict__ seg_tot) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t row = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const uint64_t rows = (uint64_t)n_built * C * F;
+    const uint64_t rows = (uint64_t)n_built * CU * F;
     if (row >= rows) return;   // wave-uniform
-    const uint32_t seg = (uint32_t)(row / ((uint64_t)C * F));
-    const uint32_t rem = (uint32_t)(row - (uint64_t)seg * C * F);
-    const uint32_t slot = plan ? plan->built[seg] : 0u;
-    long long* h = hist + ((size_t)slot * C * F + rem) * B;
+    const uint32_t seg = (uint32_t)(row / ((uint64_t)CU * F));
+    const uint32_t rem = (uint32_t)(row - (uint64_t)seg * CU * F);   // ch * F + f
     const uint32_t E = (B + 63) / 64;   // bins per lane, <= 4
     const uint32_t b0 = lane * E;
-    long long v[4];
-    long long run = 0;
-#pragma unroll
-    for (uint32_t e = 0; e < 4; ++e) {
-        const uint32_t b = b0 + e;
-        v[e] = (e < E && b < B) ? h[b] : 0;
-        run += v[e];
-        v[e] = run;
-    }
-    long long incl = run;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const long long u = __shfl_up(incl, o, 64);
-        if (lane >= (uint32_t)o) incl += u;
-    }
-    const long long off = incl - run;
-    // a dominant bin the fill left out (its cell still 0) is rebuilt as the segment's channel
-    // total minus the other bins, i.e. every prefix from that bin on grows by it
-    long long dv = 0;
+    PrefixRow r;
+    r.take(raw + ((size_t)seg * C * F + rem) * B, b0, E, B);
+    const uint32_t slot = plan ? plan->built[seg] : 0u;
+    long long* h = hist + ((size_t)slot * C * F + rem) * B;
     uint32_t d = B;
+    const long long* tot = nullptr;
     if (skip_bin) {
         const uint32_t ch = rem / F, f = rem - ch * F;
         d = skip_bin[f];
-        if (d < B) dv = seg_tot[(size_t)seg * C + ch] - __shfl(incl, 63, 64);
+        tot = seg_tot + (size_t)seg * C + ch;
     }
+    r.scan(lane, b0, d, B, tot);
 #pragma unroll
-    for (uint32_t e = 0; e < 4; ++e) {
-        const uint32_t b = b0 + e;
-        v[e] += off + (b >= d ? dv : 0);
-        if (e < E && b < B) h[b] = v[e];
-    }
+    for (uint32_t e = 0; e < 4; ++e)
+        if (e < E && b0 + e < B) h[b0 + e] = r.v[e];
     if (!parent) return;
     // sibling of the built child: parent segment seg has children seg and seg + n_built
     const uint32_t other = slot == seg ? seg + n_built : seg;
@@ -2136,28 +2151,26 @@ static __global__ __launch_bounds__(256) void hist_prefix_kernel(long long* __re
 #pragma unroll
     for (uint32_t e = 0; e < 4; ++e) {
         const uint32_t b = b0 + e;
-        if (e < E && b < B) sib[b] = pr[b] - v[e];
+        if (e < E && b < B) sib[b] = pr[b] - r.v[e];
     }
 }
 
 // The same pass for few bins: a group of GL lanes (32 or 16, up to EM bins each) per row, 64 / GL
 // rows per wave (fewer waves than the 64-lane form, whose lanes past 33 idle at 65 bins).
 template <uint32_t GL, uint32_t EM>
-static __global__ __launch_bounds__(256) void hist_prefix_group_kernel(long long* __restrict__ hist,
-                                                                       const LevelPlan* __restrict__ plan,
-                                                                       uint32_t n_built, uint32_t C, uint32_t F,
-                                                                       uint32_t B,
-                                                                       const long long* __restrict__ parent,
-                                                                       const uint32_t* __restrict__ skip_bin,
-                                                                       const long long* __restrict__ seg_tot) {
+static __global__ __launch_bounds__(256) void hist_prefix_group_kernel(
+    long long* __restrict__ raw, long long* __restrict__ hist, const LevelPlan* __restrict__ plan, uint32_t n_built,
+    uint32_t C, uint32_t CU, uint32_t F, uint32_t B, const long long* __restrict__ parent,
+    const uint32_t* __restrict__ skip_bin, const long long* __restrict__ seg_tot) {
     const uint32_t hl = threadIdx.x & (GL - 1u);
     const uint64_t row = (uint64_t)blockIdx.x * (256 / GL) + (threadIdx.x / GL);
-    const uint64_t rows = (uint64_t)n_built * C * F;
+    const uint64_t rows = (uint64_t)n_built * CU * F;
     const bool valid = row < rows;   // the shuffles below run in every lane of the wave
     const uint64_t rc = valid ? row : rows - 1;
-    const uint32_t seg = (uint32_t)(rc / ((uint64_t)C * F));
-    const uint32_t rem = (uint32_t)(rc - (uint64_t)seg * C * F);
+    const uint32_t seg = (uint32_t)(rc / ((uint64_t)CU * F));
+    const uint32_t rem = (uint32_t)(rc - (uint64_t)seg * CU * F);
     const uint32_t slot = plan ? plan->built[seg] : 0u;
+    long long* rw = raw + ((size_t)seg * C * F + rem) * B;
     long long* h = hist + ((size_t)slot * C * F + rem) * B;
     const uint32_t E = (B + GL - 1) / GL;   // bins per lane, <= EM
     const uint32_t b0 = hl * E;
@@ -2166,7 +2179,12 @@ static __global__ __launch_bounds__(256) void hist_prefix_group_kernel(long long
 #pragma unroll
     for (uint32_t e = 0; e < EM; ++e) {
         const uint32_t b = b0 + e;
-        v[e] = (e < E && b < B) ? h[b] : 0;
+        const bool in = valid && e < E && b < B;
+        v[e] = in ? rw[b] : 0;
+        if (in) rw[b] = 0;
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < EM; ++e) {
         run += v[e];
         v[e] = run;
     }
@@ -2410,7 +2428,6 @@ __device__ __forceinline__ void score_fold(const long long* __restrict__ hist, u
 
 template <int K, int NW>
 __global__ __launch_bounds__(64 * NW) void score_kernel(
-    long long* __restrict__ zero_buf, uint32_t zero_leaves, uint32_t HC,   // next level's histogram
     const long long* __restrict__ hist, uint32_t P, uint32_t F, uint32_t B,
     const uint32_t* __restrict__ n_cand, const uint8_t* __restrict__ one_hot,
     const Scales* __restrict__ sc, double l2, int sf /* CBH_SCORE_* */, double* __restrict__ best_score,
@@ -2419,11 +2436,6 @@ __global__ __launch_bounds__(64 * NW) void score_kernel(
     __shared__ uint32_t red_b[NW];
     const uint32_t f = blockIdx.x;
     const uint32_t b = threadIdx.x;
-    // clear feature f's cells of the next level's histogram [leaf][HC][F][B] (its fill adds)
-    for (uint32_t i = threadIdx.x; i < zero_leaves * HC * B; i += blockDim.x) {
-        const uint32_t lc = i / B, bb = i - lc * B;
-        zero_buf[((size_t)lc * F + f) * B + bb] = 0;
-    }
     const uint32_t nc = n_cand[f];
     if (nc == 0) {
         if (b == 0) {
@@ -2478,6 +2490,173 @@ __global__ __launch_bounds__(64 * NW) void score_kernel(
             }
         best_score[f] = s0;
         best_bin[f] = b0;
+    }
+}
+
+// Histogram finishing and split scoring of one feature in one workgroup (K == 1): the raw
+// rows of the feature become the prefix rows of the built children and their siblings (as
+// hist_prefix_kernel), kept in LDS (kLds) besides their global rows for the next level's
+// subtraction, and the borders are scored from them.  A launch of its own for the finishing cost
+// 5-8 us a level of launch and memory latency, the scorer as much again to read the rows back.
+//
+// The threads are Q = blockDim / BT groups of BT = B rounded up to 64 lanes (a border each); group
+// q takes a run of PW parents.  Each group computes its parents' terms (the divisions) side by
+// side with the others; the running (num, den) of every border passes from group to group through
+// LDS, so the terms are added in score_fold's order (side, p).
+constexpr uint32_t kFinishThreads = 1024;
+constexpr uint32_t kFinishParents = 8;   // a group's parents in flight (its terms in registers)
+constexpr uint32_t kFinishMaxFeatures = 512;
+constexpr size_t kFinishLdsMax = 128 * 1024;   // 32 parents of 256 bins
+inline size_t finish_lds(uint32_t P, uint32_t B) { return (size_t)P * 2u * B * sizeof(long long); }
+
+template <bool kLds>
+static __global__ __launch_bounds__(kFinishThreads) void finish_score_kernel(
+    long long* __restrict__ raw, long long* __restrict__ hist, const LevelPlan* __restrict__ plan, uint32_t n_built,
+    const long long* __restrict__ parent, uint32_t P, uint32_t F, uint32_t B,
+    int keep /* write the level's rows to hist (!kLds: always) */, const uint32_t* __restrict__ skip_bin,
+    const long long* __restrict__ seg_tot, const uint32_t* __restrict__ n_cand, const uint8_t* __restrict__ one_hot,
+    const Scales* __restrict__ sc, double l2, int sf /* CBH_SCORE_* */, double* __restrict__ best_score,
+    uint32_t* __restrict__ best_bin, const double* __restrict__ fweight /* nullable [F] */) {
+    extern __shared__ long long fcell[];   // kLds: [leaf][ch][B]
+    __shared__ double ch_num[256], ch_den[256];
+    __shared__ double red_s[4];
+    __shared__ uint32_t red_b[4];
+    const uint32_t f = blockIdx.x;
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t n_waves = blockDim.x >> 6;
+    const uint32_t nc = n_cand[f];
+    const double inv_d = sc->inv[kScoreDer], inv_w = sc->inv[kScoreW];
+    {
+        const uint32_t E = (B + 63) / 64, b0 = lane * E;
+        const uint32_t d = skip_bin ? skip_bin[f] : B;
+        for (uint32_t row = wave; row < 2u * n_built; row += n_waves) {   // wave-uniform
+            const uint32_t seg = row >> 1, ch = row & 1u;
+            PrefixRow r;
+            r.take(raw + ((size_t)row * F + f) * B, b0, E, B);
+            long long pv[4];
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e)
+                pv[e] = parent && e < E && b0 + e < B ? parent[((size_t)row * F + f) * B + b0 + e] : 0;
+            const uint32_t slot = plan ? plan->built[seg] : 0u;
+            const uint32_t other = slot == seg ? seg + n_built : seg;
+            r.scan(lane, b0, d, B, seg_tot + row);
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                const uint32_t b = b0 + e;
+                if (e >= E || b >= B) continue;
+                const uint32_t at = 2u * slot + ch, so = 2u * other + ch;
+                if (kLds) fcell[at * B + b] = r.v[e];
+                if (!kLds || keep) hist[((size_t)at * F + f) * B + b] = r.v[e];
+                if (parent) {
+                    const long long sv = pv[e] - r.v[e];
+                    if (kLds) fcell[so * B + b] = sv;
+                    if (!kLds || keep) hist[((size_t)so * F + f) * B + b] = sv;
+                }
+            }
+        }
+    }
+    __syncthreads();   // the feature's rows: this workgroup's own writes
+    if (nc == 0) {   // workgroup-uniform
+        if (threadIdx.x == 0) {
+            best_score[f] = -INFINITY;
+            best_bin[f] = 0;
+        }
+        return;
+    }
+    const bool oh = one_hot != nullptr && one_hot[f] != 0;
+    const uint32_t BT = (B + 63) & ~63u;
+    const uint32_t Q = min(kFinishThreads / BT, P);             // groups that take parents
+    const uint32_t PW = min(kFinishParents, (P + Q - 1) / Q);   // parents of a group per slab
+    const uint32_t q = threadIdx.x / BT, b = threadIdx.x - q * BT;
+    const uint32_t bc = min(b, B - 1), bq = bc > 0 ? bc - 1 : 0;
+    const long long* base = kLds ? fcell : hist + (size_t)f * B;
+    const size_t stride = kLds ? B : (size_t)F * B;   // from one (leaf, channel) row to the next
+    double num = 0.0, den = 0.0;
+    den += 1e-100;
+    for (uint32_t side = 0; side < 2; ++side)
+        for (uint32_t p0 = 0; p0 < P; p0 += Q * PW) {
+            const uint32_t mine = p0 + q * PW;
+            double x[kFinishParents], y[kFinishParents];
+            if (q < Q) {
+#pragma unroll
+                for (uint32_t u = 0; u < kFinishParents; ++u) {
+                    x[u] = y[u] = 0.0;
+                    const uint32_t p = mine + u;
+                    if (u >= PW || p >= P) continue;   // uniform over the group
+                    const long long* rd = base + (size_t)(2u * p) * stride;
+                    const long long* rw = rd + stride;
+                    const long long pd = rd[bc], pw = rw[bc], td = rd[B - 1], tw = rw[B - 1];
+                    long long xd, xw;
+                    if (!oh) {
+                        xd = side == 0 ? pd : td - pd;
+                        xw = side == 0 ? pw : tw - pw;
+                    } else {
+                        const long long vd = pd - (b > 0 ? rd[bq] : 0), vw = pw - (b > 0 ? rw[bq] : 0);
+                        xd = side == 0 ? td - vd : vd;
+                        xw = side == 0 ? tw - vw : vw;
+                    }
+                    const double s = (double)xd * inv_d, w = (double)xw * inv_w;
+                    if (sf > 1) {
+                        x[u] = leaf_score_term(sf, s, w);
+                    } else {
+                        const double t = s / (w + l2);
+                        const double avg = w > 0.0 ? t : 0.0;
+                        x[u] = avg * s;
+                        y[u] = avg * avg * w;
+                    }
+                }
+            }
+            // the groups' turns; a slab's groups past P have nothing to add
+            const uint32_t turns = min(Q, (P - p0 + PW - 1) / PW);
+            for (uint32_t g = 0; g < turns; ++g) {
+                if (q == g) {
+                    if (side + p0 + g > 0) {
+                        num = ch_num[b];
+                        den = ch_den[b];
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < kFinishParents; ++u) {
+                        if (u >= PW || mine + u >= P) continue;
+                        num += x[u];
+                        if (sf <= 1) den += y[u];
+                    }
+                    ch_num[b] = num;
+                    ch_den[b] = den;
+                }
+                __syncthreads();
+            }
+        }
+    double score = -INFINITY;
+    uint32_t bb = b;
+    if (q == 0) {
+        num = ch_num[b];
+        den = ch_den[b];
+        score = sf == 0 ? num / sqrt(den) : num;
+        // the model_size_reg weight of a CTR column multiplies every candidate's score
+        if (fweight) score = fweight[f] * score;
+        if (b >= nc || score != score) score = -INFINITY;
+        for (int o = 32; o > 0; o >>= 1) {
+            double os = __shfl_xor(score, o, 64);
+            uint32_t ob = __shfl_xor(bb, o, 64);
+            if (os > score || (os == score && ob < bb)) {
+                score = os;
+                bb = ob;
+            }
+        }
+        if (lane == 0) {
+            red_s[wave] = score;
+            red_b[wave] = bb;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t k = 1; k < BT / 64; ++k)
+            if (red_s[k] > score || (red_s[k] == score && red_b[k] < bb)) {
+                score = red_s[k];
+                bb = red_b[k];
+            }
+        best_score[f] = score;
+        best_bin[f] = bb;
     }
 }
 
@@ -2676,7 +2855,6 @@ __device__ __forceinline__ void score_chain(const long long* __restrict__ hist, 
 
 template <int K, int PW, bool kPartial>
 __global__ __launch_bounds__(512) void score_chain_kernel(
-    long long* __restrict__ zero_buf, uint32_t zero_leaves, uint32_t HC,   // next level's histogram
     const long long* __restrict__ hist, uint32_t P, uint32_t F, uint32_t B,
     const uint32_t* __restrict__ n_cand, const uint8_t* __restrict__ one_hot,
     const Scales* __restrict__ sc, double l2, int sf /* CBH_SCORE_COSINE or _L2 */, double* __restrict__ best_score,
@@ -2688,11 +2866,6 @@ __global__ __launch_bounds__(512) void score_chain_kernel(
     // features f .. f + nf - 1 (nf > 1: B <= 64 / nf and no one-hot features)
     const uint32_t f = blockIdx.x * nf;
     const uint32_t nfe = min(nf, F - f);
-    // clear the features' cells of the next level's histogram [leaf][HC][F][B] (its fill adds)
-    for (uint32_t i = threadIdx.x; i < zero_leaves * HC * nfe * B; i += blockDim.x) {
-        const uint32_t lc = i / (nfe * B), fb = i - lc * (nfe * B);
-        zero_buf[((size_t)lc * F + f) * B + fb] = 0;
-    }
     uint32_t any_cand = 0;
     for (uint32_t g = 0; g < nfe; ++g) any_cand |= n_cand[f + g];
     if (any_cand == 0) {   // workgroup-uniform: no wave enters the chain

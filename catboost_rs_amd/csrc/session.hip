@@ -129,7 +129,8 @@ struct cbh_session {
     uint16_t* leaf = nullptr;
     uint32_t* idx = nullptr;
     long long* hist[2] = {nullptr, nullptr};
-    size_t hist_cells_max = 0;
+    long long* raw = nullptr;        // the fill's sums of the directly built children, [segment][C][F][B]
+    size_t hist_cells_max = 0, raw_cells = 0;
     uint32_t* cnt = nullptr;         // partition: row counts [wave][leaf] of the level
     uint32_t* gcnt = nullptr;        // [level][group][leaf], cleared once per tree
     uint32_t n_part_blocks = 0, n_groups_part = 0;
@@ -294,7 +295,7 @@ struct cbh_session {
 
     void release() {
         dfree(rows); dfree(cols); dfree(weight); dfree(target); dfree(approx); dfree(sstat);
-        dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(cnt);
+        dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(raw); dfree(cnt);
         dfree(gcnt); dfree(best_score);
         dfree(best_bin); dfree(n_cand); dfree(one_hot); dfree(scales);
         dfree(leaf_sums); dfree(leaf_scaled); dfree(jump);
@@ -423,6 +424,11 @@ int session_alloc(cbh_session* s) {
     s->hist_cells_max = per_leaf << (s->depth - 1);
     CHECK(dalloc(&s->hist[0], s->hist_cells_max));
     CHECK(dalloc(&s->hist[1], s->hist_cells_max));
+    // zero outside a level's fill and finishing, which clears what it reads: cleared here once
+    s->raw_cells = per_leaf << (s->depth >= 2 ? s->depth - 2 : 0);
+    CHECK(dalloc(&s->raw, s->raw_cells));
+    zero_i64_kernel<<<grid_for(s->raw_cells, 256, 8192), 256, 0, s->stream>>>(s->raw, s->raw_cells);
+    HIP_TRY(hipGetLastError());
     s->n_part_blocks = (uint32_t)((n + kPartRows - 1) / kPartRows);
     // per level of up to 2^(depth - 1) new leaves: counts [wave][leaf], and per group of
     // workgroups [level][group][leaf]
@@ -1184,6 +1190,9 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
     CHECK(with_k((int)s->K, [&](auto kc) {
         constexpr int K = decltype(kc)::value;
         CHECK(set_fill_attr<K + 1>(s->tiles.lds_bytes));
+        if (K == 1)
+            HIP_TRY(hipFuncSetAttribute((const void*)finish_score_kernel<true>,
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFinishLdsMax));
         const size_t lds = ((size_t)1 << s->depth) * (size_t)leaf_cells<K>() * sizeof(long long);
         HIP_TRY(hipFuncSetAttribute((const void*)leaf_reduce_kernel<K>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1621,13 +1630,7 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         long long* cur = s->hist[level & 1];
         long long* par = s->hist[(level + 1) & 1];
         const uint32_t n_leaves = 1u << level;
-        // ---- fill (the histogram it accumulates into is zeroed first: here at level 0 and with
-        // pairwise scoring, else by the previous level's score kernel) ----
-        if (level == 0 || s->pairwise) {
-            CHECK(s->stage_begin(kStPrepare));
-            CHECK(launch_zero(cur, per_leaf * n_leaves, st));
-            CHECK(s->stage_end());
-        }
+        // ---- fill, into the raw buffer ----
         const uint32_t nt = s->tiles.n_tiles;
         const uint32_t G = s->fill_ranges;
         const uint32_t* lidx = level == 0 ? nullptr : s->idx;
@@ -1645,27 +1648,27 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         if (s->packed && level == 0)
             fill_packed_kernel<false, false><<<s->pk_dense.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, s->spack, nullptr, s->pk_dense.tiles16, s->F, s->B,
-                s->pk_dense.ranges, s->pk_dense.ranges_n, cur, s->pk_swap, nullptr, 0u, s->scales);
+                s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, s->pk_swap, nullptr, 0u, s->scales);
         else if (s->packed)
             fill_packed_kernel<true, false><<<s->pk_gath.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
-                s->pk_gath.ranges, 0u, cur, s->pk_swap, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
+                s->pk_gath.ranges, 0u, s->raw, s->pk_swap, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
         else if (s->count && level == 0)
             fill_packed_kernel<false, true><<<s->pk_dense.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, s->spack, nullptr, s->pk_dense.tiles16, s->F, s->B,
-                s->pk_dense.ranges, s->pk_dense.ranges_n, cur, 0u, nullptr, 0u, s->scales);
+                s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, 0u, nullptr, 0u, s->scales);
         else if (s->count)
             fill_packed_kernel<true, true><<<s->pk_gath.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
-                s->pk_gath.ranges, 0u, cur, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
+                s->pk_gath.ranges, 0u, s->raw, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
         else if (s->tiled && level == 0)
             fill_exact_kernel<false><<<s->pk_dense.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, (const long long*)s->sstat, nullptr, s->pk_dense.tiles16, s->F,
-                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, cur, nullptr, 0u, s->ex_sets, s->scales);
+                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, nullptr, 0u, s->ex_sets, s->scales);
         else if (s->tiled)
             fill_exact_kernel<true><<<s->pk_gath.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, (const long long*)s->sstat, (const long long*)s->sseq,
-                s->pk_gath.tiles16, s->F, s->B, s->pk_gath.ranges, s->pk_gath.ranges_n, cur,
+                s->pk_gath.tiles16, s->F, s->B, s->pk_gath.ranges, s->pk_gath.ranges_n, s->raw,
                 s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->ex_sets, s->scales);
         else if (s->pkk) {
             const size_t lds = (size_t)kPkkCells * sizeof(unsigned long long);
@@ -1679,57 +1682,57 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             const uint32_t npf = w0_use ? NPl - 1 : NPl;
             if (level == 0) s->l0_cached = w0_use;
             if (w0_use)
-                HIP_TRY(hipMemcpyAsync(cur + (size_t)(C - 1) * s->F * s->B, s->w0_cache,
+                HIP_TRY(hipMemcpyAsync(s->raw + (size_t)(C - 1) * s->F * s->B, s->w0_cache,
                                        sizeof(long long) * s->F * s->B, hipMemcpyDeviceToDevice, st));
             // (small tiles: 4 cells per thread, their registers leaving room for 8 blocks in flight)
             const size_t lds4 = (size_t)4 * kPkkThreads * sizeof(unsigned long long);
             if (s->pks && s->pks_small && level == 0)
                 fill_pks_kernel<C, false, 4, 8><<<grid, kPkkThreads, lds4, st>>>(
-                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur, npf);
+                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
             else if (s->pks && s->pks_small)
                 fill_pks_kernel<C, true, 4, 8><<<grid, kPkkThreads, lds4, st>>>(
-                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur, npf);
+                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
             else if (s->pks && level == 0)
                 fill_pks_kernel<C, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur, npf);
+                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
             else if (s->pks)
                 fill_pks_kernel<C, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur, npf);
+                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
             else if (s->use_skip && level == 0)
                 fill_pkk_kernel<C, true, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur,
+                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
                     s->skip_bin, npf);
             else if (s->use_skip)
                 fill_pkk_kernel<C, true, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur,
+                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
                     s->skip_bin, npf);
             else if (level == 0)
                 fill_pkk_kernel<C, false, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur,
+                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
                     nullptr, npf);
             else
                 fill_pkk_kernel<C, false, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, cur,
+                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
                     nullptr, npf);
         } else if (s->use_skip)
             fill_kernel<C, true><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, cur,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
                 s->skip_bin, (int)s->tiles.bin_major);
         else if (C == 2 && s->pairwise)
             // PairLogitPairwise scores from the der channel and the pair statistics alone: the
             // weight channel is left out of the fill (its cells stay zero; such sessions refuse
             // histogram capture)
             fill_kernel<2, false, 1><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, cur,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
                 nullptr, (int)s->tiles.bin_major);
         else
             fill_kernel<C, false><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, cur,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
                 nullptr, (int)s->tiles.bin_major);
         HIP_TRY(hipGetLastError());
         CHECK(s->stage_end());
         if (s->pkk && level == 0 && s->w_static && !s->w0_ready) {   // the weight channel's cache
-            HIP_TRY(hipMemcpyAsync(s->w0_cache, cur + (size_t)(C - 1) * s->F * s->B, sizeof(long long) * s->F * s->B,
+            HIP_TRY(hipMemcpyAsync(s->w0_cache, s->raw + (size_t)(C - 1) * s->F * s->B, sizeof(long long) * s->F * s->B,
                                    hipMemcpyDeviceToDevice, st));
             s->w0_ready = true;
         }
@@ -1747,41 +1750,37 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                                                                        fill_atomics_per_entry(s, level));
             HIP_TRY(hipGetLastError());
         }
-        // ---- histogram finishing: dominant bins, prefix form, siblings ----
-        CHECK(s->stage_begin(kStDerive));
-        {   // built children to prefix form over bins (the level's histograms stay in it), with
-            // their dominant bins rebuilt from the segment totals, and their siblings = parent -
-            // built (levels >= 1)
-            const uint64_t rows = (uint64_t)n_seg * C * s->F;
+        // ---- histogram finishing: dominant bins, prefix form, siblings; K = 1 with the scoring ----
+        const bool last = level + 1 == s->depth;
+        // one workgroup per feature finishes and scores it; many features fill the chip with the
+        // finishing's own waves and the scorer's smaller workgroups (see kFinishMaxFeatures)
+        const bool finish = K == 1 && !s->pairwise && s->F <= kFinishMaxFeatures;
+        if (!finish) {
+            CHECK(s->stage_begin(kStDerive));
+            // (PairLogitPairwise fills and reads the der channel only)
+            const bool der_only = s->pairwise && !s->packed && !s->count && !s->tiled && !s->use_skip;
+            const uint32_t CU = der_only ? 1u : (uint32_t)C;
+            const uint64_t rows = (uint64_t)n_seg * CU * s->F;
+            const long long* parent = level > 0 ? par : nullptr;
+            const uint32_t* sb = s->use_skip ? s->skip_bin : nullptr;
             if (s->B <= 72)   // 8 lanes per row
                 hist_prefix_group_kernel<8, 9><<<(unsigned)((rows + 31) / 32), 256, 0, st>>>(
-                    cur, lplan, n_seg, C, s->F, s->B, level > 0 ? par : nullptr,
-                    s->use_skip ? s->skip_bin : nullptr, s->seg_tot);
+                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else if (s->B <= 80)   // 16 lanes per row
                 hist_prefix_group_kernel<16, 5><<<(unsigned)((rows + 15) / 16), 256, 0, st>>>(
-                    cur, lplan, n_seg, C, s->F, s->B, level > 0 ? par : nullptr,
-                    s->use_skip ? s->skip_bin : nullptr, s->seg_tot);
+                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else if (s->B <= 96)   // a half-wave per row
                 hist_prefix_group_kernel<32, 3><<<(unsigned)((rows + 7) / 8), 256, 0, st>>>(
-                    cur, lplan, n_seg, C, s->F, s->B, level > 0 ? par : nullptr,
-                    s->use_skip ? s->skip_bin : nullptr, s->seg_tot);
+                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else
                 hist_prefix_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(
-                    cur, lplan, n_seg, C, s->F, s->B, level > 0 ? par : nullptr,
-                    s->use_skip ? s->skip_bin : nullptr, s->seg_tot);
+                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             HIP_TRY(hipGetLastError());
+            CHECK(s->stage_end());
         }
-        CHECK(s->stage_end());
-        if (s->hist_cap)   // the level's histograms as the scorer reads them (inspection only)
-            HIP_TRY(hipMemcpyAsync(s->hist_cap + s->hist_cap_off[level], cur, sizeof(long long) * per_leaf * n_leaves,
-                                   hipMemcpyDeviceToDevice, st));
         // ---- score + argmax ----
         if (s->ctr_n) CHECK(s->ctr_dev ? ctr_level_weights_dev(s, level) : ctr_level_weights(s, level));
         CHECK(s->stage_begin(kStScore));
-        // the score also clears the next level's histogram (the parent buffer, dead once the
-        // derive above has run)
-        long long* zbuf = level + 1 < s->depth ? par : nullptr;
-        const uint32_t zleaves = level + 1 < s->depth ? 2u * n_leaves : 0u;
         // K > 1: the parents are split over the (at most 8) waves of a feature's workgroup, 16
         // per wave from 64 parents at K >= 3 (registers), else 8 (fewer than 8: one wave)
         const uint32_t chain_pw = n_leaves >= 64 && K >= 3 ? 16u : 8u;
@@ -1791,6 +1790,15 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                            (uint64_t)chain_pw * s->C * s->F * s->B * 8u < (1ull << 31);
         if (s->pairwise) {
             CHECK(pairwise_level(s, cur, level));
+        } else if (finish) {
+            // (the last level's rows are read by nothing after it)
+            const int keep = !last || s->hist_cap ? 1 : 0;
+            const size_t lds = finish_lds(n_leaves, s->B);
+            const bool in_lds = lds <= kFinishLdsMax;
+            (in_lds ? finish_score_kernel<true> : finish_score_kernel<false>)<<<s->F, kFinishThreads, in_lds ? lds : 0, st>>>(
+                s->raw, cur, lplan, n_seg, level > 0 ? par : nullptr, n_leaves, s->F, s->B, keep,
+                s->use_skip ? s->skip_bin : nullptr, s->seg_tot, s->n_cand, s->one_hot, s->scales, s->l2, sfn,
+                s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr);
         } else if (chain) {
             // several features per workgroup when B lanes per feature leave most of a wave idle
             // (config 5's 20 bins: 3 features in 60 lanes) and no feature is one-hot; at most 64 /
@@ -1801,35 +1809,38 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             if constexpr (K >= 3) {
                 if (chain_pw == 16)
                     score_chain_kernel<K, 16, false><<<groups, 64 * (n_leaves / 16), 0, st>>>(
-                        zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
+                        cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
                         sfn, s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr, s->chain_spin,
                         &s->bounds->device_err, nf);
             }
             if constexpr (K > 1) {
                 if (chain_pw == 8 && n_leaves >= 8)
                     score_chain_kernel<K, 8, false><<<groups, 64 * (n_leaves / 8), 0, st>>>(
-                        zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
+                        cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
                         sfn, s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr, s->chain_spin,
                         &s->bounds->device_err, nf);
                 else if (chain_pw == 8)
                     score_chain_kernel<K, 8, true><<<groups, 64, 0, st>>>(
-                        zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
+                        cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot, s->scales, s->l2,
                         sfn, s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr, s->chain_spin,
                         &s->bounds->device_err, nf);
             }
         } else if (s->max_cand <= 64)
-            score_kernel<K, 1><<<s->F, 64, 0, st>>>(zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+            score_kernel<K, 1><<<s->F, 64, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                    s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
         else if (s->max_cand <= 128)
-            score_kernel<K, 2><<<s->F, 128, 0, st>>>(zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+            score_kernel<K, 2><<<s->F, 128, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                     s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
         else
-            score_kernel<K, 4><<<s->F, 256, 0, st>>>(zbuf, zleaves, s->C, cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+            score_kernel<K, 4><<<s->F, 256, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                     s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
         HIP_TRY(hipGetLastError());
+        if (s->hist_cap)   // the level's histograms as the scorer reads them (inspection only)
+            HIP_TRY(hipMemcpyAsync(s->hist_cap + s->hist_cap_off[level], cur, sizeof(long long) * per_leaf * n_leaves,
+                                   hipMemcpyDeviceToDevice, st));
         const bool fuse_argmax = s->F <= kArgmaxFuse;
         if (!fuse_argmax) {
             argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F,
@@ -1839,7 +1850,6 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         CHECK(s->stage_end());
         // ---- partition ----
         CHECK(s->stage_begin(kStPartition));
-        const bool last = level + 1 == s->depth;
         uint32_t* gcnt = last ? nullptr : s->gcnt + group_count_off(s->n_groups_part, level);
         (fuse_argmax ? split_count_kernel<true> : split_count_kernel<false>)<<<NB, 256, 0, st>>>(
             s->cols, n, s->splits + level, s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F, level,
