@@ -251,8 +251,11 @@ static __global__ __launch_bounds__(256) void prepare_kernel(
     unsigned long long* __restrict__ partials /* [gridDim.x][kPartials] */,
     const double* __restrict__ ext_der /* nullable [2][n]: der1, der2 of a pair loss */,
     const double* __restrict__ score_w /* nullable [n]: histogram weight (pairwise weights) */,
-    uint32_t* __restrict__ gcnt /* the partition's group counts, cleared for the tree */, uint32_t n_gcnt) {
+    uint32_t* __restrict__ gcnt /* the partition's group counts, cleared for the tree */, uint32_t n_gcnt,
+    long long* __restrict__ zraw /* raw segments the last level's finishing left, cleared */, size_t n_zraw) {
     constexpr int C = K + 1;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_zraw; i += (size_t)gridDim.x * blockDim.x)
+        zraw[i] = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_gcnt; i += gridDim.x * blockDim.x) gcnt[i] = 0;
     __shared__ unsigned long long red[4][kPartials];
     unsigned long long acc[kPartials] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -2084,14 +2087,15 @@ static __global__ void pack_stats_count_kernel(const double* __restrict__ sstat,
 // consecutive bins.
 struct PrefixRow {
     long long v[4];
-    // the raw bins of this lane, cleared
-    __device__ __forceinline__ void take(long long* __restrict__ raw, uint32_t b0, uint32_t E, uint32_t B) {
+    // the raw bins of this lane, cleared when the wave is their only reader
+    __device__ __forceinline__ void take(long long* __restrict__ raw, uint32_t b0, uint32_t E, uint32_t B,
+                                         bool clear = true) {
 #pragma unroll
         for (uint32_t e = 0; e < 4; ++e) {
             const uint32_t b = b0 + e;
             const bool in = e < E && b < B;
             v[e] = in ? raw[b] : 0;
-            if (in) raw[b] = 0;
+            if (in && clear) raw[b] = 0;
         }
     }
     // inclusive prefix over the wave's bins; a dominant bin d the fill left out (its cell still 0)
@@ -2493,170 +2497,297 @@ __global__ __launch_bounds__(64 * NW) void score_kernel(
     }
 }
 
-// Histogram finishing and split scoring of one feature in one workgroup (K == 1): the raw
-// rows of the feature become the prefix rows of the built children and their siblings (as
-// hist_prefix_kernel), kept in LDS (kLds) besides their global rows for the next level's
-// subtraction, and the borders are scored from them.  A launch of its own for the finishing cost
-// 5-8 us a level of launch and memory latency, the scorer as much again to read the rows back.
+// Histogram finishing and split scoring in one launch.  A workgroup takes a window of columns:
+// nf whole features when several fit 64 lanes (B <= 64), else m slices of 64 borders of one
+// feature (n_parts workgroups a feature).  The raw rows of its features become the prefix rows of
+// the built children and their siblings (as hist_prefix_kernel; a slice's workgroup scans the
+// whole row and writes its own slice), and its borders are scored from the copy it keeps in LDS.
+// As two launches the finishing cost 5-8 us a level of launch and memory latency, and the
+// scorer as much again to read the rows back.
 //
-// The threads are Q = blockDim / BT groups of BT = B rounded up to 64 lanes (a border each); group
-// q takes a run of PW parents.  Each group computes its parents' terms (the divisions) side by
-// side with the others; the running (num, den) of every border passes from group to group through
-// LDS, so the terms are added in score_fold's order (side, p).
-constexpr uint32_t kFinishThreads = 1024;
-constexpr uint32_t kFinishParents = 8;   // a group's parents in flight (its terms in registers)
-constexpr uint32_t kFinishMaxFeatures = 512;
-constexpr size_t kFinishLdsMax = 128 * 1024;   // 32 parents of 256 bins
-inline size_t finish_lds(uint32_t P, uint32_t B) { return (size_t)P * 2u * B * sizeof(long long); }
+// What bounds it is latency: the raw rows (added by other XCDs' atomics) and the parent's take
+// 1-2 us to come, so the rows of every channel are in flight together, spread over the waves;
+// then the terms of all (dimension, side, parent) triples are computed in batches of nt, a triple
+// a wave, lane = border (the divisions side by side), and wave 0 adds the batch's num terms
+// and wave 1 its den terms in score_fold's order while the other waves compute the next batch (two
+// buffers, one barrier a batch; a single batch when all terms fit).
+constexpr uint32_t kFinishThreads = 1024, kFinishWaves = kFinishThreads / 64;
+constexpr uint32_t kFinishSlices = 4;
+constexpr size_t kFinishLdsMax = 156 * 1024;   // beside the static arrays, of 160 KB
+struct FinishPlan {
+    uint32_t nf, m, n_parts, nt, blocks;   // features a workgroup (B <= 64), slices, workgroups a feature, batch
+    size_t lds;                            // 0: does not fit
+};
+__host__ __device__ inline uint32_t finish_row_cells(uint32_t m) { return 64u * m + 2u; }   // columns, total, predecessor
+inline FinishPlan plan_finish(uint32_t P, uint32_t K, uint32_t F, uint32_t B, uint32_t cus, bool one_hot) {
+    FinishPlan pl{1, 1, 1, 0, 0, 0};
+    const uint32_t ns = (B + 63) / 64;
+    if (B <= 64) {
+        pl.nf = one_hot ? 1u : std::max<uint32_t>(1u, 64u / B);
+        pl.blocks = (F + pl.nf - 1) / pl.nf;
+    } else {
+        // enough workgroups for the CUs, otherwise as few as fit: each repeats the row scans
+        pl.m = std::min(F >= cus / 2 ? 4u : F >= cus / 4 ? 2u : 1u, ns);
+    }
+    const uint32_t terms = 2 * K * P;
+    for (;; pl.m /= 2) {
+        const size_t cells = (size_t)(K + 1) * P * finish_row_cells(pl.m) * 8;
+        auto fits = [&](uint32_t nt, uint32_t bufs) {
+            pl.nt = nt;
+            pl.lds = cells + (size_t)bufs * nt * 1024;
+            return pl.lds <= kFinishLdsMax;
+        };
+        if ((terms <= 64 && fits(terms, 1)) || fits(32, 2) || fits(16, 2) || fits(8, 2)) {
+            pl.n_parts = B <= 64 ? 1u : (ns + pl.m - 1) / pl.m;
+            if (B > 64) pl.blocks = F * pl.n_parts;
+            return pl;
+        }
+        pl.lds = 0;
+        if (pl.m == 1) return pl;
+    }
+}
 
-template <bool kLds>
+template <int K>
 static __global__ __launch_bounds__(kFinishThreads) void finish_score_kernel(
     long long* __restrict__ raw, long long* __restrict__ hist, const LevelPlan* __restrict__ plan, uint32_t n_built,
-    const long long* __restrict__ parent, uint32_t P, uint32_t F, uint32_t B,
-    int keep /* write the level's rows to hist (!kLds: always) */, const uint32_t* __restrict__ skip_bin,
-    const long long* __restrict__ seg_tot, const uint32_t* __restrict__ n_cand, const uint8_t* __restrict__ one_hot,
-    const Scales* __restrict__ sc, double l2, int sf /* CBH_SCORE_* */, double* __restrict__ best_score,
-    uint32_t* __restrict__ best_bin, const double* __restrict__ fweight /* nullable [F] */) {
-    extern __shared__ long long fcell[];   // kLds: [leaf][ch][B]
-    __shared__ double ch_num[256], ch_den[256];
-    __shared__ double red_s[4];
-    __shared__ uint32_t red_b[4];
-    const uint32_t f = blockIdx.x;
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t n_waves = blockDim.x >> 6;
-    const uint32_t nc = n_cand[f];
+    const long long* __restrict__ parent, uint32_t P, uint32_t F, uint32_t B, uint32_t nf, uint32_t m,
+    uint32_t n_parts, uint32_t nt, int keep /* write the level's rows to hist */,
+    long long* __restrict__ zraw /* n_parts > 1: the other raw buffer, its n_zero segments cleared */, uint32_t n_zero,
+    const uint32_t* __restrict__ skip_bin, const long long* __restrict__ seg_tot,
+    const uint32_t* __restrict__ n_cand, const uint8_t* __restrict__ one_hot,
+    const Scales* __restrict__ sc, double l2, int sf /* CBH_SCORE_* */,
+    double* __restrict__ best_score /* [F][n_parts] */, uint32_t* __restrict__ best_bin,
+    const double* __restrict__ fweight /* nullable [F] */) {
+    constexpr uint32_t C = K + 1;
+    extern __shared__ long long fsm[];
+    __shared__ double red[kFinishSlices][64];
+    const uint32_t RS = finish_row_cells(m);
+    long long* cells = fsm;                             // [leaf][C][RS]: the window's prefix rows
+    double* tb = (double*)(fsm + (size_t)C * P * RS);   // [1 or 2][nt][num, den][64]
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const bool wide = B > 64;
+    const uint32_t f0 = wide ? blockIdx.x / n_parts : blockIdx.x * nf;
+    const uint32_t part = wide ? blockIdx.x - f0 * n_parts : 0u;
+    const uint32_t nfe = min(nf, F - f0);
+    const uint32_t s0 = part * m * 64u;                    // first bin of the window (wide)
+    const uint32_t win = wide ? min(64u * m, B - s0) : 0u; // its bins
+    // B <= 64: lane = (feature g, border gb) of the window's nfe B contiguous cells
+    const uint32_t g = wide ? 0u : min(lane / B, nfe - 1), gb = wide ? 0u : lane - (lane / B) * B;
+    const bool on = wide || lane < nfe * B;
     const double inv_d = sc->inv[kScoreDer], inv_w = sc->inv[kScoreW];
-    {
-        const uint32_t E = (B + 63) / 64, b0 = lane * E;
-        const uint32_t d = skip_bin ? skip_bin[f] : B;
-        for (uint32_t row = wave; row < 2u * n_built; row += n_waves) {   // wave-uniform
-            const uint32_t seg = row >> 1, ch = row & 1u;
-            PrefixRow r;
-            r.take(raw + ((size_t)row * F + f) * B, b0, E, B);
-            long long pv[4];
+    const uint32_t E = (B + 63) / 64, b0 = lane * E;       // wide: bins of a lane while scanning
+    const uint32_t skip = skip_bin ? skip_bin[f0 + g] : 256u;
+    const bool in_place = n_parts == 1;                    // the only reader of the raw rows clears them
+
+    // row (segment, channel): prefix rows of the built child and its sibling
+    const uint32_t n_rows = n_built * C;
+    constexpr uint32_t R = 2;   // rows of a wave in flight
+    for (uint32_t row0 = wave; row0 < n_rows; row0 += R * kFinishWaves) {   // wave-uniform
+        uint32_t slot[R], other[R], ch[R], seg[R];
 #pragma unroll
-            for (uint32_t e = 0; e < 4; ++e)
-                pv[e] = parent && e < E && b0 + e < B ? parent[((size_t)row * F + f) * B + b0 + e] : 0;
-            const uint32_t slot = plan ? plan->built[seg] : 0u;
-            const uint32_t other = slot == seg ? seg + n_built : seg;
-            r.scan(lane, b0, d, B, seg_tot + row);
+        for (uint32_t k = 0; k < R; ++k) {
+            const uint32_t row = min(row0 + k * kFinishWaves, n_rows - 1);
+            seg[k] = row / C;
+            ch[k] = row - seg[k] * C;
+            slot[k] = plan ? plan->built[seg[k]] : 0u;
+        }
+        if (wide) {
+            PrefixRow r[R];
+            long long pv[R][4];
 #pragma unroll
-            for (uint32_t e = 0; e < 4; ++e) {
-                const uint32_t b = b0 + e;
-                if (e >= E || b >= B) continue;
-                const uint32_t at = 2u * slot + ch, so = 2u * other + ch;
-                if (kLds) fcell[at * B + b] = r.v[e];
-                if (!kLds || keep) hist[((size_t)at * F + f) * B + b] = r.v[e];
-                if (parent) {
-                    const long long sv = pv[e] - r.v[e];
-                    if (kLds) fcell[so * B + b] = sv;
-                    if (!kLds || keep) hist[((size_t)so * F + f) * B + b] = sv;
+            for (uint32_t k = 0; k < R; ++k) {
+                const bool live = row0 + k * kFinishWaves < n_rows;
+                const size_t at = (((size_t)seg[k] * C + ch[k]) * F + f0) * B;
+                r[k].take(raw + at, b0, live ? E : 0u, B, in_place);
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e)
+                    pv[k][e] = live && parent && e < E && b0 + e < B ? parent[at + b0 + e] : 0;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < R; ++k) {
+                if (row0 + k * kFinishWaves >= n_rows) break;
+                other[k] = slot[k] == seg[k] ? seg[k] + n_built : seg[k];
+                r[k].scan(lane, b0, skip, B, seg_tot + (size_t)seg[k] * C + ch[k]);
+                long long* hb = hist + (((size_t)slot[k] * C + ch[k]) * F + f0) * B;
+                long long* hs = hist + (((size_t)other[k] * C + ch[k]) * F + f0) * B;
+                long long* lb = cells + ((size_t)slot[k] * C + ch[k]) * RS;
+                long long* ls = cells + ((size_t)other[k] * C + ch[k]) * RS;
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e) {
+                    const uint32_t b = b0 + e;
+                    if (e >= E || b >= B) continue;
+                    const long long v = r[k].v[e], sv = pv[k][e] - v;
+                    const uint32_t c = b - s0;   // (wraps below the window)
+                    if (c < win) {
+                        lb[c] = v;
+                        if (parent) ls[c] = sv;
+                        if (keep) {
+                            hb[b] = v;
+                            if (parent) hs[b] = sv;
+                        }
+                    }
+                    if (b == B - 1) {
+                        lb[64u * m] = v;
+                        if (parent) ls[64u * m] = sv;
+                    }
+                    if (b + 1 == s0) {
+                        lb[64u * m + 1] = v;
+                        if (parent) ls[64u * m + 1] = sv;
+                    }
+                }
+            }
+        } else {
+            long long v[R], pv[R];
+#pragma unroll
+            for (uint32_t k = 0; k < R; ++k) {
+                const bool live = on && row0 + k * kFinishWaves < n_rows;
+                const size_t at = (((size_t)seg[k] * C + ch[k]) * F + f0) * B + lane;
+                v[k] = live ? raw[at] : 0;
+                pv[k] = live && parent ? parent[at] : 0;
+                if (live) raw[at] = 0;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < R; ++k) {
+                if (row0 + k * kFinishWaves >= n_rows) break;
+                other[k] = slot[k] == seg[k] ? seg[k] + n_built : seg[k];
+                for (uint32_t o = 1; o < B; o <<= 1) {
+                    const long long u = __shfl_up(v[k], o, 64);
+                    if (gb >= o) v[k] += u;
+                }
+                if (skip_bin) {   // dominant bins rebuilt (PrefixRow::scan)
+                    const long long tot = __shfl(v[k], (int)(g * B + B - 1), 64);
+                    if (skip < B && gb >= skip) v[k] += seg_tot[(size_t)seg[k] * C + ch[k]] - tot;
+                }
+                const long long sv = pv[k] - v[k];
+                cells[((size_t)slot[k] * C + ch[k]) * RS + lane] = v[k];
+                if (parent) cells[((size_t)other[k] * C + ch[k]) * RS + lane] = sv;
+                if (keep && on) {
+                    hist[(((size_t)slot[k] * C + ch[k]) * F + f0) * B + lane] = v[k];
+                    if (parent) hist[(((size_t)other[k] * C + ch[k]) * F + f0) * B + lane] = sv;
                 }
             }
         }
     }
-    __syncthreads();   // the feature's rows: this workgroup's own writes
-    if (nc == 0) {   // workgroup-uniform
-        if (threadIdx.x == 0) {
-            best_score[f] = -INFINITY;
-            best_bin[f] = 0;
+
+    if (!in_place)   // the window's cells of the other raw buffer, all read by the level before
+        for (uint32_t row = wave; row < n_zero * C; row += kFinishWaves)
+            for (uint32_t c = lane; c < win; c += 64) zraw[((size_t)row * F + f0) * B + s0 + c] = 0;
+    uint32_t cand = 0;   // candidates of the window
+    if (wide) {
+        const uint32_t nc = n_cand[f0];
+        cand = nc > s0 ? nc - s0 : 0u;
+    } else {
+        for (uint32_t k = 0; k < nfe; ++k) cand |= n_cand[f0 + k];
+    }
+    const bool oh = one_hot != nullptr && one_hot[f0] != 0;
+    const uint32_t slices = wide ? min(m, (cand + 63u) / 64u) : (cand ? 1u : 0u);   // those with a candidate
+    double acc[kFinishSlices];   // wave 0: num, wave 1: den
+#pragma unroll
+    for (uint32_t k = 0; k < kFinishSlices; ++k) acc[k] = wave == 1 ? 1e-100 : 0.0;
+    __syncthreads();
+    const uint32_t n_terms = 2u * (uint32_t)K * P;   // (d, side, p): p fastest
+    const uint32_t lgP = 31u - __clz((int)P);
+    uint32_t buf = 0;
+    for (uint32_t k = 0; k < slices; ++k) {   // workgroup-uniform
+        const uint32_t col = 64u * k + lane;
+        const uint32_t tot_at = wide ? 64u * m : g * B + B - 1;
+        const uint32_t b = wide ? s0 + col : gb;
+        const uint32_t prev_at = wide ? (col > 0 ? col - 1 : 64u * m + 1) : (lane > 0 ? lane - 1 : 0u);
+        double run = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < kFinishSlices; ++j) run = j == k ? acc[j] : run;
+        for (uint32_t t0 = 0; t0 < n_terms; t0 += nt) {
+            double* t = tb + (size_t)buf * nt * 128;
+            const uint32_t t1 = min(t0 + nt, n_terms);
+#pragma unroll 2
+            for (uint32_t i = t0 + wave; i < t1; i += kFinishWaves) {
+                const uint32_t p = i & (P - 1), ds = i >> lgP, side = ds & 1u, d = ds >> 1;
+                const long long* rd = cells + ((size_t)p * C + d) * RS;
+                const long long* rw = cells + ((size_t)p * C + K) * RS;
+                const long long td = rd[tot_at], tw = rw[tot_at];
+                long long xd = rd[col], xw = rw[col];
+                if (oh) {   // equality split: the bin itself is the TRUE side
+                    xd = td - (xd - (b > 0 ? rd[prev_at] : 0));
+                    xw = tw - (xw - (b > 0 ? rw[prev_at] : 0));
+                }
+                const double s = (double)(side == 0 ? xd : td - xd) * inv_d;
+                const double w = (double)(side == 0 ? xw : tw - xw) * inv_w;
+                double x, y = 0.0;
+                if (sf > 1) {
+                    x = leaf_score_term(sf, s, w);
+                } else {
+                    const double q = s / (w + l2);
+                    const double avg = w > 0.0 ? q : 0.0;
+                    x = avg * s;
+                    y = avg * avg * w;
+                }
+                t[(i - t0) * 128 + lane] = x;
+                t[(i - t0) * 128 + 64 + lane] = y;
+            }
+            __syncthreads();
+            if (wave < 2) {
+                const double* src = t + wave * 64 + lane;
+#pragma unroll 8
+                for (uint32_t u = 0; u < t1 - t0; ++u) run += src[u * 128];
+            }
+            if (n_terms > nt) buf ^= 1u;
+            else if (k + 1 < slices) __syncthreads();   // one buffer: read before the next slice's terms
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kFinishSlices; ++j) acc[j] = j == k ? run : acc[j];
+    }
+    if (wave == 1)
+#pragma unroll
+        for (uint32_t k = 0; k < kFinishSlices; ++k) red[k][lane] = acc[k];
+    __syncthreads();
+    if (wave != 0) return;   // no barrier follows
+    double score = -INFINITY;
+    uint32_t bb = 0;
+    for (uint32_t k = 0; k < slices; ++k) {   // slices in border order: strict first-wins
+        double num = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < kFinishSlices; ++j) num = j == k ? acc[j] : num;
+        double v = sf == 0 ? num / sqrt(red[k][lane]) : num;
+        // the model_size_reg weight of a CTR column multiplies every candidate's score
+        const uint32_t f = f0 + g, b = wide ? s0 + 64u * k + lane : gb;
+        if (fweight) v = fweight[f] * v;
+        if (!on || b >= n_cand[f] || v != v) v = -INFINITY;
+        if (v > score) {
+            score = v;
+            bb = b;
+        }
+    }
+    if (nf > 1) {   // lane g scans feature f0 + g's B borders in order
+        red[0][lane] = score;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < nfe) {
+            double best = -INFINITY;
+            uint32_t bk = 0;
+            for (uint32_t k = 0; k < B; ++k) {
+                const double v = red[0][lane * B + k];
+                if (v > best) {
+                    best = v;
+                    bk = k;
+                }
+            }
+            best_score[f0 + lane] = best;
+            best_bin[f0 + lane] = bk;
         }
         return;
     }
-    const bool oh = one_hot != nullptr && one_hot[f] != 0;
-    const uint32_t BT = (B + 63) & ~63u;
-    const uint32_t Q = min(kFinishThreads / BT, P);             // groups that take parents
-    const uint32_t PW = min(kFinishParents, (P + Q - 1) / Q);   // parents of a group per slab
-    const uint32_t q = threadIdx.x / BT, b = threadIdx.x - q * BT;
-    const uint32_t bc = min(b, B - 1), bq = bc > 0 ? bc - 1 : 0;
-    const long long* base = kLds ? fcell : hist + (size_t)f * B;
-    const size_t stride = kLds ? B : (size_t)F * B;   // from one (leaf, channel) row to the next
-    double num = 0.0, den = 0.0;
-    den += 1e-100;
-    for (uint32_t side = 0; side < 2; ++side)
-        for (uint32_t p0 = 0; p0 < P; p0 += Q * PW) {
-            const uint32_t mine = p0 + q * PW;
-            double x[kFinishParents], y[kFinishParents];
-            if (q < Q) {
-#pragma unroll
-                for (uint32_t u = 0; u < kFinishParents; ++u) {
-                    x[u] = y[u] = 0.0;
-                    const uint32_t p = mine + u;
-                    if (u >= PW || p >= P) continue;   // uniform over the group
-                    const long long* rd = base + (size_t)(2u * p) * stride;
-                    const long long* rw = rd + stride;
-                    const long long pd = rd[bc], pw = rw[bc], td = rd[B - 1], tw = rw[B - 1];
-                    long long xd, xw;
-                    if (!oh) {
-                        xd = side == 0 ? pd : td - pd;
-                        xw = side == 0 ? pw : tw - pw;
-                    } else {
-                        const long long vd = pd - (b > 0 ? rd[bq] : 0), vw = pw - (b > 0 ? rw[bq] : 0);
-                        xd = side == 0 ? td - vd : vd;
-                        xw = side == 0 ? tw - vw : vw;
-                    }
-                    const double s = (double)xd * inv_d, w = (double)xw * inv_w;
-                    if (sf > 1) {
-                        x[u] = leaf_score_term(sf, s, w);
-                    } else {
-                        const double t = s / (w + l2);
-                        const double avg = w > 0.0 ? t : 0.0;
-                        x[u] = avg * s;
-                        y[u] = avg * avg * w;
-                    }
-                }
-            }
-            // the groups' turns; a slab's groups past P have nothing to add
-            const uint32_t turns = min(Q, (P - p0 + PW - 1) / PW);
-            for (uint32_t g = 0; g < turns; ++g) {
-                if (q == g) {
-                    if (side + p0 + g > 0) {
-                        num = ch_num[b];
-                        den = ch_den[b];
-                    }
-#pragma unroll
-                    for (uint32_t u = 0; u < kFinishParents; ++u) {
-                        if (u >= PW || mine + u >= P) continue;
-                        num += x[u];
-                        if (sf <= 1) den += y[u];
-                    }
-                    ch_num[b] = num;
-                    ch_den[b] = den;
-                }
-                __syncthreads();
-            }
-        }
-    double score = -INFINITY;
-    uint32_t bb = b;
-    if (q == 0) {
-        num = ch_num[b];
-        den = ch_den[b];
-        score = sf == 0 ? num / sqrt(den) : num;
-        // the model_size_reg weight of a CTR column multiplies every candidate's score
-        if (fweight) score = fweight[f] * score;
-        if (b >= nc || score != score) score = -INFINITY;
-        for (int o = 32; o > 0; o >>= 1) {
-            double os = __shfl_xor(score, o, 64);
-            uint32_t ob = __shfl_xor(bb, o, 64);
-            if (os > score || (os == score && ob < bb)) {
-                score = os;
-                bb = ob;
-            }
-        }
-        if (lane == 0) {
-            red_s[wave] = score;
-            red_b[wave] = bb;
+    for (int o = 32; o > 0; o >>= 1) {
+        const double os = __shfl_xor(score, o, 64);
+        const uint32_t ob = __shfl_xor(bb, o, 64);
+        if (os > score || (os == score && ob < bb)) {
+            score = os;
+            bb = ob;
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 1; k < BT / 64; ++k)
-            if (red_s[k] > score || (red_s[k] == score && red_b[k] < bb)) {
-                score = red_s[k];
-                bb = red_b[k];
-            }
-        best_score[f] = score;
-        best_bin[f] = bb;
+    if (lane == 0) {
+        best_score[(size_t)f0 * n_parts + part] = score;
+        best_bin[(size_t)f0 * n_parts + part] = bb;
     }
 }
 
@@ -2935,47 +3066,55 @@ __global__ __launch_bounds__(512) void score_chain_kernel(
 template <uint32_t NT>
 __device__ __forceinline__ SplitRec block_argmax(const double* __restrict__ best_score,
                                                  const uint32_t* __restrict__ best_bin,
-                                                 const uint8_t* __restrict__ one_hot, uint32_t F) {
+                                                 const uint8_t* __restrict__ one_hot, uint32_t F,
+                                                 uint32_t parts /* entries a feature, in border order */) {
     constexpr uint32_t NW = NT / 64;
     __shared__ double rs[NW];
-    __shared__ uint32_t rk[NW];
+    __shared__ uint32_t rk[NW], rb[NW];
     double s = -INFINITY;
-    uint32_t key = 0xFFFFFFFFu;
-    for (uint32_t f = threadIdx.x; f < F; f += NT) {
-        const double v = best_score[f];
-        const uint32_t k = f + ((one_hot && one_hot[f]) ? F : 0u);
+    uint32_t key = 0xFFFFFFFFu, bin = 0;   // the bin travels with its score: no load after the reduction
+    const uint32_t n_ent = F * parts;
+    for (uint32_t e = threadIdx.x; e < n_ent; e += NT) {
+        const double v = best_score[e];
+        const uint32_t vb = best_bin[e];
+        const uint32_t k = e + ((one_hot && one_hot[e / parts]) ? n_ent : 0u);
         if (v > s || (v == s && k < key)) {
             s = v;
             key = k;
+            bin = vb;
         }
     }
     for (int o = 32; o > 0; o >>= 1) {
-        double os = __shfl_xor(s, o, 64);
-        uint32_t ok = __shfl_xor(key, o, 64);
+        const double os = __shfl_xor(s, o, 64);
+        const uint32_t ok = __shfl_xor(key, o, 64), ob = __shfl_xor(bin, o, 64);
         if (os > s || (os == s && ok < key)) {
             s = os;
             key = ok;
+            bin = ob;
         }
     }
     const uint32_t wave = threadIdx.x >> 6;
     if (lane_id() == 0) {
         rs[wave] = s;
         rk[wave] = key;
+        rb[wave] = bin;
     }
     __syncthreads();
     s = rs[0];
     key = rk[0];
+    bin = rb[0];
 #pragma unroll
     for (uint32_t k = 1; k < NW; ++k)
         if (rs[k] > s || (rs[k] == s && rk[k] < key)) {
             s = rs[k];
             key = rk[k];
+            bin = rb[k];
         }
     SplitRec r;
     r.valid = (s > -INFINITY) ? 1u : 0u;
-    r.feature = key == 0xFFFFFFFFu ? 0u : (key >= F ? key - F : key);
-    r.one_hot = (key != 0xFFFFFFFFu && key >= F) ? 1u : 0u;
-    r.bin = r.valid ? best_bin[r.feature] : 0u;
+    r.feature = key == 0xFFFFFFFFu ? 0u : (key >= n_ent ? key - n_ent : key) / parts;
+    r.one_hot = (key != 0xFFFFFFFFu && key >= n_ent) ? 1u : 0u;
+    r.bin = r.valid ? bin : 0u;
     r.score = s;
     return r;
 }
@@ -2984,8 +3123,8 @@ __device__ __forceinline__ SplitRec block_argmax(const double* __restrict__ best
 static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __restrict__ best_score,
                                                              const uint32_t* __restrict__ best_bin,
                                                              const uint8_t* __restrict__ one_hot, uint32_t F,
-                                                             SplitRec* __restrict__ out) {
-    const SplitRec r = block_argmax<1024>(best_score, best_bin, one_hot, F);
+                                                             uint32_t parts, SplitRec* __restrict__ out) {
+    const SplitRec r = block_argmax<1024>(best_score, best_bin, one_hot, F, parts);
     if (threadIdx.x == 0) *out = r;
 }
 
@@ -3004,8 +3143,11 @@ static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __res
 // and the scan of the counts ride in the kernels that need their results: each workgroup of
 // split_count repeats the argmax, each workgroup of compact sums the counts before it.
 // ---------------------------------------------------------------------------------
-constexpr uint32_t kPartRows = 4096;   // rows per partition block (4 waves)
-constexpr uint32_t kPartWaveRows = kPartRows / 4;
+// Rows per wave (4 waves a workgroup): PR = 1024 keeps the counts few at many rows, 256 shortens
+// the waves' chains (a row a lane at a time) where workgroups are too few to fill the chip.
+constexpr uint32_t kPartSmall = 256, kPartLarge = 1024;
+constexpr uint64_t kPartSmallMaxRows = 1u << 20;
+inline uint32_t part_wave_rows(uint64_t n) { return n <= kPartSmallMaxRows ? kPartSmall : kPartLarge; }
 // Workgroups a group of the counts covers: compact reads groups + 4 kGroupBlocks counts per leaf
 // (10M rows: 153 + 64), and a group count takes kGroupBlocks atomics on one address (about 66 ns
 // each, one after another, 1 us in all).
@@ -3029,29 +3171,29 @@ __device__ __forceinline__ uint64_t wave_peers(uint32_t key, bool valid, uint32_
     return mask;
 }
 
-// Leaf update of one level and the row counts of every new leaf.  Each wave owns kPartWaveRows
+// Leaf update of one level and the row counts of every new leaf.  Each wave owns PR
 // consecutive rows; its counts go to cnt[wave][leaf].  Up to 4 new leaves a
 // leader per distinct leaf adds the popcount of its peers (one ballot per key bit, so no LDS
 // cell takes more than one add per 64 rows); with more leaves every row adds 1 to its leaf's
 // LDS counter (few lanes share a counter, and the ballots would grow with the level).
 // kArgmax: the level's split is the argmax of the features' best candidates, taken by every
 // workgroup while its rows' leaves load (workgroup 0 stores it); else it is read from *split.
-template <bool kArgmax>
+template <bool kArgmax, uint32_t PR>
 static __global__ __launch_bounds__(256) void split_count_kernel(
     const uint8_t* __restrict__ cols, uint64_t n, SplitRec* __restrict__ split,
     const double* __restrict__ best_score, const uint32_t* __restrict__ best_bin,
-    const uint8_t* __restrict__ one_hot, uint32_t F, uint32_t level, uint16_t* __restrict__ leaf,
+    const uint8_t* __restrict__ one_hot, uint32_t F, uint32_t parts, uint32_t level, uint16_t* __restrict__ leaf,
     uint32_t* __restrict__ cnt, uint32_t* __restrict__ gcnt /* nullable: no counts */) {
     __shared__ uint32_t c[4][kMaxLeaves];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t n_new = 2u << level;
     for (uint32_t k = lane; k < n_new; k += 64) c[wave][k] = 0;
     const uint64_t wid = (uint64_t)blockIdx.x * 4 + wave;
-    const uint64_t beg = wid * kPartWaveRows;
-    const uint64_t end = min(beg + kPartWaveRows, n);
+    const uint64_t beg = wid * PR;
+    const uint64_t end = min(beg + PR, n);
     // every load of the wave's rows is issued before any is used (one memory round trip
     // per wave instead of one per 64 rows)
-    constexpr int U = kPartWaveRows / 64;
+    constexpr int U = PR / 64;
     uint32_t bin[U], lf[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -3060,7 +3202,7 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
     }
     SplitRec s;
     if (kArgmax) {
-        s = block_argmax<256>(best_score, best_bin, one_hot, F);
+        s = block_argmax<256>(best_score, best_bin, one_hot, F, parts);
         if (blockIdx.x == 0 && threadIdx.x == 0) *split = s;
     } else {
         s = *split;
@@ -3112,7 +3254,7 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
 // (at most 128 parents, one wave) and block 0 stores it for the kernels after.  The totals and
 // the rows before a block are sums of the groups' counts and of its own group's wave counts
 // (integers: the order does not matter), read while the block's leaf ids load.
-template <int SPW>
+template <int SPW, uint32_t PR>
 static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __restrict__ leaf, uint64_t n,
                                                       uint32_t level, const uint32_t* __restrict__ cnt,
                                                       const uint32_t* __restrict__ gcnt, uint32_t n_groups,
@@ -3127,9 +3269,9 @@ static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __r
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t n_parent = 1u << level, n_new = 2u << level;
     const uint64_t wid = (uint64_t)blockIdx.x * 4 + wave;
-    const uint64_t beg = wid * kPartWaveRows;
-    const uint64_t end = min(beg + kPartWaveRows, n);
-    constexpr int U = kPartWaveRows / 64;
+    const uint64_t beg = wid * PR;
+    const uint64_t end = min(beg + PR, n);
+    constexpr int U = PR / 64;
     uint32_t lfs[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {   // all loads in flight before the first use

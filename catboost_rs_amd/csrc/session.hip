@@ -129,11 +129,15 @@ struct cbh_session {
     uint16_t* leaf = nullptr;
     uint32_t* idx = nullptr;
     long long* hist[2] = {nullptr, nullptr};
-    long long* raw = nullptr;        // the fill's sums of the directly built children, [segment][C][F][B]
+    // the fill's sums of the directly built children, [segment][C][F][B]: level l's in
+    // raw[l & raw_alt] (raw_alt: several workgroups read a row, so the next level clears it)
+    long long* raw[2] = {nullptr, nullptr};
+    uint32_t raw_alt = 0;
+    bool fuse_finish = false;        // finish_score_kernel at every level
     size_t hist_cells_max = 0, raw_cells = 0;
     uint32_t* cnt = nullptr;         // partition: row counts [wave][leaf] of the level
     uint32_t* gcnt = nullptr;        // [level][group][leaf], cleared once per tree
-    uint32_t n_part_blocks = 0, n_groups_part = 0;
+    uint32_t n_part_blocks = 0, n_groups_part = 0, part_rows = kPartLarge;   // rows per wave
     LevelPlan* plans = nullptr;   // [depth]
     SplitRec* splits = nullptr;   // [depth]
     double* best_score = nullptr;
@@ -295,7 +299,7 @@ struct cbh_session {
 
     void release() {
         dfree(rows); dfree(cols); dfree(weight); dfree(target); dfree(approx); dfree(sstat);
-        dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(raw); dfree(cnt);
+        dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(raw[0]); dfree(raw[1]); dfree(cnt);
         dfree(gcnt); dfree(best_score);
         dfree(best_bin); dfree(n_cand); dfree(one_hot); dfree(scales);
         dfree(leaf_sums); dfree(leaf_scaled); dfree(jump);
@@ -410,6 +414,12 @@ int validate_config(const cbh_config* cfg, uint32_t n_bins, uint64_t n, uint32_t
     return CBH_OK;
 }
 
+int launch_zero(long long* p, size_t n, hipStream_t st) {
+    zero_i64_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(p, n);
+    HIP_TRY(hipGetLastError());
+    return CBH_OK;
+}
+
 int session_alloc(cbh_session* s) {
     const uint64_t n = s->n;
     CHECK(dalloc(&s->rows, (size_t)n * s->Ws));
@@ -424,12 +434,9 @@ int session_alloc(cbh_session* s) {
     s->hist_cells_max = per_leaf << (s->depth - 1);
     CHECK(dalloc(&s->hist[0], s->hist_cells_max));
     CHECK(dalloc(&s->hist[1], s->hist_cells_max));
-    // zero outside a level's fill and finishing, which clears what it reads: cleared here once
     s->raw_cells = per_leaf << (s->depth >= 2 ? s->depth - 2 : 0);
-    CHECK(dalloc(&s->raw, s->raw_cells));
-    zero_i64_kernel<<<grid_for(s->raw_cells, 256, 8192), 256, 0, s->stream>>>(s->raw, s->raw_cells);
-    HIP_TRY(hipGetLastError());
-    s->n_part_blocks = (uint32_t)((n + kPartRows - 1) / kPartRows);
+    s->part_rows = part_wave_rows(n);
+    s->n_part_blocks = (uint32_t)((n + 4 * s->part_rows - 1) / (4 * s->part_rows));
     // per level of up to 2^(depth - 1) new leaves: counts [wave][leaf], and per group of
     // workgroups [level][group][leaf]
     CHECK(dalloc(&s->cnt, ((size_t)s->n_part_blocks * 4) << (s->depth - 1)));
@@ -452,8 +459,8 @@ int session_alloc(cbh_session* s) {
         s->pin_bounds = (Bounds*)(s->pin_out + o_bounds);
         s->pin_leaves = (double*)(s->pin_out + o_leaves);
     }
-    CHECK(dalloc(&s->best_score, s->F));
-    CHECK(dalloc(&s->best_bin, s->F));
+    CHECK(dalloc(&s->best_score, (size_t)s->F * kFinishSlices));
+    CHECK(dalloc(&s->best_bin, (size_t)s->F * kFinishSlices));
     CHECK(dalloc(&s->n_cand, s->F));
     CHECK(dalloc(&s->scales, 1));
     const uint32_t CL = s->K == 1 ? 3 : s->K + s->K * (s->K + 1) / 2;
@@ -1190,9 +1197,8 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
     CHECK(with_k((int)s->K, [&](auto kc) {
         constexpr int K = decltype(kc)::value;
         CHECK(set_fill_attr<K + 1>(s->tiles.lds_bytes));
-        if (K == 1)
-            HIP_TRY(hipFuncSetAttribute((const void*)finish_score_kernel<true>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFinishLdsMax));
+        HIP_TRY(hipFuncSetAttribute((const void*)finish_score_kernel<K>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)kFinishLdsMax));
         const size_t lds = ((size_t)1 << s->depth) * (size_t)leaf_cells<K>() * sizeof(long long);
         HIP_TRY(hipFuncSetAttribute((const void*)leaf_reduce_kernel<K>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1220,6 +1226,21 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
         CHECK(dalloc(&s->one_hot, F));
         HIP_TRY(hipMemcpy(s->one_hot, s->one_hot_host.data(), F, hipMemcpyHostToDevice));
     }
+    // the raw buffers: zero outside a level's fill and finishing, cleared here once
+    // (K > 1 with at most 64 candidates: the chained scorer, several features a wave; measured
+    // 1M x 4096 x 20 bins, K = 10, depth 8: 8.97 against 9.99 ms a tree)
+    const bool chain_ok = s->K > 1 && s->score_chain && s->cfg.score_function <= CBH_SCORE_L2 && s->max_cand <= 64;
+    s->fuse_finish = !s->pairwise && !chain_ok;
+    for (uint32_t l = 0; l < s->depth && s->fuse_finish; ++l) {
+        const FinishPlan pl = plan_finish(1u << l, s->K, F, n_bins, s->cus, any_oh);
+        if (pl.lds == 0) s->fuse_finish = false;
+        if (pl.n_parts > 1) s->raw_alt = 1;
+    }
+    if (!s->fuse_finish) s->raw_alt = 0;
+    for (uint32_t k = 0; k <= s->raw_alt; ++k) {
+        CHECK(dalloc(&s->raw[k], s->raw_cells));
+        CHECK(launch_zero(s->raw[k], s->raw_cells, s->stream));
+    }
     // feature-major u8 bins in place, then pack the row-major words on the device
     CHECK(load_cols(s.get()));
     pack_rows_kernel<<<grid_for((uint64_t)n * s->Ws, 256), 256, 0, s->stream>>>(s->cols, n, F, s->Ws, s->rows);
@@ -1241,12 +1262,6 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
     }
     HIP_TRY(hipStreamSynchronize(s->stream));
     *out = s.release();
-    return CBH_OK;
-}
-
-int launch_zero(long long* p, size_t n, hipStream_t st) {
-    zero_i64_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(p, n);
-    HIP_TRY(hipGetLastError());
     return CBH_OK;
 }
 
@@ -1606,7 +1621,8 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         apply_prev && !s->ranking ? s->leaf_scaled : nullptr,   // a pair loss applied them above
         s->smp_dev, s->jt(), use_host_sample ? s->host_sample : nullptr, s->sstat, newton, s->partials,
         s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, s->gcnt,
-        (uint32_t)group_count_off(s->n_groups_part, s->depth - 1));
+        (uint32_t)group_count_off(s->n_groups_part, s->depth - 1),
+        s->raw_alt ? s->raw[(s->depth - 1) & 1] : nullptr, s->raw_alt ? s->raw_cells : 0);
     HIP_TRY(hipGetLastError());
     scales_kernel<<<1, 256, 0, st>>>(s->partials, pgrid, s->bounds, s->scales,
                                      (s->packed || s->pkk) ? s->pack_bits : 0, s->count ? 1 : 0);
@@ -1631,6 +1647,7 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         long long* par = s->hist[(level + 1) & 1];
         const uint32_t n_leaves = 1u << level;
         // ---- fill, into the raw buffer ----
+        long long* raw = s->raw[level & s->raw_alt];
         const uint32_t nt = s->tiles.n_tiles;
         const uint32_t G = s->fill_ranges;
         const uint32_t* lidx = level == 0 ? nullptr : s->idx;
@@ -1648,27 +1665,27 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         if (s->packed && level == 0)
             fill_packed_kernel<false, false><<<s->pk_dense.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, s->spack, nullptr, s->pk_dense.tiles16, s->F, s->B,
-                s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, s->pk_swap, nullptr, 0u, s->scales);
+                s->pk_dense.ranges, s->pk_dense.ranges_n, raw, s->pk_swap, nullptr, 0u, s->scales);
         else if (s->packed)
             fill_packed_kernel<true, false><<<s->pk_gath.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
-                s->pk_gath.ranges, 0u, s->raw, s->pk_swap, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
+                s->pk_gath.ranges, 0u, raw, s->pk_swap, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
         else if (s->count && level == 0)
             fill_packed_kernel<false, true><<<s->pk_dense.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, s->spack, nullptr, s->pk_dense.tiles16, s->F, s->B,
-                s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, 0u, nullptr, 0u, s->scales);
+                s->pk_dense.ranges, s->pk_dense.ranges_n, raw, 0u, nullptr, 0u, s->scales);
         else if (s->count)
             fill_packed_kernel<true, true><<<s->pk_gath.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
-                s->pk_gath.ranges, 0u, s->raw, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
+                s->pk_gath.ranges, 0u, raw, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
         else if (s->tiled && level == 0)
             fill_exact_kernel<false><<<s->pk_dense.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, (const long long*)s->sstat, nullptr, s->pk_dense.tiles16, s->F,
-                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, s->raw, nullptr, 0u, s->ex_sets, s->scales);
+                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, raw, nullptr, 0u, s->ex_sets, s->scales);
         else if (s->tiled)
             fill_exact_kernel<true><<<s->pk_gath.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, (const long long*)s->sstat, (const long long*)s->sseq,
-                s->pk_gath.tiles16, s->F, s->B, s->pk_gath.ranges, s->pk_gath.ranges_n, s->raw,
+                s->pk_gath.tiles16, s->F, s->B, s->pk_gath.ranges, s->pk_gath.ranges_n, raw,
                 s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->ex_sets, s->scales);
         else if (s->pkk) {
             const size_t lds = (size_t)kPkkCells * sizeof(unsigned long long);
@@ -1682,57 +1699,57 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             const uint32_t npf = w0_use ? NPl - 1 : NPl;
             if (level == 0) s->l0_cached = w0_use;
             if (w0_use)
-                HIP_TRY(hipMemcpyAsync(s->raw + (size_t)(C - 1) * s->F * s->B, s->w0_cache,
+                HIP_TRY(hipMemcpyAsync(raw + (size_t)(C - 1) * s->F * s->B, s->w0_cache,
                                        sizeof(long long) * s->F * s->B, hipMemcpyDeviceToDevice, st));
             // (small tiles: 4 cells per thread, their registers leaving room for 8 blocks in flight)
             const size_t lds4 = (size_t)4 * kPkkThreads * sizeof(unsigned long long);
             if (s->pks && s->pks_small && level == 0)
                 fill_pks_kernel<C, false, 4, 8><<<grid, kPkkThreads, lds4, st>>>(
-                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
+                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw, npf);
             else if (s->pks && s->pks_small)
                 fill_pks_kernel<C, true, 4, 8><<<grid, kPkkThreads, lds4, st>>>(
-                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
+                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw, npf);
             else if (s->pks && level == 0)
                 fill_pks_kernel<C, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
+                    s->pks_a, s->pks_b, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw, npf);
             else if (s->pks)
                 fill_pks_kernel<C, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw, npf);
+                    s->pks_a, s->pks_b, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw, npf);
             else if (s->use_skip && level == 0)
                 fill_pkk_kernel<C, true, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
+                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw,
                     s->skip_bin, npf);
             else if (s->use_skip)
                 fill_pkk_kernel<C, true, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
+                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw,
                     s->skip_bin, npf);
             else if (level == 0)
                 fill_pkk_kernel<C, false, false><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
+                    s->rows, s->W, s->Ws, n, nullptr, nullptr, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw,
                     nullptr, npf);
             else
                 fill_pkk_kernel<C, false, true><<<grid, kPkkThreads, lds, st>>>(
-                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, s->raw,
+                    s->rows, s->W, s->Ws, n, lidx, lplan, s->spack, s->pkk_tiles, s->F, s->B, s->pkk_ranges, raw,
                     nullptr, npf);
         } else if (s->use_skip)
             fill_kernel<C, true><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, raw,
                 s->skip_bin, (int)s->tiles.bin_major);
         else if (C == 2 && s->pairwise)
             // PairLogitPairwise scores from the der channel and the pair statistics alone: the
             // weight channel is left out of the fill (its cells stay zero; such sessions refuse
             // histogram capture)
             fill_kernel<2, false, 1><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, raw,
                 nullptr, (int)s->tiles.bin_major);
         else
             fill_kernel<C, false><<<G * nt, 1024, s->tiles.lds_bytes, st>>>(
-                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, s->raw,
+                s->rows, s->W, s->Ws, n, lidx, lplan, (const long long*)s->sstat, nt, s->tiles.tw, s->F, s->B, G, raw,
                 nullptr, (int)s->tiles.bin_major);
         HIP_TRY(hipGetLastError());
         CHECK(s->stage_end());
         if (s->pkk && level == 0 && s->w_static && !s->w0_ready) {   // the weight channel's cache
-            HIP_TRY(hipMemcpyAsync(s->w0_cache, s->raw + (size_t)(C - 1) * s->F * s->B, sizeof(long long) * s->F * s->B,
+            HIP_TRY(hipMemcpyAsync(s->w0_cache, raw + (size_t)(C - 1) * s->F * s->B, sizeof(long long) * s->F * s->B,
                                    hipMemcpyDeviceToDevice, st));
             s->w0_ready = true;
         }
@@ -1752,9 +1769,8 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         }
         // ---- histogram finishing: dominant bins, prefix form, siblings; K = 1 with the scoring ----
         const bool last = level + 1 == s->depth;
-        // one workgroup per feature finishes and scores it; many features fill the chip with the
-        // finishing's own waves and the scorer's smaller workgroups (see kFinishMaxFeatures)
-        const bool finish = K == 1 && !s->pairwise && s->F <= kFinishMaxFeatures;
+        const bool finish = s->fuse_finish;
+        uint32_t parts = 1;   // best entries a feature
         if (!finish) {
             CHECK(s->stage_begin(kStDerive));
             // (PairLogitPairwise fills and reads the der channel only)
@@ -1765,16 +1781,16 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             const uint32_t* sb = s->use_skip ? s->skip_bin : nullptr;
             if (s->B <= 72)   // 8 lanes per row
                 hist_prefix_group_kernel<8, 9><<<(unsigned)((rows + 31) / 32), 256, 0, st>>>(
-                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else if (s->B <= 80)   // 16 lanes per row
                 hist_prefix_group_kernel<16, 5><<<(unsigned)((rows + 15) / 16), 256, 0, st>>>(
-                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else if (s->B <= 96)   // a half-wave per row
                 hist_prefix_group_kernel<32, 3><<<(unsigned)((rows + 7) / 8), 256, 0, st>>>(
-                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             else
                 hist_prefix_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(
-                    s->raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
             HIP_TRY(hipGetLastError());
             CHECK(s->stage_end());
         }
@@ -1793,10 +1809,11 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         } else if (finish) {
             // (the last level's rows are read by nothing after it)
             const int keep = !last || s->hist_cap ? 1 : 0;
-            const size_t lds = finish_lds(n_leaves, s->B);
-            const bool in_lds = lds <= kFinishLdsMax;
-            (in_lds ? finish_score_kernel<true> : finish_score_kernel<false>)<<<s->F, kFinishThreads, in_lds ? lds : 0, st>>>(
-                s->raw, cur, lplan, n_seg, level > 0 ? par : nullptr, n_leaves, s->F, s->B, keep,
+            const FinishPlan pl = plan_finish(n_leaves, K, s->F, s->B, s->cus, s->one_hot != nullptr);
+            parts = pl.n_parts;
+            finish_score_kernel<K><<<pl.blocks, kFinishThreads, pl.lds, st>>>(
+                raw, cur, lplan, n_seg, level > 0 ? par : nullptr, n_leaves, s->F, s->B, pl.nf, pl.m, pl.n_parts, pl.nt,
+                keep, s->raw[(level + 1) & 1], level >= 1 ? std::max(1u, n_seg / 2) : 0u,
                 s->use_skip ? s->skip_bin : nullptr, s->seg_tot, s->n_cand, s->one_hot, s->scales, s->l2, sfn,
                 s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr);
         } else if (chain) {
@@ -1825,47 +1842,49 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                         sfn, s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr, s->chain_spin,
                         &s->bounds->device_err, nf);
             }
-        } else if (s->max_cand <= 64)
-            score_kernel<K, 1><<<s->F, 64, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+        } else if constexpr (K > 1) {   // (K = 1 always finishes and scores in one launch)
+            if (s->max_cand <= 64)
+                score_kernel<K, 1><<<s->F, 64, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                    s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
-        else if (s->max_cand <= 128)
-            score_kernel<K, 2><<<s->F, 128, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+            else if (s->max_cand <= 128)
+                score_kernel<K, 2><<<s->F, 128, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                     s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
-        else
-            score_kernel<K, 4><<<s->F, 256, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
+            else
+                score_kernel<K, 4><<<s->F, 256, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                     s->scales, s->l2, sfn, s->best_score, s->best_bin,
                                                    s->ctr_n ? s->fweight : nullptr);
+        }
         HIP_TRY(hipGetLastError());
         if (s->hist_cap)   // the level's histograms as the scorer reads them (inspection only)
             HIP_TRY(hipMemcpyAsync(s->hist_cap + s->hist_cap_off[level], cur, sizeof(long long) * per_leaf * n_leaves,
                                    hipMemcpyDeviceToDevice, st));
-        const bool fuse_argmax = s->F <= kArgmaxFuse;
+        const bool fuse_argmax = s->F * parts <= kArgmaxFuse;
         if (!fuse_argmax) {
             argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F,
-                                              s->splits + level);
+                                              parts, s->splits + level);
             HIP_TRY(hipGetLastError());
         }
         CHECK(s->stage_end());
         // ---- partition ----
         CHECK(s->stage_begin(kStPartition));
         uint32_t* gcnt = last ? nullptr : s->gcnt + group_count_off(s->n_groups_part, level);
-        (fuse_argmax ? split_count_kernel<true> : split_count_kernel<false>)<<<NB, 256, 0, st>>>(
-            s->cols, n, s->splits + level, s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F, level,
-            s->leaf, s->cnt, gcnt);
+        const bool small = s->part_rows == kPartSmall;
+        (fuse_argmax ? (small ? split_count_kernel<true, kPartSmall> : split_count_kernel<true, kPartLarge>)
+                     : (small ? split_count_kernel<false, kPartSmall> : split_count_kernel<false, kPartLarge>))
+            <<<NB, 256, 0, st>>>(s->cols, n, s->splits + level, s->best_score, s->best_bin,
+                                 s->pairwise ? nullptr : s->one_hot, s->F, parts, level, s->leaf, s->cnt, gcnt);
         HIP_TRY(hipGetLastError());
         if (!last) {
-            const uint32_t ng = s->n_groups_part;
-            if (s->packed || s->count)   // the listed rows' packed statistic
-                compact_kernel<1><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
-                                                      s->spack, s->sseq);
-            else if (s->tiled && s->sseq)   // both f64 score channels of the listed rows
-                compact_kernel<2><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
-                                                      (const unsigned long long*)s->sstat, s->sseq);
-            else
-                compact_kernel<0><<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, ng, s->plans + level, s->idx,
-                                                      nullptr, nullptr);
+            // beside the index: the listed row's packed statistic, or both f64 score channels
+            const int spw = s->packed || s->count ? 1 : s->tiled && s->sseq ? 2 : 0;
+            const unsigned long long* sp = spw == 1 ? s->spack : spw == 2 ? (const unsigned long long*)s->sstat : nullptr;
+            (spw == 1   ? (small ? compact_kernel<1, kPartSmall> : compact_kernel<1, kPartLarge>)
+             : spw == 2 ? (small ? compact_kernel<2, kPartSmall> : compact_kernel<2, kPartLarge>)
+                        : (small ? compact_kernel<0, kPartSmall> : compact_kernel<0, kPartLarge>))
+                <<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, s->n_groups_part, s->plans + level, s->idx, sp,
+                                     spw ? s->sseq : nullptr);
             HIP_TRY(hipGetLastError());
         }
         CHECK(s->stage_end());
@@ -2244,7 +2263,7 @@ int cbh_session_read_approx(cbh_session* s, double* approx_out, uint64_t n_times
             prepare_kernel<K><<<grid_for(s->n, 256, kPrepBlocks), 256, 0, s->stream>>>(
                 s->n, s->cfg.loss == CBH_LOSS_RMSE ? 0 : 1, s->approx, s->target, s->weight, s->leaf,
                 s->leaf_scaled, s->smp_dev + 1, s->jt(), nullptr, s->sstat, 0, s->partials, nullptr,
-                nullptr, nullptr, 0u);
+                nullptr, nullptr, 0u, nullptr, 0);
             HIP_TRY(hipGetLastError());
             return CBH_OK;
         });
