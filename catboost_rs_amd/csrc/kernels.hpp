@@ -1567,6 +1567,192 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
 }
 
 // ---------------------------------------------------------------------------------
+// Narrow-tile exact fill: tiles of 2 words (8 features), C channels of a row, one exact 64-bit LDS
+// atomic per (row, feature, channel) as in the tiled exact fill above.
+//
+// At mid-size inputs what a launch costs beside its atomics is the flush: every workgroup adds
+// its LDS image to the raw buffer with global atomics (about 1e11 cells/s over the whole chip, 45-80
+// us for 256 workgroups of 16K cells), and with every CU at work the images' total is the tile
+// width times a constant.  These tiles flush a quarter of what the 32-feature tiles do for the
+// same atomics (tiles of 16 features measured 3-8% slower a tree); they read a row's statistics
+// once per 8 features, which costs at many rows and features (narrow_pays).
+// 100k x 50, 129 bins: 22 -> 9 us dense, 15 -> 9 us gathered; 300k x 60, 128 bins, 6 channels: 43
+// (one atomic per channel over feature-major LDS) -> 21 us.
+//
+// LDS [bin][ch][16] of u64.  A 16-lane DPP row takes 8 rows a pass, lane 2 j + w word w of row j;
+// the 16 positions it covers in a block of 1024 are staged one per lane (the channels' f64
+// values; gathered, the row index), lane 2 j + u that of row j in pass u, and pass u broadcasts
+// it over the row's two lanes (quad_perm).  Step k of a lane visits byte (k + j) & 3 of its word
+// into copy j / 4 of the 8 columns (the copies are summed at the flush): the 16 lanes of an atomic
+// hit 16 distinct columns, i.e. bank pairs, whatever the bins.
+//
+// Positions past the range read zero statistics (a buffer load past the resource returns 0) and
+// add 0; bins are below B everywhere, so every cell address is inside the B * C * 16 cells.
+// ---------------------------------------------------------------------------------
+constexpr uint32_t kNtThreads = 1024, kNtBlockRows = 1024, kNtWords = 2;
+__host__ __device__ constexpr size_t narrow_lds(uint32_t B, uint32_t C) { return (size_t)B * C * 16u * 8u; }
+constexpr size_t kNarrowLdsMax = 160 * 1024 - 256;
+
+template <int C>
+struct NtSet {
+    uint32_t w[2], ix;
+    unsigned long long st[C];
+};
+
+template <int C, bool kGather>
+struct NtRange {
+    unsigned long long* cells;
+    __amdgpu_buffer_rsrc_t rbase, ibase, sbase;
+    uint32_t row_bytes, wl4, l, j, r0, stat_bytes, pos, end;
+    bool seq;
+    uint32_t off8[4];
+    double md, mw;
+
+    __device__ __forceinline__ uint32_t staged(uint32_t bb) const {   // this lane's position in block bb
+        return bb + 16u * r0 + 8u * (l & 1u) + (l >> 1);
+    }
+    __device__ __forceinline__ uint32_t stage_ix(uint32_t bb) const {
+        const uint32_t p = staged(bb);
+        return ldw(ibase, 4u * (p < end ? p : pos));
+    }
+    template <int U>
+    __device__ __forceinline__ void load_word(NtSet<C>& S, uint32_t bb) const {
+        const uint32_t row = kGather ? quad_pair_bcast<U>(S.ix) : bb + 16u * r0 + 8u * U + j;
+        S.w[U] = ldw(rbase, row * row_bytes + wl4);
+    }
+    __device__ __forceinline__ void load(NtSet<C>& S, uint32_t bb, uint32_t ahead) const {
+        const uint32_t p = staged(bb);
+        const uint32_t so = p < end ? (kGather && !seq ? S.ix : p) * stat_bytes : kPastEnd16;
+#pragma unroll
+        for (int c = 0; c + 1 < C; c += 2) ldq2(sbase, p < end ? so + 8u * c : kPastEnd16, S.st[c], S.st[c + 1]);
+        if (C & 1) S.st[C - 1] = ldq(sbase, p < end ? so + 8u * (C - 1) : kPastEnd16);
+        load_word<0>(S, bb);
+        load_word<1>(S, bb);
+        if (kGather) S.ix = stage_ix(bb + ahead);
+    }
+    template <int U>
+    __device__ __forceinline__ void pass(const NtSet<C>& S, const unsigned long long* q) const {
+        unsigned long long v[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) v[c] = quad_pair_bcast64<U>(q[c]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t bin = __builtin_amdgcn_ubfe(S.w[U], off8[k], 8);
+            unsigned long long* cell = (unsigned long long*)((char*)cells + (__umul24(bin, C * 128u) + off8[k]));
+#pragma unroll
+            for (int c = 0; c < C; ++c) atomicAdd(cell + 16 * c, v[c]);
+        }
+    }
+    // (the weight channel is the last; a der-only fill, C == 1, has none)
+    __device__ __forceinline__ void consume(const NtSet<C>& S) const {
+        unsigned long long q[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) q[c] = stat_fixed(S.st[c], C > 1 && c == C - 1 ? mw : md);
+        pass<0>(S, q);
+        pass<1>(S, q);
+    }
+    __device__ __forceinline__ void run() const {
+        constexpr int NS = C <= 2 ? 4 : C <= 4 ? 3 : C <= 8 ? 2 : 1;   // blocks in flight (registers)
+        NtSet<C> S[NS];
+        if (kGather) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) S[s].ix = stage_ix(pos + s * kNtBlockRows);
+        }
+        // the sets load in the loop's order, so its first use waits for that set's loads only
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            load(S[s], pos + s * kNtBlockRows, NS * kNtBlockRows);
+            asm volatile("" ::: "memory");
+        }
+        for (uint32_t bb = pos;; bb += NS * kNtBlockRows) {   // workgroup-uniform
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                consume(S[s]);
+                if (bb + (s + 1) * kNtBlockRows >= end) return;
+                load(S[s], bb + (NS + s) * kNtBlockRows, NS * kNtBlockRows);
+            }
+        }
+    }
+};
+
+template <int C, bool kGather>
+static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
+    const uint32_t* __restrict__ trows /* tile-major 2-word slices (pack_tiles_kernel) */, uint32_t W, uint64_t n,
+    const uint32_t* __restrict__ idx, const LevelPlan* __restrict__ plan,
+    const double* __restrict__ sstat /* [n][CS] */, uint32_t CS,
+    const double* __restrict__ sseq /* kGather, nullable: [V][CS], the listed rows' channels in idx order */,
+    uint32_t n_tiles, uint32_t F, uint32_t B, uint32_t G, long long* __restrict__ raw /* [segment][CS][F][B] */,
+    const uint32_t* __restrict__ rows_rm /* nullable, kGather: row-major words, row_bytes a row */,
+    uint32_t row_bytes, const Scales* __restrict__ sc) {
+    extern __shared__ unsigned long long ex[];
+    // block -> (tile, range) as in fill_exact_kernel: all tiles of a range share one XCD's L2
+    const uint32_t pairs = n_tiles * G, per = (pairs + 7u) / 8u;
+    const uint32_t i = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || i >= pairs) return;   // workgroup-uniform, before any barrier
+    const uint32_t t = i % n_tiles, g = i / n_tiles;
+    const uint32_t w0 = t * kNtWords, f0 = 4u * w0;
+    const uint32_t TWt = min(kNtWords, W - w0), TF = min(4u * TWt, F - f0);
+    const uint32_t V = kGather ? plan->rows : (uint32_t)n;
+    const uint32_t n_seg = kGather ? plan->n_parent : 1u;
+    uint32_t rb = (uint32_t)(((uint64_t)V * g) / G), re = (uint32_t)(((uint64_t)V * (g + 1)) / G);
+    if (kGather) balanced_range(plan, n_seg, V, g, G, kExSegmentCost, rb, re);
+    uint32_t seg = kGather ? first_segment(plan, n_seg, rb) : 0u;
+    for (uint32_t k = threadIdx.x; k < B * C * 16u; k += kNtThreads) ex[k] = 0ull;
+    NtRange<C, kGather> R;
+    R.cells = ex;
+    R.l = threadIdx.x & 15u;
+    R.r0 = threadIdx.x >> 4;
+    R.j = R.l >> 1;
+    const uint32_t wl = R.l & 1u;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        R.off8[k] = 8u * (8u * (R.j >> 2) + 4u * wl + ((k + R.j) & 3u));
+    R.wl4 = 4u * wl;
+    R.md = sc->mul[kScoreDer];
+    R.mw = sc->mul[kScoreW];
+    const bool rm = kGather && rows_rm != nullptr;
+    R.row_bytes = rm ? row_bytes : 4u * packed_slice_words(TWt);
+    R.rbase = rm ? make_rsrc(rows_rm + w0, n * row_bytes - 4ull * w0) : make_rsrc(trows + n * w0, n * R.row_bytes);
+    R.seq = kGather && sseq != nullptr;
+    R.stat_bytes = 8u * CS;
+    R.sbase = make_rsrc(R.seq ? sseq : sstat, n * R.stat_bytes);
+    R.ibase = make_rsrc(kGather ? (const void*)idx : (const void*)sstat, kGather ? n * 4u : 0u);
+    __syncthreads();
+    uint32_t pos = rb;
+    while (pos < re) {
+        const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
+        const uint32_t end = min(re, seg_end);
+        if (end > pos) {
+            R.pos = pos;
+            R.end = end;
+            R.run();
+            __syncthreads();
+            // flush: a wave takes 8 features x 8 bins of a channel; the ranges start at different
+            // places, so that workgroups flushing together do not queue on the same cells (64-byte
+            // runs of bins, 2 tiles x 128 ranges: 80 us from one start, 45 us spread)
+            const uint32_t nbb = (B + 7) / 8, units = C * nbb;
+            const uint32_t rot = (uint32_t)((uint64_t)g * units / G);
+            const uint32_t lane = threadIdx.x & 63u;
+            long long* dst = raw + (size_t)seg * CS * F * B;
+            for (uint32_t u0 = threadIdx.x >> 6; u0 < units; u0 += kNtThreads / 64) {
+                uint32_t u = u0 + rot;
+                if (u >= units) u -= units;
+                const uint32_t ch = u / nbb, f = lane >> 3, bin = (u - ch * nbb) * 8 + (lane & 7u);
+                if (f >= TF || bin >= B) continue;
+                unsigned long long* cell = ex + (bin * C + ch) * 16u + f;
+                const unsigned long long v = cell[0] + cell[8];
+                cell[0] = 0ull;
+                cell[8] = 0ull;
+                if (v != 0) atomicAdd((unsigned long long*)dst + ((size_t)ch * F + f0 + f) * B + bin, v);
+            }
+            __syncthreads();
+        }
+        pos = end;
+        ++seg;
+    }
+}
+
+// ---------------------------------------------------------------------------------
 // Packed multi-channel fill (K > 1, NP * B <= 512 with NP = ceil(C / 2) planes).  The score
 // channels 2j and 2j + 1 of a row travel in one 64-bit word, p_j = q_{2j+1} * 2^32 + q_{2j}
 // (mod 2^64), each |q| <= 2^kPkkBits - 1 (rounded on the scale of the largest row, clamped), so

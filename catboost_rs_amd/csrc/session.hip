@@ -216,6 +216,11 @@ struct cbh_session {
     bool count = false;
     bool int_w = true;                         // every object weight is an integer in [0, 2^20]
     uint32_t ex_sets = 3;                      // tiled: blocks in flight of the full loop
+    // narrow-tile exact fill (any K): tiles of kNtWords words, nt_ranges row ranges each
+    bool narrow = false;
+    uint32_t nt_tiles = 0, nt_ranges = 1;
+    bool nt_rm = false;                        // gathered levels read row-major words
+    bool der_only = false;                     // PairLogitPairwise: the fill adds the der channel only
     // packed multi-channel fill (K > 1: two score channels per 64-bit word, NP = ceil(C/2) planes)
     bool pkk = false;
     uint32_t pkk_tiles = 0, pkk_ranges = 8;
@@ -727,6 +732,62 @@ int plan_pkk(cbh_session* s, const std::string& v) {
     return CBH_OK;
 }
 
+// The narrow tiles against the 32-feature tiles (K == 1): they save about 0.12 B + 10 us of
+// flushing and latency a level and read rows and statistics four times as often, 0.195 us a level
+// per million (row, feature).  Measured, us a tree of depth 6, narrow against 32-feature: 255
+// bins 1M x 50 415 / 603, 2M x 100 824 / 828, 4M x 50 935 / 953, 1M x 200 820 / 799, 4M x 200 2386 /
+// 1637; 33 bins 1M x 50 345 / 371, 4M x 50 886 / 750.  Below 2^16 rows the 32-feature tiles are
+// not planned.
+bool narrow_pays(uint64_t n, uint32_t F, uint32_t B) {
+    return n < (1ull << 16) || (double)n * F <= 1e6 * (51.0 + 0.615 * B);
+}
+
+// Row ranges G of the narrow-tile exact fill.  A launch takes n / G rows a
+// workgroup at 0.75 C cycles each (6 cycles an LDS atomic of a wave) and flushes G images of
+// F B C cells at 1e11 cells/s (both measured): G balances the two, at most one round of the CUs
+// (half and twice that G measured 2-5% slower at 100k rows, the same at 500k and more).
+uint32_t narrow_ranges(const cbh_session* s, uint32_t cus, uint32_t C) {
+    const uint32_t nt = (s->W + kNtWords - 1) / kNtWords;
+    const double row_us = 0.375 * C * kNtWords / 2400.0, flush_us = (double)s->F * s->B * C * 1e-5;
+    const double best = std::sqrt((double)s->n * row_us / flush_us);
+    return std::max<uint32_t>(1, std::min<uint32_t>(std::max<uint32_t>(1, cus / nt), (uint32_t)best));
+}
+
+template <int C>
+int set_narrow_attr(size_t lds) {
+    for (const void* k : {(const void*)fill_narrow_kernel<C, false>, (const void*)fill_narrow_kernel<C, true>})
+        HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    return CBH_OK;
+}
+
+// Takes the narrow-tile exact fill when its tiles fit and its buffers stay within 32-bit offsets.
+int plan_narrow_fill(cbh_session* s, uint32_t cus, bool& taken) {
+    taken = false;
+    const uint32_t C = s->pairwise ? 1u : s->C;
+    constexpr uint32_t TW = kNtWords;
+    const size_t lds = narrow_lds(s->B, C);
+    if (lds > kNarrowLdsMax || s->n * 8ull * s->C >= (1ull << 31) || s->n * 16ull >= (1ull << 31)) return CBH_OK;
+    CHECK(with_k((int)s->K, [&](auto kc) { return set_narrow_attr<decltype(kc)::value + 1>(narrow_lds(s->B, s->C)); }));
+    if (C == 1) CHECK(set_narrow_attr<1>(lds));
+    s->nt_ranges = narrow_ranges(s, cus, C);
+    s->narrow = true;
+    s->nt_tiles = (s->W + TW - 1) / TW;
+    s->der_only = s->pairwise;
+    s->nt_rm = s->n * 4ull * s->Ws < (1ull << 32);
+    const uint32_t tw_last = s->W - TW * (s->nt_tiles - 1);
+    const uint64_t words = (uint64_t)s->n * (TW * (s->nt_tiles - 1) + packed_slice_words(tw_last));
+    CHECK(dalloc(&s->trows, words));
+    pack_tiles_kernel<<<grid_for(words, 256), 256, 0, s->stream>>>(s->cols, s->n, s->F, s->W, s->trows, words, TW);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s->stream) != hipSuccess)
+        return fail(CBH_ERR_DEVICE, "tile-major packing failed");
+    if (s->K == 1 && !s->pairwise) CHECK(dalloc(&s->sseq, (size_t)s->n * 2u));
+    s->tiled = true;
+    s->use_skip = false;
+    s->n_skip = 0;
+    taken = true;
+    return CBH_OK;
+}
+
 // Fill plan.  The default: K == 1 with integer score weights from 2^22 rows the count-packed
 // fill, else from 2^16 rows (2^20 with pairs) the tiled exact fill (which visits every bin: its
 // lanes add to distinct features, so a dominant bin does not serialize them); K > 1 from 500000
@@ -738,8 +799,19 @@ int plan_fill_mode(cbh_session* s) {
     s->packed = s->tiled = s->pkk = s->count = false;
     const char* e = std::getenv("CBH_FILL");
     const std::string v = e ? e : "";
-    if (s->K > 1) return (v.empty() || v == "packed") ? plan_pkk(s, v) : CBH_OK;
+    int cus_n = 0;
+    HIP_TRY(hipDeviceGetAttribute(&cus_n, hipDeviceAttributeMultiprocessorCount, s->device));
+    bool narrow_taken = false;
+    if (s->K > 1) {
+        if (v.empty() || v == "packed") CHECK(plan_pkk(s, v));
+        if (!s->pkk && v.empty()) CHECK(plan_narrow_fill(s, (uint32_t)cus_n, narrow_taken));
+        return CBH_OK;
+    }
     if (v == "generic") return CBH_OK;
+    if (v.empty() && narrow_pays(s->n, s->F, s->B)) {
+        CHECK(plan_narrow_fill(s, (uint32_t)cus_n, narrow_taken));
+        if (narrow_taken) return CBH_OK;
+    }
     // integer score weights: no per-row sample beyond Bernoulli's keep mask, integer object
     // weights, no pair weights (they arrive after the plan)
     const bool count_ok = !s->ranking && !s->cfg.sample_from_host && s->int_w &&
@@ -1590,7 +1662,7 @@ int ctr_level_weights_dev(cbh_session* s, uint32_t level) {
 uint32_t fill_atomics_per_entry(const cbh_session* s, uint32_t level) {
     if (s->packed || s->count) return 1u;
     if (s->pkk) return (s->C + 1) / 2 - ((level == 0 && s->l0_cached) ? 1u : 0u);
-    return s->C;
+    return s->der_only ? 1u : s->C;
 }
 
 template <int K>
@@ -1678,7 +1750,19 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             fill_packed_kernel<true, true><<<s->pk_gath.blocks, kPackThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
                 s->pk_gath.ranges, 0u, raw, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
-        else if (s->tiled && level == 0)
+        else if (s->narrow) {
+            const unsigned blocks = 8 * ((s->nt_tiles * s->nt_ranges + 7) / 8);
+            const uint32_t rb = 4u * s->Ws;
+            auto launch = [&](auto cc) {
+                constexpr int CF = decltype(cc)::value;   // channels filled
+                const size_t lds = narrow_lds(s->B, CF);
+                (level == 0 ? fill_narrow_kernel<CF, false> : fill_narrow_kernel<CF, true>)<<<blocks, kNtThreads, lds, st>>>(
+                    s->trows, s->W, n, lidx, lplan, s->sstat, s->C, (const double*)s->sseq, s->nt_tiles, s->F, s->B,
+                    s->nt_ranges, raw, level > 0 && s->nt_rm ? s->rows : nullptr, rb, s->scales);
+            };
+            if (s->der_only) launch(std::integral_constant<int, 1>{});
+            else launch(std::integral_constant<int, C>{});
+        } else if (s->tiled && level == 0)
             fill_exact_kernel<false><<<s->pk_dense.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, (const long long*)s->sstat, nullptr, s->pk_dense.tiles16, s->F,
                 s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, raw, nullptr, 0u, s->ex_sets, s->scales);
@@ -1774,7 +1858,7 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         if (!finish) {
             CHECK(s->stage_begin(kStDerive));
             // (PairLogitPairwise fills and reads the der channel only)
-            const bool der_only = s->pairwise && !s->packed && !s->count && !s->tiled && !s->use_skip;
+            const bool der_only = s->pairwise && !s->packed && !s->count && (!s->tiled || s->der_only) && !s->use_skip;
             const uint32_t CU = der_only ? 1u : (uint32_t)C;
             const uint64_t rows = (uint64_t)n_seg * CU * s->F;
             const long long* parent = level > 0 ? par : nullptr;

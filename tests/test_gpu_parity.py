@@ -1143,3 +1143,51 @@ def test_recorded_tree_replays_equal_eager_trees(loss, boot, K):
                 continue
             assert np.array_equal(np.asarray(x).view(np.uint8), np.asarray(y_).view(np.uint8))
             assert np.array_equal(np.asarray(x).view(np.uint8), np.asarray(z).view(np.uint8))
+
+
+@pytest.mark.parametrize("n,F,B,K,loss", [
+    (1, 3, 4, 1, "RMSE"), (1023, 1, 2, 1, "Logloss"), (1025, 9, 256, 1, "RMSE"), (5000, 8, 33, 1, "Logloss"),
+    (16_385, 17, 255, 1, "RMSE"), (40_000, 33, 97, 2, "MultiClass"), (20_001, 5, 200, 5, "MultiClass"),
+    (9_999, 12, 75, 16, "MultiClass"), (30_000, 70, 66, 1, "RMSE")])
+def test_narrow_tile_fill_histograms(n, F, B, K, loss):
+    """The narrow-tile exact fill (8-feature tiles, any K) and the fused finishing / scoring at the
+    edges of their tiles: one row, one feature, last tiles of one word, bin counts at the wave and
+    window edges, one to seventeen channels.  Every level histogram of a first tree equals the sums
+    over the rows of each leaf (der channels and weights, to the fixed-point step of the level's
+    largest cell), and no default session of these sizes leaves the tiled fill."""
+    g = np.random.default_rng(n * 7 + F)
+    bins = g.integers(0, B, (F, n)).astype(np.uint8)
+    bins[0, :] = np.minimum(bins[0, :], B - 1)
+    y = g.integers(0, K, n).astype(np.float64) if K > 1 else (
+        g.standard_normal(n) if loss == "RMSE" else g.integers(0, 2, n).astype(np.float64))
+    w = g.uniform(0.5, 2.0, n)
+    depth = 4
+    be = cb.HipBackend()
+    assert be.begin_device_training(loss, depth, True, 1, "Cosine", bins, w, n, F, B, 0.1, 3.0, approx_dim=K,
+                                    leaf_method="Newton" if K > 1 else "Gradient",
+                                    real_folds=np.full(F, B, np.uint32))
+    try:
+        be.capture_hists()
+        t = be.grow_tree_on_device(target=y, want_leaf_of=True)
+        hists = [be.level_hist(l, F, B) for l in range(depth)]
+        assert be.stats()["fill_mode"] == 2
+    finally:
+        be.end_device_training()
+    if K > 1:
+        der = -np.full((K, n), 1.0 / K)
+        der[y.astype(np.int64), np.arange(n)] += 1.0
+    else:
+        der = (y - (0.0 if loss == "RMSE" else 0.5))[None]
+    chans = np.concatenate([der * w, w[None]])
+    leaf = t["leaf_of"].astype(np.int64)
+    for level in range(depth):
+        lf = leaf & ((1 << level) - 1)
+        exp = np.zeros((1 << level, F, B, K + 1))
+        for f in range(F):
+            for c in range(K + 1):
+                np.add.at(exp[:, f, :, c], (lf, bins[f]), chans[c])
+        # a row's value is rounded to 2^-S of at most 2^-61 of the channel's sum: n rows differ by
+        # less than n 2^-60 of it; the f64 sums of the expectation by n eps of the cell
+        scale = np.abs(chans).sum(1)
+        err = np.abs(hists[level] - exp).max(axis=(0, 1, 2))
+        assert np.all(err <= scale * n * 2.0**-52), (level, err, scale)
