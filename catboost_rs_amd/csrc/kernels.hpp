@@ -239,30 +239,40 @@ __device__ __forceinline__ void sample_row(const SampleParams& smp, const JumpTa
 // fixed-point scales (summed deterministically by scales_kernel).
 // ---------------------------------------------------------------------------------
 constexpr int kPrepBlocks = 2048;
-constexpr int kPartials = 8;   // per block: 4 bounds, sampled rows, 3 spare
+constexpr int kPartials = 8;   // per slot: 4 bounds, sampled rows, 2 maxima, 1 spare
+// The workgroups' partial bounds are added into kBoundSlots rows (a workgroup's row by its
+// index), so that the kernels needing the tree's scales sum 64 rows instead of waiting for a
+// launch that sums 2048; an address takes at most 32 atomics of about 66 ns.
+constexpr uint32_t kBoundSlots = 64;
+
+// Words a tree's first kernel clears for the kernels after it.
+struct ClearList {
+    unsigned long long* p[4];
+    uint32_t n[4];
+};
 
 template <int K>
 static __global__ __launch_bounds__(256) void prepare_kernel(
     uint64_t n, int loss, double* __restrict__ approx, const double* __restrict__ target,
     const double* __restrict__ weight, uint16_t* __restrict__ leaf,
     const double* __restrict__ pending /* [leaves][K] lr-scaled, nullable */,
-    const SampleParams* __restrict__ smpp, JumpTabs jt, const double* __restrict__ host_sample,
+    SampleParams smp, JumpTabs jt, const double* __restrict__ host_sample,
     double* __restrict__ sstat /* [n][K+1] */, int newton,
-    unsigned long long* __restrict__ partials /* [gridDim.x][kPartials] */,
+    unsigned long long* __restrict__ slots /* [kBoundSlots][kPartials], zero before */,
     const double* __restrict__ ext_der /* nullable [2][n]: der1, der2 of a pair loss */,
     const double* __restrict__ score_w /* nullable [n]: histogram weight (pairwise weights) */,
-    uint32_t* __restrict__ gcnt /* the partition's group counts, cleared for the tree */, uint32_t n_gcnt,
-    long long* __restrict__ zraw /* raw segments the last level's finishing left, cleared */, size_t n_zraw) {
+    ClearList clear, long long* __restrict__ zraw /* raw segments the last level's finishing left, cleared */,
+    size_t n_zraw) {
     constexpr int C = K + 1;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_zraw; i += (size_t)gridDim.x * blockDim.x)
         zraw[i] = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_gcnt; i += gridDim.x * blockDim.x) gcnt[i] = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < clear.n[k]; i += gridDim.x * blockDim.x)
+            clear.p[k][i] = 0;
     __shared__ unsigned long long red[4][kPartials];
     unsigned long long acc[kPartials] = {0, 0, 0, 0, 0, 0, 0, 0};
     const double bscale = (double)(1 << kBoundShift);
-    // the tree's sampling parameters live in device memory, so a recorded launch sequence
-    // replays unchanged from tree to tree
-    const SampleParams smp = *smpp;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * blockDim.x) {
         double a[K];
@@ -354,7 +364,11 @@ static __global__ __launch_bounds__(256) void prepare_kernel(
             const unsigned long long u = red[w][threadIdx.x];
             v = mx ? (u > v ? u : v) : v + u;
         }
-        partials[(size_t)blockIdx.x * kPartials + threadIdx.x] = v;
+        unsigned long long* at = slots + (size_t)(blockIdx.x % kBoundSlots) * kPartials + threadIdx.x;
+        if (v != 0) {
+            if (mx) atomicMax(at, v);
+            else atomicAdd(at, v);
+        }
     }
 }
 
@@ -384,62 +398,52 @@ __host__ __device__ inline CountPack count_pack_plan(int e, unsigned long long w
     return cp;
 }
 
-// Sum the per-block partials (integers: exact in any order) and pick S per slot so that
+// Sum the bound slots (integers: exact in any order) and pick S per slot so that
 // 2^S * sum|v| <= 2^61: no partial sum of rounded values can overflow int64.  With
 // pack_bits > 0 the two score slots instead take S = pack_bits - e for the largest row
 // bound M < 2^e, so every rounded row value fits pack_bits bits (|q| <= 2^pack_bits): the
 // rounded packed fill's 32-bit fields.  With count set (the count-packed fill: integer score
 // weights) the weight slot takes S = 0 (the weights themselves) and the der slot the finest
 // scale whose packed cells stay decodable (count_pack_plan).
-static __global__ __launch_bounds__(256) void scales_kernel(const unsigned long long* __restrict__ partials,
-                                                           uint32_t n_blocks, Bounds* __restrict__ b,
-                                                           Scales* __restrict__ sc, int pack_bits, int count) {
-    __shared__ unsigned long long red[4][7];   // per wave (256 threads)
-    unsigned long long acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t i = threadIdx.x; i < n_blocks; i += blockDim.x) {
-        for (int k = 0; k < 5; ++k) acc[k] += partials[(size_t)i * kPartials + k];
-        for (int k = 5; k < 7; ++k) {
-            const unsigned long long u = partials[(size_t)i * kPartials + k];
-            acc[k] = u > acc[k] ? u : acc[k];
-        }
-    }
-    // integer sums and maxima: any order gives the same values
-    const uint32_t wave = threadIdx.x >> 6;
+// One wave; every lane returns with the scales stored to *sc by lane 0 and, with b given, the
+// tree's bounds (its error word cleared for the kernels that may set it).
+__device__ __forceinline__ void wave_scales(const unsigned long long* __restrict__ slots, int pack_bits, int count,
+                                            Scales* sc, Bounds* b) {
+    const uint32_t lane = threadIdx.x & 63u;
+    unsigned long long acc[7];
+    static_assert(kBoundSlots == 64, "a slot a lane");
+#pragma unroll
+    for (int k = 0; k < 7; ++k) acc[k] = slots[(size_t)lane * kPartials + k];
 #pragma unroll
     for (int k = 0; k < 7; ++k) {
-        unsigned long long v = acc[k];
         if (k < 5) {
-            v = wave_sum_u64(v);
+            acc[k] = wave_sum_u64(acc[k]);
         } else {
             for (int o = 32; o > 0; o >>= 1) {
-                const unsigned long long u = __shfl_xor(v, o, 64);
-                v = u > v ? u : v;
+                const unsigned long long u = __shfl_xor(acc[k], o, 64);
+                acc[k] = u > acc[k] ? u : acc[k];
             }
         }
-        if (lane_id() == 0) red[wave][k] = v;
     }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 7; ++k) {
+    if (lane == 0 && b) {
+        for (int k = 0; k < kNumScales; ++k) b->sum_abs[k] = acc[k];
+        b->sampled_rows = acc[4];
+        b->device_err = 0;
+    }
+    if (lane < (uint32_t)kNumScales) {   // scale `lane`
+        const bool is_d = lane == (uint32_t)kScoreDer, is_w = lane == (uint32_t)kScoreW;
+        const bool packed = pack_bits > 0 && (is_d || is_w);
         unsigned long long v = 0;
-        for (uint32_t w = 0; w < blockDim.x / 64; ++w) {
-            const unsigned long long u = red[w][k];
-            v = k < 5 ? v + u : (u > v ? u : v);
-        }
-        acc[k] = v;
-    }
-    for (int k = 0; k < kNumScales; ++k) b->sum_abs[k] = acc[k];
-    b->sampled_rows = acc[4];
-    b->device_err = 0;   // the tree's kernels after this one report a failed bounded wait here
-    for (int k = 0; k < kNumScales; ++k) {
-        const bool packed = pack_bits > 0 && (k == kScoreDer || k == kScoreW);
-        const double bound = (double)acc[packed ? 5 + k : k] / (double)(1 << kBoundShift);
+#pragma unroll
+        for (int k = 0; k < kNumScales; ++k) v = lane == (uint32_t)k ? acc[k] : v;
+        if (packed) v = is_d ? acc[5] : acc[6];
+        const double bound = (double)v / (double)(1 << kBoundShift);
         int e = -20;
         if (bound > 0.0) frexp(bound, &e);   // bound < 2^e
         int s = (packed ? pack_bits : 61) - e;
         if (s > 100) s = 100;
-        if (count && k == kScoreW) s = 0;
-        if (count && k == kScoreDer) {
+        if (count && is_w) s = 0;
+        if (count && is_d) {
             int mx = -20;   // largest row |der * w * s| < 2^mx
             const double mb = (double)acc[5] / (double)(1 << kBoundShift);
             if (mb > 0.0) frexp(mb, &mx);
@@ -448,9 +452,32 @@ static __global__ __launch_bounds__(256) void scales_kernel(const unsigned long 
             sc->pk_k = cp.k;
             sc->pk_swap = cp.swap;
         }
-        sc->shift[k] = s;
-        sc->mul[k] = ldexp(1.0, s);
-        sc->inv[k] = ldexp(1.0, -s);
+        sc->shift[lane] = s;
+        sc->mul[lane] = ldexp(1.0, s);
+        sc->inv[lane] = ldexp(1.0, -s);
+    }
+}
+
+// The scales as a launch of their own: for fills whose row statistics are packed or quantized
+// before the fill.  The tiled fills' level-0 kernel takes them itself (fill_scales).
+static __global__ __launch_bounds__(64) void scales_kernel(const unsigned long long* __restrict__ slots,
+                                                           Bounds* __restrict__ b, Scales* __restrict__ sc,
+                                                           int pack_bits, int count) {
+    wave_scales(slots, pack_bits, count, sc, b);
+}
+
+// The tree's scales inside its first fill: every workgroup sums the slots (wave 0, while the other
+// waves clear the LDS cells), workgroup 0 stores them for the kernels after.  Call it before the
+// barrier that ends the clearing, read *local after it.
+__device__ __forceinline__ void fill_scales(const unsigned long long* __restrict__ slots, Scales* local,
+                                            Scales* __restrict__ sc, Bounds* __restrict__ b) {
+    if (threadIdx.x >= 64) return;
+    wave_scales(slots, 0, 0, local, blockIdx.x == 0 ? b : nullptr);
+    const uint32_t k = threadIdx.x;
+    if (blockIdx.x == 0 && k < (uint32_t)kNumScales) {   // (the lane that stored them to *local)
+        sc->shift[k] = local->shift[k];
+        sc->mul[k] = local->mul[k];
+        sc->inv[k] = local->inv[k];
     }
 }
 
@@ -1474,9 +1501,10 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
     uint32_t n_tiles, uint32_t F, uint32_t B, uint32_t G, uint32_t Gn, long long* __restrict__ hist,
     const uint32_t* __restrict__ rows_rm /* nullable, kGather: row-major words, 2^rm_sh bytes per row */,
     uint32_t rm_sh, uint32_t sets /* blocks in flight of the full loop: 2 to 4 */,
-    const Scales* __restrict__ sc /* the score channels' scales: sfix and sseq hold f64 values */) {
+    Scales* __restrict__ sc /* the score channels' scales: sfix and sseq hold f64 values */,
+    const unsigned long long* __restrict__ slots, Bounds* __restrict__ bounds /* dense: the scales come from the slots */) {
     extern __shared__ unsigned long long ex[];
-    const double md = sc->mul[kScoreDer], mw = sc->mul[kScoreW];
+    __shared__ Scales lsc;
     // blocks: n_tiles tiles of the 8-lane loop in G row ranges each, numbered range-major and
     // dealt to the 8 XCDs in runs (block b to XCD b % 8: XCD x takes pairs [x per, (x + 1) per)),
     // so all tiles of a range share one L2; then, when Gn > 0, the narrow last tile (tile
@@ -1504,6 +1532,7 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
     const uint32_t TF = min(4u * TW, F - f0);
     const bool rm = kGather && rows_rm != nullptr;
     const uint32_t sh = rm ? rm_sh : packed_slice_shift(TW);
+    if (!kGather) fill_scales(slots, &lsc, sc, bounds);
     for (uint32_t i = threadIdx.x; i < kExCells; i += kExThreads) ex[i] = 0ull;
     const uint32_t r0 = threadIdx.x >> 4;   // DPP row of the workgroup
     const uint32_t l = threadIdx.x & 15u;   // lane in the DPP row
@@ -1524,6 +1553,8 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
         wl4 = 4u * w;
     }
     __syncthreads();
+    const double md = kGather ? sc->mul[kScoreDer] : lsc.mul[kScoreDer];
+    const double mw = kGather ? sc->mul[kScoreW] : lsc.mul[kScoreW];
     const uint32_t V = kGather ? plan->rows : (uint32_t)n;
     const uint32_t n_seg = kGather ? plan->n_parent : 1u;
     uint32_t rb = (uint32_t)(((uint64_t)V * g) / GR), re = (uint32_t)(((uint64_t)V * (g + 1)) / GR);
@@ -1683,8 +1714,10 @@ static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
     const double* __restrict__ sseq /* kGather, nullable: [V][CS], the listed rows' channels in idx order */,
     uint32_t n_tiles, uint32_t F, uint32_t B, uint32_t G, long long* __restrict__ raw /* [segment][CS][F][B] */,
     const uint32_t* __restrict__ rows_rm /* nullable, kGather: row-major words, row_bytes a row */,
-    uint32_t row_bytes, const Scales* __restrict__ sc) {
+    uint32_t row_bytes, Scales* __restrict__ sc,
+    const unsigned long long* __restrict__ slots, Bounds* __restrict__ bounds /* dense: the scales come from the slots */) {
     extern __shared__ unsigned long long ex[];
+    __shared__ Scales lsc;
     // block -> (tile, range) as in fill_exact_kernel: all tiles of a range share one XCD's L2
     const uint32_t pairs = n_tiles * G, per = (pairs + 7u) / 8u;
     const uint32_t i = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
@@ -1697,6 +1730,7 @@ static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
     uint32_t rb = (uint32_t)(((uint64_t)V * g) / G), re = (uint32_t)(((uint64_t)V * (g + 1)) / G);
     if (kGather) balanced_range(plan, n_seg, V, g, G, kExSegmentCost, rb, re);
     uint32_t seg = kGather ? first_segment(plan, n_seg, rb) : 0u;
+    if (!kGather) fill_scales(slots, &lsc, sc, bounds);
     for (uint32_t k = threadIdx.x; k < B * C * 16u; k += kNtThreads) ex[k] = 0ull;
     NtRange<C, kGather> R;
     R.cells = ex;
@@ -1708,8 +1742,6 @@ static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
     for (uint32_t k = 0; k < 4; ++k)
         R.off8[k] = 8u * (8u * (R.j >> 2) + 4u * wl + ((k + R.j) & 3u));
     R.wl4 = 4u * wl;
-    R.md = sc->mul[kScoreDer];
-    R.mw = sc->mul[kScoreW];
     const bool rm = kGather && rows_rm != nullptr;
     R.row_bytes = rm ? row_bytes : 4u * packed_slice_words(TWt);
     R.rbase = rm ? make_rsrc(rows_rm + w0, n * row_bytes - 4ull * w0) : make_rsrc(trows + n * w0, n * R.row_bytes);
@@ -1718,6 +1750,8 @@ static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
     R.sbase = make_rsrc(R.seq ? sseq : sstat, n * R.stat_bytes);
     R.ibase = make_rsrc(kGather ? (const void*)idx : (const void*)sstat, kGather ? n * 4u : 0u);
     __syncthreads();
+    R.md = kGather ? sc->mul[kScoreDer] : lsc.mul[kScoreDer];
+    R.mw = kGather ? sc->mul[kScoreW] : lsc.mul[kScoreW];
     uint32_t pos = rb;
     while (pos < re) {
         const uint32_t seg_end = (kGather && seg + 1 < n_seg) ? plan->seg_begin[seg + 1] : V;
@@ -3761,9 +3795,11 @@ static __global__ __launch_bounds__(kLeafThreads) void leaf_reduce_kernel(
     uint64_t n, int loss, int newton, const double* __restrict__ approx,
     const double* __restrict__ target, const double* __restrict__ weight,
     const uint16_t* __restrict__ leaf, const Scales* __restrict__ sc, uint32_t n_leaves,
-    long long* __restrict__ out, const double* __restrict__ ext_der,
-    const double* __restrict__ score_w) {
+    long long* __restrict__ out, const double* __restrict__ ext_der, const double* __restrict__ score_w,
+    unsigned long long* __restrict__ slots /* the bound slots, cleared for the next tree's prepare */) {
     constexpr int CL = leaf_cells<K>();
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < kBoundSlots * kPartials; i += blockDim.x) slots[i] = 0;
     extern __shared__ long long acc[];
     const uint32_t cells = n_leaves * CL;
     for (uint32_t i = threadIdx.x; i < cells; i += blockDim.x) acc[i] = 0;
@@ -3848,29 +3884,49 @@ __device__ inline int cholesky_solve_dev(int k, double* a, const double* b, doub
 
 // Leaf values (leaf.rs:161-335): one thread per leaf.  raw[leaf][d] unscaled, scaled =
 // raw * learning_rate (NormalizeLeafValues, boosting.rs:2879-2881).
+// The tree's results to the host: the device block's words into its pinned mirror (a copy node
+// costs twice the kernel's launch).
+__device__ __forceinline__ void publish(const uint4* __restrict__ src, uint4* __restrict__ host, uint32_t n16) {
+    for (uint32_t i = threadIdx.x; i < n16; i += blockDim.x) host[i] = src[i];
+}
+static __global__ __launch_bounds__(256) void publish_kernel(const uint4* __restrict__ src, uint4* __restrict__ host,
+                                                             uint32_t n16) {
+    publish(src, host, n16);
+}
+
+// K == 1: one workgroup of 256 threads (at most 256 leaves), which then publishes the results
+// (raw is part of the block).
 template <int K>
 static __global__ void leaf_values_kernel(const long long* __restrict__ sums, const Scales* __restrict__ sc,
                                    uint32_t n_leaves, int newton, double l2, double lr,
-                                   double* __restrict__ raw, double* __restrict__ scaled) {
+                                   double* __restrict__ raw, double* __restrict__ scaled,
+                                   const uint4* __restrict__ out /* nullable: nothing to publish */,
+                                   uint4* __restrict__ host, uint32_t n16) {
     constexpr int CL = leaf_cells<K>();
     const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
+    if (K == 1) {
+        static_assert(kMaxLeaves <= 256, "a leaf a thread");
+        if (l < n_leaves) {
+            const double sd = (double)sums[(size_t)l * CL] * sc->inv[kLeafDer];
+            const double sw = (double)sums[(size_t)l * CL + 1] * sc->inv[kLeafW];
+            double v;
+            if (newton) {
+                const double den = -sw + l2;
+                v = den == 0.0 ? 0.0 : sd / den;
+            } else {
+                v = sw > 0.0 ? sd / (sw + l2) : 0.0;
+            }
+            raw[l] = v;
+            scaled[l] = v * lr;
+        }
+        if (!out) return;
+        __syncthreads();
+        publish(out, host, n16);
+        return;
+    }
     if (l >= n_leaves) return;
     const long long* s = sums + (size_t)l * CL;
     const double id = sc->inv[kLeafDer], iw = sc->inv[kLeafW];
-    if (K == 1) {
-        const double sd = (double)s[0] * id;
-        const double sw = (double)s[1] * iw;
-        double v;
-        if (newton) {
-            const double den = -sw + l2;
-            v = den == 0.0 ? 0.0 : sd / den;
-        } else {
-            v = sw > 0.0 ? sd / (sw + l2) : 0.0;
-        }
-        raw[l] = v;
-        scaled[l] = v * lr;
-        return;
-    }
     double h[kMaxK * kMaxK], nd[kMaxK], x[kMaxK];
     int idx = 0;
     for (int i = 0; i < K; ++i)

@@ -157,7 +157,7 @@ struct cbh_session {
     uint32_t fill_ranges = 8;   // row ranges per tile (multiple of 8)
     uint64_t* jump = nullptr;               // [2048 + 2 * n_coarse]: fine a, fine d, coarse a, coarse d
     uint64_t n_coarse = 0;
-    unsigned long long* partials = nullptr; // [kPrepBlocks][kPartials]
+    unsigned long long* slots = nullptr;    // [2][kBoundSlots][kPartials]
 
     // pair losses (PairLogit: pointwise scoring over pairwise weights; PairLogitPairwise:
     // pairwise statistics scoring and Cholesky leaves)
@@ -279,14 +279,11 @@ struct cbh_session {
     uint8_t* pin_ctr_used = nullptr;
     uint64_t* phantom_off_lv = nullptr;         // [depth][cat_n] word offsets at each level
 
-    // per-tree launch sequence recorded once and replayed (index: host sample given or not)
-    hipGraphExec_t tree_graph[2] = {nullptr, nullptr};
+    // per-tree launch sequence after prepare, recorded once and replayed
+    hipGraphExec_t tree_graph = nullptr;
     bool graph_off = false;          // recording failed once: stay eager
-    SampleParams* smp_dev = nullptr; // [2]: the tree's sampling parameters, an inert set
-    // pinned staging of the per-tree results (the recorded copies land here)
-    SampleParams* pin_smp = nullptr;
-    // the per-tree results (splits, plans, bounds, raw leaves) live in one device block and come
-    // back in one copy into its pinned mirror; the pointers below are views into the blocks
+    // the per-tree results (splits, plans, bounds, raw leaves) live in one device block, which the
+    // tree's last kernel writes to its pinned mirror; the pointers below are views into the blocks
     unsigned char* out_dev = nullptr;
     unsigned char* pin_out = nullptr;
     size_t out_bytes = 0;
@@ -310,7 +307,7 @@ struct cbh_session {
         dfree(leaf_sums); dfree(leaf_scaled); dfree(jump);
         dfree(out_dev);
         plans = nullptr; splits = nullptr; bounds = nullptr; leaf_raw = nullptr;
-        dfree(partials);
+        dfree(slots);
         dfree(group_off); dfree(los_off); dfree(los_idx); dfree(comp_off); dfree(comp_win); dfree(comp_los); dfree(comp_w);
         dfree(comp_wq); dfree(ext_der); dfree(score_w); dfree(pair_st);
         dfree(cand_scores); dfree(leaf_w); dfree(skip_bin); dfree(seg_tot); dfree(spack); dfree(sseq); dfree(trows); dfree(pks_a); dfree(pks_b); dfree(row_ent); dfree(fill_ent); dfree(w0_cache);
@@ -321,13 +318,10 @@ struct cbh_session {
         dfree(phantom_off_lv); dfree(hist_cap);
         if (pin_ctr_used) (void)hipHostFree(pin_ctr_used);
         pin_ctr_used = nullptr;
-        for (auto& g : tree_graph)
-            if (g) (void)hipGraphExecDestroy(g);
-        tree_graph[0] = tree_graph[1] = nullptr;
-        dfree(smp_dev);
-        for (void* p : {(void*)pin_smp, (void*)pin_out})
-            if (p) (void)hipHostFree(p);
-        pin_smp = nullptr; pin_out = nullptr;
+        if (tree_graph) (void)hipGraphExecDestroy(tree_graph);
+        tree_graph = nullptr;
+        if (pin_out) (void)hipHostFree(pin_out);
+        pin_out = nullptr;
         pin_splits = nullptr; pin_plans = nullptr; pin_bounds = nullptr; pin_leaves = nullptr;
         for (auto& t : timers) {
             if (t.second.a) (void)hipEventDestroy(t.second.a);
@@ -446,13 +440,13 @@ int session_alloc(cbh_session* s) {
     // workgroups [level][group][leaf]
     CHECK(dalloc(&s->cnt, ((size_t)s->n_part_blocks * 4) << (s->depth - 1)));
     s->n_groups_part = part_groups(s->n_part_blocks);
-    CHECK(dalloc(&s->gcnt, group_count_off(s->n_groups_part, s->depth - 1) + 1));
+    CHECK(dalloc(&s->gcnt, group_count_off(s->n_groups_part, s->depth - 1) + 2));
     {   // one block for the per-tree results, sections 256-byte aligned
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         const size_t o_plans = up(sizeof(SplitRec) * s->depth);
         const size_t o_bounds = o_plans + up(sizeof(LevelPlan) * s->depth);
         const size_t o_leaves = o_bounds + up(sizeof(Bounds));
-        s->out_bytes = o_leaves + sizeof(double) * ((size_t)1 << s->depth) * s->K;
+        s->out_bytes = up(o_leaves + sizeof(double) * ((size_t)1 << s->depth) * s->K);
         CHECK(dalloc(&s->out_dev, s->out_bytes));
         HIP_TRY(hipHostMalloc((void**)&s->pin_out, s->out_bytes, hipHostMallocDefault));
         s->splits = (SplitRec*)s->out_dev;
@@ -523,11 +517,10 @@ int session_alloc(cbh_session* s) {
         }
         if (ws_doubles) CHECK(dalloc(&s->pair_ws, ws_doubles));
     }
-    CHECK(dalloc(&s->smp_dev, 2));
-    HIP_TRY(hipMemset(s->smp_dev, 0, 2 * sizeof(SampleParams)));
-    HIP_TRY(hipHostMalloc((void**)&s->pin_smp, sizeof(SampleParams), hipHostMallocDefault));
     CHECK(dalloc(&s->leaf_scaled, ((size_t)1 << s->depth) * s->K));
-    CHECK(dalloc(&s->partials, (size_t)kPrepBlocks * kPartials));
+    // bound slots of the trees, and a set nobody reads (the update arm of read_approx)
+    CHECK(dalloc(&s->slots, (size_t)2 * kBoundSlots * kPartials));
+    CHECK(launch_zero((long long*)s->slots, (size_t)2 * kBoundSlots * kPartials, s->stream));
     s->n_coarse = (n >> 10) + 2;
     CHECK(dalloc(&s->jump, 2048 + 2 * s->n_coarse));
     {
@@ -957,7 +950,7 @@ int plan_skip_bins(cbh_session* s) {
     }
     if (!any) return CBH_OK;
     CHECK(dalloc(&s->skip_bin, s->F));
-    CHECK(dalloc(&s->seg_tot, (size_t)(kMaxLeaves / 2) * s->C));
+    CHECK(dalloc(&s->seg_tot, ((size_t)s->C << (s->depth - 1)) + s->C));   // [level][segment][C]
     HIP_TRY(hipMemcpy(s->skip_bin, skip.data(), sizeof(uint32_t) * s->F, hipMemcpyHostToDevice));
     return CBH_OK;
 }
@@ -1342,10 +1335,9 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
 // row in pair order (calc_pairwise_weights, boosting.rs:1760-1783), pair weights in fixed
 // point 2^shift with 2^shift * sum|w| <= 2^60 (every statistic and weight-matrix entry is a
 // sum of at most 4 sum|w|), uploaded once.
-void drop_tree_graphs(cbh_session* s) {
-    for (auto& g : s->tree_graph)
-        if (g) (void)hipGraphExecDestroy(g);
-    s->tree_graph[0] = s->tree_graph[1] = nullptr;
+void drop_tree_graph(cbh_session* s) {
+    if (s->tree_graph) (void)hipGraphExecDestroy(s->tree_graph);
+    s->tree_graph = nullptr;
 }
 
 int upload_pairs(cbh_session* s, const cbh_family* fam) {
@@ -1393,7 +1385,7 @@ int upload_pairs(cbh_session* s, const cbh_family* fam) {
     if (neg && s->packed) {   // the packed fill takes non-negative weights only: back to the two-channel fill
         s->packed = false;
         s->pk_signed_w = true;
-        drop_tree_graphs(s);
+        drop_tree_graph(s);
     }
     int e = 0;
     if (sum_abs > 0.0) std::frexp(sum_abs, &e);
@@ -1410,7 +1402,7 @@ int upload_pairs(cbh_session* s, const cbh_family* fam) {
     }
     // a recorded tree holds the pair count, the group count, the weight scale and the pair
     // buffers: a change of any of them records it again
-    if (m != s->n_pairs || G != s->n_groups || std::ldexp(1.0, -shift) != s->pair_inv) drop_tree_graphs(s);
+    if (m != s->n_pairs || G != s->n_groups || std::ldexp(1.0, -shift) != s->pair_inv) drop_tree_graph(s);
     s->pair_inv = std::ldexp(1.0, -shift);
     if (m != s->n_pairs || !s->comp_win) {
         dfree(s->comp_win); dfree(s->comp_los); dfree(s->comp_w); dfree(s->comp_wq); dfree(s->los_idx);
@@ -1665,17 +1657,15 @@ uint32_t fill_atomics_per_entry(const cbh_session* s, uint32_t level) {
     return s->der_only ? 1u : s->C;
 }
 
+// A tree's first kernels: the previous tree's leaves applied, ders, sample, score channels, bounds.
+// Launched with the tree's sampling parameters as arguments, ahead of the recorded rest.
 template <int K>
-int enqueue_tree(cbh_session* s, bool use_host_sample) {
-    constexpr int C = K + 1;
-    const bool apply_prev = s->pending;   // the previous tree's leaves are applied by prepare
+int enqueue_prepare(cbh_session* s, const SampleParams& smp, bool use_host_sample) {
+    const bool apply_prev = s->pending;
     const uint64_t n = s->n;
     hipStream_t st = s->stream;
     const int newton = s->cfg.leaf_method == CBH_LEAF_NEWTON ? 1 : 0;
-    const int sfn = s->cfg.score_function;   // CBH_SCORE_*
     const int loss = s->cfg.loss == CBH_LOSS_RMSE ? 0 : 1;
-
-    // ---- prepare: apply previous tree, ders, sample, score channels, bounds ----
     CHECK(s->stage_begin(kStPrepare));
     if (s->ranking) {   // pair ders need every row's updated approximant: apply, then ders
         if (apply_prev) {
@@ -1687,30 +1677,50 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                                                                   s->ext_der, s->ext_der + n);
         HIP_TRY(hipGetLastError());
     }
-    const unsigned pgrid = grid_for(n, 256, kPrepBlocks);
-    prepare_kernel<K><<<pgrid, 256, 0, st>>>(
+    const uint32_t n_leaves = 1u << s->depth;
+    const ClearList clear{{(unsigned long long*)s->gcnt, (unsigned long long*)s->leaf_sums, (unsigned long long*)s->leaf_w,
+                           (unsigned long long*)s->seg_tot},
+                          {(uint32_t)(group_count_off(s->n_groups_part, s->depth - 1) + 1) / 2,
+                           n_leaves * (uint32_t)leaf_cells<K>(), s->pairwise ? n_leaves * n_leaves : 0u,
+                           s->use_skip ? ((uint32_t)s->C << (s->depth - 1)) + s->C : 0u}};
+    prepare_kernel<K><<<grid_for(n, 256, kPrepBlocks), 256, 0, st>>>(
         n, loss, s->approx, s->target, s->weight, s->leaf,
         apply_prev && !s->ranking ? s->leaf_scaled : nullptr,   // a pair loss applied them above
-        s->smp_dev, s->jt(), use_host_sample ? s->host_sample : nullptr, s->sstat, newton, s->partials,
-        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, s->gcnt,
-        (uint32_t)group_count_off(s->n_groups_part, s->depth - 1),
+        smp, s->jt(), use_host_sample ? s->host_sample : nullptr, s->sstat, newton, s->slots,
+        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, clear,
         s->raw_alt ? s->raw[(s->depth - 1) & 1] : nullptr, s->raw_alt ? s->raw_cells : 0);
     HIP_TRY(hipGetLastError());
-    scales_kernel<<<1, 256, 0, st>>>(s->partials, pgrid, s->bounds, s->scales,
-                                     (s->packed || s->pkk) ? s->pack_bits : 0, s->count ? 1 : 0);
-    HIP_TRY(hipGetLastError());
-    if (s->pkk)
-        quantize_pack_kernel<C><<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack,
-                                                                        (1ll << s->pack_bits) - 1);
-    else if (s->packed)
-        pack_stats_fixed_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack,
-                                                                         (1ll << s->pack_bits) - 1);
-    else if (s->count)
-        pack_stats_count_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack);
-    else if (!s->tiled)   // (the tiled exact fill rounds the f64 channels as it stages them)
-        quantize_stats_kernel<C><<<grid_for(n * C, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales);
-    HIP_TRY(hipGetLastError());
-    CHECK(s->stage_end());
+    return s->stage_end();
+}
+
+template <int K>
+int enqueue_tree(cbh_session* s) {
+    constexpr int C = K + 1;
+    const uint64_t n = s->n;
+    hipStream_t st = s->stream;
+    const int newton = s->cfg.leaf_method == CBH_LEAF_NEWTON ? 1 : 0;
+    const int sfn = s->cfg.score_function;   // CBH_SCORE_*
+    const int loss = s->cfg.loss == CBH_LOSS_RMSE ? 0 : 1;
+
+    // ---- scales and packed statistics (the tiled exact fills take both as they go) ----
+    if (!s->tiled) {
+        CHECK(s->stage_begin(kStPrepare));
+        scales_kernel<<<1, 64, 0, st>>>(s->slots, s->bounds, s->scales, (s->packed || s->pkk) ? s->pack_bits : 0,
+                                        s->count ? 1 : 0);
+        HIP_TRY(hipGetLastError());
+        if (s->pkk)
+            quantize_pack_kernel<C><<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack,
+                                                                            (1ll << s->pack_bits) - 1);
+        else if (s->packed)
+            pack_stats_fixed_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack,
+                                                                             (1ll << s->pack_bits) - 1);
+        else if (s->count)
+            pack_stats_count_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales, s->spack);
+        else
+            quantize_stats_kernel<C><<<grid_for(n * C, 256, 8192), 256, 0, st>>>(s->sstat, n, s->scales);
+        HIP_TRY(hipGetLastError());
+        CHECK(s->stage_end());
+    }
 
     const size_t per_leaf = (size_t)s->F * s->B * C;
     const uint32_t NB = s->n_part_blocks;
@@ -1725,11 +1735,12 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         const uint32_t* lidx = level == 0 ? nullptr : s->idx;
         const LevelPlan* lplan = level == 0 ? nullptr : s->plans + (level - 1);
         const uint32_t n_seg = level == 0 ? 1u : (1u << (level - 1));
+        // the level's segment totals (levels of 1, 1, 2, 4, ... segments one after another)
+        long long* seg_tot = s->seg_tot ? s->seg_tot + (size_t)(level == 0 ? 0u : n_seg) * C : nullptr;
         if (s->use_skip) {   // segment totals for the dominant-bin rebuild (timed with the finishing)
             CHECK(s->stage_begin(kStDerive));
-            CHECK(launch_zero(s->seg_tot, (size_t)n_seg * C, st));
             seg_totals_kernel<<<grid_for(n, 256, 1024), 256, 0, st>>>(lidx, lplan, n,
-                                                                     (const long long*)s->sstat, C, s->seg_tot);
+                                                                     (const long long*)s->sstat, C, seg_tot);
             HIP_TRY(hipGetLastError());
             CHECK(s->stage_end());
         }
@@ -1758,19 +1769,19 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                 const size_t lds = narrow_lds(s->B, CF);
                 (level == 0 ? fill_narrow_kernel<CF, false> : fill_narrow_kernel<CF, true>)<<<blocks, kNtThreads, lds, st>>>(
                     s->trows, s->W, n, lidx, lplan, s->sstat, s->C, (const double*)s->sseq, s->nt_tiles, s->F, s->B,
-                    s->nt_ranges, raw, level > 0 && s->nt_rm ? s->rows : nullptr, rb, s->scales);
+                    s->nt_ranges, raw, level > 0 && s->nt_rm ? s->rows : nullptr, rb, s->scales, s->slots, s->bounds);
             };
             if (s->der_only) launch(std::integral_constant<int, 1>{});
             else launch(std::integral_constant<int, C>{});
         } else if (s->tiled && level == 0)
             fill_exact_kernel<false><<<s->pk_dense.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, nullptr, nullptr, (const long long*)s->sstat, nullptr, s->pk_dense.tiles16, s->F,
-                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, raw, nullptr, 0u, s->ex_sets, s->scales);
+                s->B, s->pk_dense.ranges, s->pk_dense.ranges_n, raw, nullptr, 0u, s->ex_sets, s->scales, s->slots, s->bounds);
         else if (s->tiled)
             fill_exact_kernel<true><<<s->pk_gath.blocks, kExThreads, s->pk_lds, st>>>(
                 s->trows, s->W, n, lidx, lplan, (const long long*)s->sstat, (const long long*)s->sseq,
                 s->pk_gath.tiles16, s->F, s->B, s->pk_gath.ranges, s->pk_gath.ranges_n, raw,
-                s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->ex_sets, s->scales);
+                s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->ex_sets, s->scales, nullptr, nullptr);
         else if (s->pkk) {
             const size_t lds = (size_t)kPkkCells * sizeof(unsigned long long);
             const unsigned grid = s->pkk_ranges * s->pkk_tiles;
@@ -1865,16 +1876,16 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             const uint32_t* sb = s->use_skip ? s->skip_bin : nullptr;
             if (s->B <= 72)   // 8 lanes per row
                 hist_prefix_group_kernel<8, 9><<<(unsigned)((rows + 31) / 32), 256, 0, st>>>(
-                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, seg_tot);
             else if (s->B <= 80)   // 16 lanes per row
                 hist_prefix_group_kernel<16, 5><<<(unsigned)((rows + 15) / 16), 256, 0, st>>>(
-                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, seg_tot);
             else if (s->B <= 96)   // a half-wave per row
                 hist_prefix_group_kernel<32, 3><<<(unsigned)((rows + 7) / 8), 256, 0, st>>>(
-                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, seg_tot);
             else
                 hist_prefix_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(
-                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, s->seg_tot);
+                    raw, cur, lplan, n_seg, C, CU, s->F, s->B, parent, sb, seg_tot);
             HIP_TRY(hipGetLastError());
             CHECK(s->stage_end());
         }
@@ -1898,7 +1909,7 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
             finish_score_kernel<K><<<pl.blocks, kFinishThreads, pl.lds, st>>>(
                 raw, cur, lplan, n_seg, level > 0 ? par : nullptr, n_leaves, s->F, s->B, pl.nf, pl.m, pl.n_parts, pl.nt,
                 keep, s->raw[(level + 1) & 1], level >= 1 ? std::max(1u, n_seg / 2) : 0u,
-                s->use_skip ? s->skip_bin : nullptr, s->seg_tot, s->n_cand, s->one_hot, s->scales, s->l2, sfn,
+                s->use_skip ? s->skip_bin : nullptr, seg_tot, s->n_cand, s->one_hot, s->scales, s->l2, sfn,
                 s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr);
         } else if (chain) {
             // several features per workgroup when B lanes per feature leave most of a wave idle
@@ -1983,16 +1994,16 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
     CHECK(s->stage_begin(kStLeaf));
     const uint32_t n_leaves = 1u << s->depth;
     const uint32_t CL = (uint32_t)leaf_cells<K>();
-    CHECK(launch_zero(s->leaf_sums, (size_t)n_leaves * CL, st));
     const size_t lds = (size_t)n_leaves * CL * sizeof(long long);   // attribute set at open
     // one workgroup of 1024 threads a CU: each flushes its LDS sums once (n_leaves * CL global
     // atomics a workgroup: 16.6k at K = 10 and 256 leaves, so few workgroups)
     leaf_reduce_kernel<K><<<grid_for(n, kLeafThreads, s->cus), kLeafThreads, lds, st>>>(
         n, loss, newton, s->approx, s->target, s->weight, s->leaf, s->scales, n_leaves, s->leaf_sums,
-        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr);
+        s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, s->slots);
     HIP_TRY(hipGetLastError());
+    const uint32_t n16 = (uint32_t)(s->out_bytes / 16);
+    bool published = false;
     if (s->pairwise) {
-        CHECK(launch_zero(s->leaf_w, (size_t)n_leaves * n_leaves, st));
         if (s->n_pairs) {
             const size_t lw_bytes = (size_t)n_leaves * n_leaves * sizeof(long long);
             const bool lw_lds = lw_bytes <= kPairLdsMax;
@@ -2011,8 +2022,10 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
                 s->leaf_scaled, s->pair_leaf_lds ? nullptr : s->pair_ws);
         HIP_TRY(hipGetLastError());
     } else {
-        leaf_values_kernel<K><<<(n_leaves + 63) / 64, 64, 0, st>>>(s->leaf_sums, s->scales, n_leaves, newton,
-                                                                  s->l2, s->lr, s->leaf_raw, s->leaf_scaled);
+        published = K == 1 && !s->ranking;
+        leaf_values_kernel<K><<<K == 1 ? 1 : (n_leaves + 63) / 64, K == 1 ? 256 : 64, 0, st>>>(
+            s->leaf_sums, s->scales, n_leaves, newton, s->l2, s->lr, s->leaf_raw, s->leaf_scaled,
+            published ? (const uint4*)s->out_dev : nullptr, (uint4*)s->pin_out, n16);
         HIP_TRY(hipGetLastError());
         if (s->ranking) {
             pairwise_center_kernel<<<1, 64, 0, st>>>(s->leaf_raw, s->leaf_sums, CL, n_leaves, s->lr,
@@ -2021,23 +2034,25 @@ int enqueue_tree(cbh_session* s, bool use_host_sample) {
         }
     }
     CHECK(s->stage_end());
-
-    HIP_TRY(hipMemcpyAsync(s->pin_out, s->out_dev, s->out_bytes, hipMemcpyDeviceToHost, st));
+    if (!published) {
+        publish_kernel<<<1, 256, 0, st>>>((const uint4*)s->out_dev, (uint4*)s->pin_out, n16);
+        HIP_TRY(hipGetLastError());
+    }
     return CBH_OK;
 }
 
-// Record the steady-state tree (previous leaves pending) once per host-sample mode.  A
-// recording failure leaves the session eager for good; it never fails the tree.
+// Record the steady-state tree (everything after its prepare) once.  A recording failure
+// leaves the session eager for good; it never fails the tree.
 template <int K>
-void record_tree(cbh_session* s, bool use_host_sample) {
-    hipGraphExec_t& ge = s->tree_graph[use_host_sample ? 1 : 0];
+void record_tree(cbh_session* s) {
+    hipGraphExec_t& ge = s->tree_graph;
     hipGraph_t g = nullptr;
     if (hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) {
         (void)hipGetLastError();
         s->graph_off = true;
         return;
     }
-    const int rc = enqueue_tree<K>(s, use_host_sample);
+    const int rc = enqueue_tree<K>(s);
     const hipError_t e = hipStreamEndCapture(s->stream, &g);
     if (rc != CBH_OK || e != hipSuccess || !g || hipGraphInstantiateWithFlags(&ge, g, 0) != hipSuccess) {
         (void)hipGetLastError();
@@ -2052,10 +2067,8 @@ int grow_impl(cbh_session* s, const SampleParams& smp, bool use_host_sample,
               std::vector<SplitRec>& splits_out, std::vector<LevelPlan>& plans_out,
               Bounds& bounds_out, std::vector<double>& leaf_out) {
     hipStream_t st = s->stream;
-    *s->pin_smp = smp;
-    HIP_TRY(hipMemcpyAsync(s->smp_dev, s->pin_smp, sizeof(SampleParams), hipMemcpyHostToDevice, st));
-    // replay the recorded tree when nothing differs from it: previous leaves pending, no
-    // per-stage events
+    // replay the recorded tree when nothing differs from it: a tree has run before, no per-stage
+    // events
     // a CTR session replays once every CTR group is in the model (no per-level host step left)
     const bool ctr_static = !s->ctr_n || s->ctr_dev || (ctr_all_used(s) && s->fweight_one);
     if (s->ctr_dev) {   // the groups earlier trees used (and whether all are), for this tree
@@ -2063,13 +2076,13 @@ int grow_impl(cbh_session* s, const SampleParams& smp, bool use_host_sample,
         s->pin_ctr_used[s->ctr_n] = ctr_all_used(s) ? 1 : 0;   // then no phantom count is needed
         HIP_TRY(hipMemcpyAsync(s->ctr_used_dev, s->pin_ctr_used, s->ctr_n + 1, hipMemcpyHostToDevice, st));
     }
-    const bool replay = s->pending && !s->cfg.profile && !s->graph_off && ctr_static && !s->hist_cap;
-    hipGraphExec_t& ge = s->tree_graph[use_host_sample ? 1 : 0];
-    if (replay && !ge) record_tree<K>(s, use_host_sample);
-    if (replay && ge) {
-        HIP_TRY(hipGraphLaunch(ge, st));
+    const bool replay = (s->pending || s->tree_graph) && !s->cfg.profile && !s->graph_off && ctr_static && !s->hist_cap;
+    if (replay && !s->tree_graph) record_tree<K>(s);
+    CHECK(enqueue_prepare<K>(s, smp, use_host_sample));
+    if (replay && s->tree_graph) {
+        HIP_TRY(hipGraphLaunch(s->tree_graph, st));
     } else {
-        CHECK(enqueue_tree<K>(s, use_host_sample));
+        CHECK(enqueue_tree<K>(s));
     }
     s->pending = true;
     if (s->overlap_fn) s->overlap_fn(s->overlap_arg);   // host work while the tree grows
@@ -2264,11 +2277,7 @@ int cbh_session_grow(cbh_session* s, const double* approx, const double* target,
         // a per-tree sample in a session opened without bootstrap: the weight channel changes from
         // tree to tree, so its level-0 cache and the trees recorded with it are dropped
         s->w_static = s->w0_ready = false;
-        for (hipGraphExec_t& g : s->tree_graph)
-            if (g) {
-                (void)hipGraphExecDestroy(g);
-                g = nullptr;
-            }
+        drop_tree_graph(s);
     }
     hipStream_t st = s->stream;
     if (target) {
@@ -2346,8 +2355,8 @@ int cbh_session_read_approx(cbh_session* s, double* approx_out, uint64_t n_times
             constexpr int K = decltype(kc)::value;
             prepare_kernel<K><<<grid_for(s->n, 256, kPrepBlocks), 256, 0, s->stream>>>(
                 s->n, s->cfg.loss == CBH_LOSS_RMSE ? 0 : 1, s->approx, s->target, s->weight, s->leaf,
-                s->leaf_scaled, s->smp_dev + 1, s->jt(), nullptr, s->sstat, 0, s->partials, nullptr,
-                nullptr, nullptr, 0u, nullptr, 0);
+                s->leaf_scaled, SampleParams{}, s->jt(), nullptr, s->sstat, 0, s->slots + kBoundSlots * kPartials,
+                nullptr, nullptr, ClearList{}, nullptr, 0);
             HIP_TRY(hipGetLastError());
             return CBH_OK;
         });
