@@ -12,7 +12,14 @@
 // values of a leaf contiguously; the output is dim-major [K][n].
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
 #include <string>
+#include <thread>
+#include <vector>
 
 #include "../../include/cbhip.h"
 #include "common.hpp"
@@ -21,49 +28,6 @@ int cbh_internal_fail(int code, const std::string& msg);  // session.hip
 
 namespace {
 
-template <int K>
-__global__ __launch_bounds__(256) void apply_oblivious_kernel(
-    const float* __restrict__ x, uint64_t n, uint32_t F, const uint32_t* __restrict__ split_features,
-    const double* __restrict__ split_borders, const uint32_t* __restrict__ tree_split_offsets,
-    const double* __restrict__ leaf_values, const uint32_t* __restrict__ tree_leaf_offsets,
-    uint32_t n_trees, const double* __restrict__ bias, const uint8_t* __restrict__ nan_as_true,
-    double* __restrict__ out) {
-    for (uint64_t obj = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; obj < n;
-         obj += (uint64_t)gridDim.x * blockDim.x) {
-        double acc[K];
-#pragma unroll
-        for (int d = 0; d < K; ++d) acc[d] = 0.0;
-        for (uint32_t t = 0; t < n_trees; ++t) {
-            uint32_t leaf = 0, bit = 0;
-            for (uint32_t s = tree_split_offsets[t]; s < tree_split_offsets[t + 1]; ++s, ++bit) {
-                const uint32_t f = split_features[s];
-                bool pass = false;
-                if (f < F) {
-                    const float v = x[(size_t)f * n + obj];
-                    pass = isnan(v) ? (nan_as_true != nullptr && nan_as_true[f] != 0)
-                                    : ((double)v > split_borders[s]);
-                }
-                leaf |= (uint32_t)pass << bit;
-            }
-            const uint32_t li = tree_leaf_offsets[t] + leaf;
-            const bool in = li < tree_leaf_offsets[t + 1];
-#pragma unroll
-            for (int d = 0; d < K; ++d) acc[d] += in ? leaf_values[(size_t)li * K + d] : 0.0;
-        }
-#pragma unroll
-        for (int d = 0; d < K; ++d) out[(size_t)d * n + obj] = acc[d] + (bias ? bias[d] : 0.0);
-    }
-}
-
-template <typename T>
-struct Buf {
-    T* p = nullptr;
-    ~Buf() {
-        if (p) (void)hipFree(p);
-    }
-    hipError_t alloc(size_t count) { return hipMalloc((void**)&p, (count ? count : 1) * sizeof(T)); }
-};
-
 #define APPLY_TRY(expr)                                                                          \
     do {                                                                                         \
         hipError_t e_ = (expr);                                                                  \
@@ -71,16 +35,319 @@ struct Buf {
             return cbh_internal_fail(CBH_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(e_)); \
     } while (0)
 
+// The model on the device.  Split arrays hold kSplitPad entries past the last split, so that a
+// tree's splits are read eight at a time whatever its depth.
+constexpr uint32_t kSplitPad = 8;
+struct Model {
+    const uint32_t* sf;    // [splits + pad] feature
+    const double* sb;      // [splits + pad] border
+    const uint32_t* so;    // [trees + 1]
+    const double* lv;
+    const uint32_t* lo;    // [trees + 1]
+    const double* bias;          // nullable
+    const uint8_t* nan_true;     // nullable [F]
+    uint32_t trees, F;
+};
+
+// 64 objects (lanes) a workgroup, its eight waves sharing the trees: what bounds a tree is the chain
+// of its scalar loads (offsets, then features and borders) and its objects' values, about 1 us,
+// so eight chains run side by side, two trees to a wave and step, their splits read eight at a
+// time.  The objects' values are staged in LDS [F][64] (kLds; more features than fit are read
+// through the caches).  The leaf indices of kApplyTrees trees go to LDS, and wave d adds dimension
+// d's leaf values in tree order while the other waves go on to the next trees (two index buffers).
+// One object a thread over all trees, value by value from memory, took 240 us for 1024 x 50 and
+// 30 trees with its allocations, and read 6 GB through the caches for 500k x 100 and 500 trees.
+constexpr uint32_t kApplyObj = 64, kApplyWaves = 8, kApplyTrees = 32;
+constexpr uint32_t kNoLeaf = 0xFFFFFFFFu;
+template <int K, bool kLds>
+__global__ __launch_bounds__(kApplyObj * kApplyWaves) void apply_oblivious_kernel(
+    const float* __restrict__ x /* value of feature f, object i at x[f * ld + i] */, uint64_t ld, uint64_t n, Model M,
+    double* __restrict__ out /* [K][ldo] */, uint64_t ldo) {
+    __shared__ uint32_t leaves[2][kApplyTrees][kApplyObj];
+    extern __shared__ float xs[];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kApplyObj), lane = threadIdx.x % kApplyObj;
+    const uint64_t obj = (uint64_t)blockIdx.x * kApplyObj + lane;
+    const uint64_t oc = obj < n ? obj : n - 1;
+    if (kLds) {
+#pragma unroll 4
+        for (uint32_t f = wave; f < M.F; f += kApplyWaves) xs[f * kApplyObj + lane] = x[(size_t)f * ld + oc];
+        __syncthreads();
+    }
+    auto bits8 = [&](uint32_t s) -> uint32_t {   // the tests of splits s .. s + 7
+        uint32_t f[8];
+        double b[8];
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            f[k] = M.sf[s + k];
+            b[k] = M.sb[s + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t fc = f[k] < M.F ? f[k] : 0u;
+            v[k] = M.F == 0 ? 0.0f : kLds ? xs[fc * kApplyObj + lane] : x[(size_t)fc * ld + oc];
+        }
+        uint32_t bits = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool have = f[k] < M.F;   // (a split on an absent feature fails)
+            bool pass = (double)v[k] > b[k];   // false for NaN
+            if (M.nan_true) pass |= v[k] != v[k] && M.nan_true[have ? f[k] : 0u] != 0;
+            bits |= (uint32_t)(pass && have) << k;
+        }
+        return bits;
+    };
+    constexpr int KD = (K + (int)kApplyWaves - 1) / (int)kApplyWaves;   // dimensions of a wave
+    double acc[KD];
+#pragma unroll
+    for (int j = 0; j < KD; ++j) acc[j] = 0.0;
+    uint32_t buf = 0;
+    for (uint32_t t0 = 0; t0 < M.trees; t0 += kApplyTrees, buf ^= 1u) {
+        const uint32_t nt = min(kApplyTrees, M.trees - t0);
+        for (uint32_t i = wave; i < nt; i += 2 * kApplyWaves) {   // wave-uniform
+            const uint32_t i1 = min(i + kApplyWaves, nt - 1);     // (the second tree, or a repeat)
+            const uint32_t t[2] = {t0 + i, t0 + i1};
+            uint32_t s0[2], s1[2], l0[2], l1[2], leaf[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                s0[u] = M.so[t[u]];
+                s1[u] = M.so[t[u] + 1];
+                l0[u] = M.lo[t[u]];
+                l1[u] = M.lo[t[u] + 1];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {   // bits past the tree's last split: another tree's, or padding
+                const uint32_t m = s1[u] - s0[u];
+                leaf[u] = bits8(s0[u]);
+                if (m < 8) leaf[u] &= (1u << m) - 1u;
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                for (uint32_t s = s0[u] + 8; s < s1[u]; s += 8) {
+                    const uint32_t m = s1[u] - s;
+                    const uint32_t bits = bits8(s);
+                    leaf[u] |= (m < 8 ? bits & ((1u << m) - 1u) : bits) << (s - s0[u]);
+                }
+                const uint32_t li = l0[u] + leaf[u];
+                leaves[buf][t[u] - t0][lane] = li < l1[u] ? li : kNoLeaf;
+            }
+        }
+        // one barrier a chunk: the other buffer's readers pass it only after reading it
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KD; ++j) {
+            const uint32_t d = wave + (uint32_t)j * kApplyWaves;
+            if (d >= (uint32_t)K) break;
+#pragma unroll 1
+            for (uint32_t i = 0; i < nt; i += 8) {
+                double v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t li = leaves[buf][min(i + (uint32_t)u, nt - 1)][lane];
+                    v[u] = li != kNoLeaf ? M.lv[(size_t)li * K + d] : 0.0;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i + (uint32_t)u < nt) acc[j] += v[u];
+            }
+        }
+    }
+    if (obj >= n) return;
+#pragma unroll
+    for (int j = 0; j < KD; ++j) {
+        const uint32_t d = wave + (uint32_t)j * kApplyWaves;
+        if (d < (uint32_t)K) out[(size_t)d * ldo + obj] = acc[j] + (M.bias ? M.bias[d] : 0.0);
+    }
+}
+
+constexpr size_t kApplyLdsMax = 128 * 1024;
+
 template <int K>
-int launch(const float* x, uint64_t n, uint32_t F, const uint32_t* sf, const double* sb, const uint32_t* so,
-           const double* lv, const uint32_t* lo, uint32_t T, const double* bias, const uint8_t* nan_true,
-           double* out) {
-    uint64_t g = (n + 255) / 256;
-    if (g > 65535ull * 16) g = 65535ull * 16;
-    if (g < 1) g = 1;
-    apply_oblivious_kernel<K><<<(unsigned)g, 256>>>(x, n, F, sf, sb, so, lv, lo, T, bias, nan_true, out);
+int launch(const float* x, uint64_t ld, uint64_t n, const Model& M, double* out, uint64_t ldo, hipStream_t st) {
+    const size_t lds = (size_t)M.F * kApplyObj * sizeof(float);
+    const unsigned grid = (unsigned)((n + kApplyObj - 1) / kApplyObj);
+    if (lds <= kApplyLdsMax) {
+        if (lds > 32 * 1024)
+            APPLY_TRY(hipFuncSetAttribute((const void*)apply_oblivious_kernel<K, true>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kApplyLdsMax));
+        apply_oblivious_kernel<K, true><<<grid, kApplyObj * kApplyWaves, lds, st>>>(x, ld, n, M, out, ldo);
+    } else {
+        apply_oblivious_kernel<K, false><<<grid, kApplyObj * kApplyWaves, 0, st>>>(x, ld, n, M, out, ldo);
+    }
     APPLY_TRY(hipGetLastError());
     return CBH_OK;
+}
+
+int launch_k(uint32_t K, const float* x, uint64_t ld, uint64_t n, const Model& M, double* out, uint64_t ldo,
+             hipStream_t st) {
+    switch (K) {
+#define CASE(k) case k: return launch<k>(x, ld, n, M, out, ldo, st);
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(10) CASE(12) CASE(16)
+#undef CASE
+        default: return cbh_internal_fail(CBH_ERR_UNSUPPORTED, "approx_dim " + std::to_string(K) + " has no apply variant");
+    }
+}
+bool has_variant(uint32_t K) { return (K >= 1 && K <= 8) || K == 10 || K == 12 || K == 16; }
+
+// A call's buffers: a device block, a pinned block and a stream.  Allocating and freeing them per
+// call (eight of each, each free a device synchronization) was most of a small call's time, so
+// up to kKeep idle workspaces are kept, each a call's own while it runs (any number of threads);
+// one that has grown past kKeepBytes is freed with its call, as are those above kKeep.
+struct Workspace {
+    int device = -1;
+    hipStream_t stream = nullptr, copy = nullptr;   // copy: a large table's uploads, beside the kernels
+    unsigned char* dev = nullptr;
+    unsigned char* pin = nullptr;
+    size_t dev_cap = 0, pin_cap = 0;
+    hipEvent_t ev[6] = {};   // of the three chunk buffers: uploaded, then read by the kernel
+
+    void release() {
+        if (dev) (void)hipFree(dev);
+        if (pin) (void)hipHostFree(pin);
+        for (auto& e : ev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (stream) (void)hipStreamDestroy(stream);
+        if (copy) (void)hipStreamDestroy(copy);
+        copy = nullptr;
+        dev = pin = nullptr;
+        dev_cap = pin_cap = 0;
+        stream = nullptr;
+    }
+    int grow(size_t need_dev, size_t need_pin) {
+        if (!stream) APPLY_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        if (need_dev > dev_cap) {
+            if (dev) (void)hipFree(dev);
+            dev = nullptr;
+            dev_cap = 0;
+            need_dev = std::max<size_t>(need_dev, 1 << 20);
+            APPLY_TRY(hipMalloc((void**)&dev, need_dev));
+            dev_cap = need_dev;
+        }
+        if (need_pin > pin_cap) {
+            if (pin) (void)hipHostFree(pin);
+            pin = nullptr;
+            pin_cap = 0;
+            need_pin = std::max<size_t>(need_pin, 1 << 20);
+            APPLY_TRY(hipHostMalloc((void**)&pin, need_pin, hipHostMallocDefault));
+            pin_cap = need_pin;
+        }
+        return CBH_OK;
+    }
+};
+constexpr size_t kKeep = 2, kKeepBytes = (size_t)64 << 20;
+std::mutex g_ws_mu;
+std::vector<Workspace>& idle_workspaces() {
+    static std::vector<Workspace>* v = [] {   // (never destroyed: no frees after the runtime has gone)
+        auto* p = new std::vector<Workspace>();
+        p->reserve(kKeep);
+        return p;
+    }();
+    return *v;
+}
+struct Lease {
+    Workspace ws;
+    bool ok = false;   // the call went through: nothing is running on the stream
+    explicit Lease(int device) {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        auto& idle = idle_workspaces();
+        for (size_t k = 0; k < idle.size(); ++k)
+            if (idle[k].device == device) {
+                ws = idle[k];
+                idle.erase(idle.begin() + (long)k);
+                return;
+            }
+        ws.device = device;
+    }
+    ~Lease() {
+        if (!ok && ws.copy) (void)hipStreamSynchronize(ws.copy);
+        if (!ok && ws.stream) (void)hipStreamSynchronize(ws.stream);
+        if (ok && ws.dev_cap <= kKeepBytes && ws.pin_cap <= kKeepBytes) {
+            std::lock_guard<std::mutex> lock(g_ws_mu);
+            if (idle_workspaces().size() < kKeep) {
+                idle_workspaces().push_back(ws);
+                return;
+            }
+        }
+        ws.release();
+    }
+};
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// Host threads that copy a large table into pinned memory (the CPU share of a shared host).
+unsigned copy_threads() {
+    unsigned t = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
+    if (const char* e = std::getenv("OMP_NUM_THREADS")) {
+        const long v = std::strtol(e, nullptr, 10);
+        if (v >= 1 && (unsigned long)v < t) t = (unsigned)v;
+    }
+    return t;
+}
+
+constexpr size_t kChunkBytes = (size_t)6 << 20;   // of a table in pinned chunks, three in flight
+
+// A large table in chunks of objects: the threads copy a chunk's runs of every feature into one of
+// three pinned buffers, which goes to its device buffer and through the kernel while the next one
+// fills (the runtime's own path for pageable memory copies with one thread: 200 MB in 7 ms).
+int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, uint32_t K, const Model& M, size_t dev_x,
+                 size_t pin_x, uint64_t chunk, double* d_out) {
+    const uint64_t n_chunks = (n + chunk - 1) / chunk;
+    const size_t cbytes = align256(sizeof(float) * chunk * F);
+    for (auto& e : w.ev)
+        if (!e) APPLY_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (!w.copy) APPLY_TRY(hipStreamCreateWithFlags(&w.copy, hipStreamNonBlocking));
+    const unsigned T = copy_threads();
+    // chunk c may be filled once `open` is past it; `done[c]` counts the threads that have copied
+    // their features of it
+    std::atomic<uint64_t> open{std::min<uint64_t>(2, n_chunks)};
+    std::vector<std::atomic<uint32_t>> done(n_chunks);
+    for (auto& d : done) d.store(0, std::memory_order_relaxed);
+    std::atomic<bool> stop{false};
+    auto copy = [&](unsigned t) {
+        for (uint64_t c = 0; c < n_chunks; ++c) {
+            while (open.load(std::memory_order_acquire) <= c) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                std::this_thread::yield();
+            }
+            const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
+            float* dst = (float*)(w.pin + pin_x + (c % 3) * cbytes);
+            for (uint32_t f = t; f < F; f += T)
+                std::memcpy(dst + (size_t)f * m, features + (size_t)f * n + o0, sizeof(float) * m);
+            done[c].fetch_add(1, std::memory_order_release);
+        }
+    };
+    std::vector<std::thread> pool;
+    int rc = CBH_OK;
+    try {
+        for (unsigned t = 0; t < T; ++t) pool.emplace_back(copy, t);
+    } catch (...) {
+        rc = cbh_internal_fail(CBH_ERR_DEVICE, "no host thread for the table's copy");
+    }
+    for (uint64_t c = 0; c < n_chunks && rc == CBH_OK; ++c) {
+        while (done[c].load(std::memory_order_acquire) < T) std::this_thread::yield();
+        const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
+        const size_t b = (c % 3) * cbytes;
+        float* dx = (float*)(w.dev + dev_x + b);
+        hipEvent_t up = w.ev[c % 3], read = w.ev[3 + c % 3];
+        if ((c >= 3 && hipStreamWaitEvent(w.copy, read, 0) != hipSuccess) ||   // chunk c - 3's kernel
+            hipMemcpyAsync(dx, w.pin + pin_x + b, sizeof(float) * m * F, hipMemcpyHostToDevice, w.copy) != hipSuccess ||
+            hipEventRecord(up, w.copy) != hipSuccess || hipStreamWaitEvent(w.stream, up, 0) != hipSuccess)
+            rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+        if (rc == CBH_OK) rc = launch_k(K, dx, m, m, M, d_out + o0, n, w.stream);
+        if (rc == CBH_OK && hipEventRecord(read, w.stream) != hipSuccess)
+            rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+        if (rc == CBH_OK && c + 2 < n_chunks) {   // chunk c + 2 takes the buffer of chunk c - 1
+            if (c >= 1 && hipEventSynchronize(w.ev[(c - 1) % 3]) != hipSuccess)
+                rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+            else
+                open.store(c + 3, std::memory_order_release);
+        }
+    }
+    stop.store(true);
+    for (auto& th : pool) th.join();
+    return rc;
 }
 
 }  // namespace
@@ -110,42 +377,57 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
         return cbh_internal_fail(CBH_ERR_INVALID_ARG, "model arrays are null");
     const uint32_t K = approx_dim;
     if (n_objects == 0) return CBH_OK;
-    Buf<float> x;
-    Buf<uint32_t> sf, so, lo;
-    Buf<double> sb, lv, db, dout;
-    Buf<uint8_t> na;
-    APPLY_TRY(x.alloc(n_objects * n_features));
-    APPLY_TRY(sf.alloc(n_splits));
-    APPLY_TRY(sb.alloc(n_splits));
-    APPLY_TRY(so.alloc((size_t)n_trees + 1));
-    APPLY_TRY(lv.alloc((size_t)n_leaves * K));
-    APPLY_TRY(lo.alloc((size_t)n_trees + 1));
-    APPLY_TRY(dout.alloc(n_objects * K));
-    if (n_features)
-        APPLY_TRY(hipMemcpy(x.p, features_fm, sizeof(float) * n_objects * n_features, hipMemcpyHostToDevice));
-    if (n_splits) {
-        APPLY_TRY(hipMemcpy(sf.p, split_features, sizeof(uint32_t) * n_splits, hipMemcpyHostToDevice));
-        APPLY_TRY(hipMemcpy(sb.p, split_borders, sizeof(double) * n_splits, hipMemcpyHostToDevice));
-    }
-    APPLY_TRY(hipMemcpy(so.p, tree_split_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1), hipMemcpyHostToDevice));
-    APPLY_TRY(hipMemcpy(lo.p, tree_leaf_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1), hipMemcpyHostToDevice));
-    if (n_leaves) APPLY_TRY(hipMemcpy(lv.p, leaf_values, sizeof(double) * n_leaves * K, hipMemcpyHostToDevice));
-    if (bias) {
-        APPLY_TRY(db.alloc(K));
-        APPLY_TRY(hipMemcpy(db.p, bias, sizeof(double) * K, hipMemcpyHostToDevice));
-    }
-    if (nan_as_true && n_features) {
-        APPLY_TRY(na.alloc(n_features));
-        APPLY_TRY(hipMemcpy(na.p, nan_as_true, n_features, hipMemcpyHostToDevice));
-    }
-    int rc;
-    switch (K) {
-#define CASE(k) case k: rc = launch<k>(x.p, n_objects, n_features, sf.p, sb.p, so.p, lv.p, lo.p, n_trees, bias ? db.p : nullptr, na.p, dout.p); break;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(10) CASE(12) CASE(16)
-#undef CASE
-        default: return cbh_internal_fail(CBH_ERR_UNSUPPORTED, "approx_dim " + std::to_string(K) + " has no apply variant");
-    }
+    if (!has_variant(K))
+        return cbh_internal_fail(CBH_ERR_UNSUPPORTED, "approx_dim " + std::to_string(K) + " has no apply variant");
+    const uint64_t n = n_objects;
+    const uint32_t F = n_features;
+    // one block: the model (and a small table) as uploaded in one copy, the table's chunks, the output
+    const size_t o_sb = 0, o_lv = o_sb + align256(sizeof(double) * ((size_t)n_splits + kSplitPad));
+    const size_t o_bias = o_lv + align256(sizeof(double) * n_leaves * K), o_sf = o_bias + align256(sizeof(double) * K);
+    const size_t o_so = o_sf + align256(sizeof(uint32_t) * ((size_t)n_splits + kSplitPad));
+    const size_t o_lo = o_so + align256(sizeof(uint32_t) * ((size_t)n_trees + 1));
+    const size_t o_na = o_lo + align256(sizeof(uint32_t) * ((size_t)n_trees + 1)), o_x = o_na + align256(F);
+    const size_t x_bytes = sizeof(float) * n * F, out_bytes = sizeof(double) * n * K;
+    const bool chunked = x_bytes > 2 * kChunkBytes;
+    const uint64_t chunk = chunked ? std::max<uint64_t>(64, kChunkBytes / (sizeof(float) * F) / 64 * 64) : n;
+    const size_t x_dev = chunked ? 3 * align256(sizeof(float) * chunk * F) : align256(x_bytes);
+    const size_t o_out = o_x + x_dev;
+    int dev = 0;
+    APPLY_TRY(hipGetDevice(&dev));
+    Lease L(dev);
+    Workspace& w = L.ws;
+    const bool pin_out = out_bytes <= ((size_t)4 << 20);   // the kernel's results through pinned memory
+    int rc = w.grow(o_out + out_bytes, o_x + x_dev + (pin_out ? out_bytes : 0));
     if (rc != CBH_OK) return rc;
-    APPLY_TRY(hipMemcpy(out, dout.p, sizeof(double) * n_objects * K, hipMemcpyDeviceToHost));
+    unsigned char* h = w.pin;
+    if (n_splits) std::memcpy(h + o_sb, split_borders, sizeof(double) * n_splits);
+    std::memset(h + o_sb + sizeof(double) * n_splits, 0, sizeof(double) * kSplitPad);
+    if (n_leaves) std::memcpy(h + o_lv, leaf_values, sizeof(double) * n_leaves * K);
+    if (bias) std::memcpy(h + o_bias, bias, sizeof(double) * K);
+    if (n_splits) std::memcpy(h + o_sf, split_features, sizeof(uint32_t) * n_splits);
+    std::memset(h + o_sf + sizeof(uint32_t) * n_splits, 0, sizeof(uint32_t) * kSplitPad);
+    std::memcpy(h + o_so, tree_split_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1));
+    std::memcpy(h + o_lo, tree_leaf_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1));
+    if (nan_as_true && F) std::memcpy(h + o_na, nan_as_true, F);
+    if (!chunked && x_bytes) std::memcpy(h + o_x, features_fm, x_bytes);
+    const Model M{(const uint32_t*)(w.dev + o_sf), (const double*)(w.dev + o_sb), (const uint32_t*)(w.dev + o_so),
+                  (const double*)(w.dev + o_lv), (const uint32_t*)(w.dev + o_lo),
+                  bias ? (const double*)(w.dev + o_bias) : nullptr,
+                  nan_as_true && F ? (const uint8_t*)(w.dev + o_na) : nullptr, n_trees, F};
+    double* d_out = (double*)(w.dev + o_out);
+    APPLY_TRY(hipMemcpyAsync(w.dev, h, chunked ? o_x : o_x + x_bytes, hipMemcpyHostToDevice, w.stream));
+    rc = chunked ? apply_chunks(w, features_fm, n, F, K, M, o_x, o_x, chunk, d_out)
+                 : launch_k(K, (const float*)(w.dev + o_x), n, n, M, d_out, n, w.stream);
+    if (rc != CBH_OK) return rc;
+    if (pin_out) {
+        unsigned char* ho = h + o_x + x_dev;
+        APPLY_TRY(hipMemcpyAsync(ho, d_out, out_bytes, hipMemcpyDeviceToHost, w.stream));
+        APPLY_TRY(hipStreamSynchronize(w.stream));
+        std::memcpy(out, ho, out_bytes);
+    } else {
+        APPLY_TRY(hipMemcpyAsync(out, d_out, out_bytes, hipMemcpyDeviceToHost, w.stream));
+        APPLY_TRY(hipStreamSynchronize(w.stream));
+    }
+    L.ok = true;
     return CBH_OK;
 }

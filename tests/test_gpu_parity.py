@@ -1191,3 +1191,38 @@ def test_narrow_tile_fill_histograms(n, F, B, K, loss):
         scale = np.abs(chans).sum(1)
         err = np.abs(hists[level] - exp).max(axis=(0, 1, 2))
         assert np.all(err <= scale * n * 2.0**-52), (level, err, scale)
+
+
+@pytest.mark.parametrize("n,F,T,D,K", [(1, 1, 1, 1, 1), (65, 7, 5, 3, 3), (1024, 50, 30, 6, 1), (70_001, 50, 9, 9, 1),
+                                       (1_201, 3_000, 6, 4, 2), (200_000, 16, 11, 17, 1)])
+def test_apply_oblivious_paths_match_reference(n, F, T, D, K):
+    """Every route of a prediction call: a small table in one upload, a large one in pinned chunks
+    (over 12 MB; a last chunk that is no multiple of 64), features staged in LDS or, above 512 of
+    them, read through the caches, trees of one to three groups of eight splits, absent features
+    and NaN.  The sums are in tree order, so the result is bit-equal to the same order in f64.
+    Two host threads predicting at once get the same."""
+    g = np.random.default_rng(n + F)
+    x = g.standard_normal((F, n), dtype=np.float32)
+    x[g.random((F, n)) < 0.01] = np.nan
+    sf = g.integers(0, F + 1, T * D).astype(np.uint32)   # feature F is absent
+    sb = g.standard_normal(T * D).astype(np.float32).astype(np.float64)
+    so = np.arange(0, T * D + 1, D, dtype=np.uint32)
+    lv = g.standard_normal((T << D) * K)
+    lo = np.arange(0, (T << D) + 1, 1 << D, dtype=np.uint32)
+    na = (g.random(F) < 0.5).astype(np.uint8)
+    bias = g.standard_normal(K)
+    exp = np.zeros((K, n))
+    for t in range(T):
+        leaf = np.zeros(n, np.int64)
+        for i in range(D):
+            f = sf[t * D + i]
+            if f < F:
+                v = x[f].astype(np.float64)
+                leaf |= np.where(np.isnan(v), bool(na[f]), v > sb[t * D + i]).astype(np.int64) << i
+        exp += lv.reshape(-1, K)[(t << D) + leaf].T
+    exp += bias[:, None]
+    from concurrent.futures import ThreadPoolExecutor
+    with ThreadPoolExecutor(2) as ex:
+        for got in ex.map(lambda _: cb.apply_oblivious(x, sf, sb, so, lv, lo, approx_dim=K, bias=bias, nan_as_true=na),
+                          range(4)):
+            assert np.array_equal(got, exp)
