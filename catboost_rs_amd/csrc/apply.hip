@@ -18,6 +18,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -161,11 +162,18 @@ __global__ __launch_bounds__(kApplyObj * kApplyWaves) void apply_oblivious_kerne
 }
 
 constexpr size_t kApplyLdsMax = 128 * 1024;
+constexpr uint64_t kMaxBlocks = (uint64_t)1 << 22;
 
 template <int K>
 int launch(const float* x, uint64_t ld, uint64_t n, const Model& M, double* out, uint64_t ldo, hipStream_t st) {
     const size_t lds = (size_t)M.F * kApplyObj * sizeof(float);
-    const unsigned grid = (unsigned)((n + kApplyObj - 1) / kApplyObj);
+    const uint64_t blocks = (n + kApplyObj - 1) / kApplyObj;
+    if (blocks > kMaxBlocks) {   // (a launch holds fewer than 2^32 threads)
+        const uint64_t n0 = kMaxBlocks * kApplyObj;
+        const int rc = launch<K>(x, ld, n0, M, out, ldo, st);
+        return rc != CBH_OK ? rc : launch<K>(x + n0, ld, n - n0, M, out + n0, ldo, st);
+    }
+    const unsigned grid = (unsigned)blocks;
     if (lds <= kApplyLdsMax) {
         if (lds > 32 * 1024)
             APPLY_TRY(hipFuncSetAttribute((const void*)apply_oblivious_kernel<K, true>,
@@ -274,6 +282,11 @@ struct Lease {
     }
 };
 
+// Leaf values that go up through the pinned block: what fits its smallest size beside the other
+// arrays.  More go up from the caller's memory: pinning 3 MB for them took the first call on 100 trees
+// of depth 12 from 1.2 to 2.2 ms, which a call's 0.1 ms of copying does not pay back.
+constexpr size_t kPinModel = (size_t)512 << 10;
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Host threads that copy a large table into pinned memory (the CPU share of a shared host).
@@ -298,34 +311,44 @@ int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, ui
     for (auto& e : w.ev)
         if (!e) APPLY_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (!w.copy) APPLY_TRY(hipStreamCreateWithFlags(&w.copy, hipStreamNonBlocking));
-    const unsigned T = copy_threads();
+    const unsigned want = copy_threads();
     // chunk c may be filled once `open` is past it; `done[c]` counts the threads that have copied
-    // their features of it
+    // their features of it.  `threads` is how many there are, 0 until all have been started; the
+    // calling thread copies when none could be.
+    std::atomic<unsigned> threads{0};
     std::atomic<uint64_t> open{std::min<uint64_t>(2, n_chunks)};
     std::vector<std::atomic<uint32_t>> done(n_chunks);
     for (auto& d : done) d.store(0, std::memory_order_relaxed);
     std::atomic<bool> stop{false};
+    auto copy_chunk = [&](uint64_t c, uint32_t first, uint32_t step) {
+        const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
+        float* dst = (float*)(w.pin + pin_x + (c % 3) * cbytes);
+        for (uint32_t f = first; f < F; f += step)
+            std::memcpy(dst + (size_t)f * m, features + (size_t)f * n + o0, sizeof(float) * m);
+    };
     auto copy = [&](unsigned t) {
+        unsigned T;
+        while ((T = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
         for (uint64_t c = 0; c < n_chunks; ++c) {
             while (open.load(std::memory_order_acquire) <= c) {
                 if (stop.load(std::memory_order_relaxed)) return;
                 std::this_thread::yield();
             }
-            const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
-            float* dst = (float*)(w.pin + pin_x + (c % 3) * cbytes);
-            for (uint32_t f = t; f < F; f += T)
-                std::memcpy(dst + (size_t)f * m, features + (size_t)f * n + o0, sizeof(float) * m);
+            copy_chunk(c, t, T);
             done[c].fetch_add(1, std::memory_order_release);
         }
     };
     std::vector<std::thread> pool;
     int rc = CBH_OK;
+    pool.reserve(want);
     try {
-        for (unsigned t = 0; t < T; ++t) pool.emplace_back(copy, t);
-    } catch (...) {
-        rc = cbh_internal_fail(CBH_ERR_DEVICE, "no host thread for the table's copy");
+        for (unsigned t = 0; t < want; ++t) pool.emplace_back(copy, t);
+    } catch (const std::system_error&) {   // no more threads: those there are take all of it
     }
+    const unsigned T = (unsigned)pool.size();
+    threads.store(T, std::memory_order_release);
     for (uint64_t c = 0; c < n_chunks && rc == CBH_OK; ++c) {
+        if (T == 0) copy_chunk(c, 0, 1);   // (its buffer is free: waited for below, two chunks ago)
         while (done[c].load(std::memory_order_acquire) < T) std::this_thread::yield();
         const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
         const size_t b = (c % 3) * cbytes;
@@ -382,14 +405,19 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
     const uint64_t n = n_objects;
     const uint32_t F = n_features;
     // one block: the model (and a small table) as uploaded in one copy, the table's chunks, the output
-    const size_t o_sb = 0, o_lv = o_sb + align256(sizeof(double) * ((size_t)n_splits + kSplitPad));
-    const size_t o_bias = o_lv + align256(sizeof(double) * n_leaves * K), o_sf = o_bias + align256(sizeof(double) * K);
+    const size_t o_sb = 0, o_bias = o_sb + align256(sizeof(double) * ((size_t)n_splits + kSplitPad));
+    const size_t o_sf = o_bias + align256(sizeof(double) * K);
     const size_t o_so = o_sf + align256(sizeof(uint32_t) * ((size_t)n_splits + kSplitPad));
     const size_t o_lo = o_so + align256(sizeof(uint32_t) * ((size_t)n_trees + 1));
-    const size_t o_na = o_lo + align256(sizeof(uint32_t) * ((size_t)n_trees + 1)), o_x = o_na + align256(F);
+    const size_t o_na = o_lo + align256(sizeof(uint32_t) * ((size_t)n_trees + 1)), o_lv = o_na + align256(F);
+    const size_t o_x = o_lv + align256(sizeof(double) * n_leaves * K);
     const size_t x_bytes = sizeof(float) * n * F, out_bytes = sizeof(double) * n * K;
-    const bool chunked = x_bytes > 2 * kChunkBytes;
-    const uint64_t chunk = chunked ? std::max<uint64_t>(64, kChunkBytes / (sizeof(float) * F) / 64 * 64) : n;
+    // a table in chunks of at least 64 objects; one with more features than that leaves room for,
+    // and a model's leaf values past kPinModel, are uploaded from the caller's memory (pinning
+    // them would take longer than the runtime's copy)
+    const bool big = x_bytes > 2 * kChunkBytes, chunked = big && kChunkBytes / (sizeof(float) * F) >= 64;
+    const bool pin_table = !big, pin_lv = sizeof(double) * n_leaves * K <= kPinModel;
+    const uint64_t chunk = chunked ? kChunkBytes / (sizeof(float) * F) / 64 * 64 : n;
     const size_t x_dev = chunked ? 3 * align256(sizeof(float) * chunk * F) : align256(x_bytes);
     const size_t o_out = o_x + x_dev;
     int dev = 0;
@@ -397,30 +425,46 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
     Lease L(dev);
     Workspace& w = L.ws;
     const bool pin_out = out_bytes <= ((size_t)4 << 20);   // the kernel's results through pinned memory
-    int rc = w.grow(o_out + out_bytes, o_x + x_dev + (pin_out ? out_bytes : 0));
+    // the pinned block: the model's arrays and a small table laid out as on the device, so that they
+    // go up in one copy, or the chunk buffers, then the results
+    const size_t h_x = pin_lv ? o_x : o_lv, h_out = h_x + (chunked || pin_table ? x_dev : 0);
+    int rc = w.grow(o_out + out_bytes, h_out + (pin_out ? out_bytes : 0));
     if (rc != CBH_OK) return rc;
     unsigned char* h = w.pin;
     if (n_splits) std::memcpy(h + o_sb, split_borders, sizeof(double) * n_splits);
     std::memset(h + o_sb + sizeof(double) * n_splits, 0, sizeof(double) * kSplitPad);
-    if (n_leaves) std::memcpy(h + o_lv, leaf_values, sizeof(double) * n_leaves * K);
+    if (n_leaves && pin_lv) std::memcpy(h + o_lv, leaf_values, sizeof(double) * n_leaves * K);
     if (bias) std::memcpy(h + o_bias, bias, sizeof(double) * K);
     if (n_splits) std::memcpy(h + o_sf, split_features, sizeof(uint32_t) * n_splits);
     std::memset(h + o_sf + sizeof(uint32_t) * n_splits, 0, sizeof(uint32_t) * kSplitPad);
     std::memcpy(h + o_so, tree_split_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1));
     std::memcpy(h + o_lo, tree_leaf_offsets, sizeof(uint32_t) * ((size_t)n_trees + 1));
     if (nan_as_true && F) std::memcpy(h + o_na, nan_as_true, F);
-    if (!chunked && x_bytes) std::memcpy(h + o_x, features_fm, x_bytes);
+    if (pin_table && x_bytes) std::memcpy(h + h_x, features_fm, x_bytes);
     const Model M{(const uint32_t*)(w.dev + o_sf), (const double*)(w.dev + o_sb), (const uint32_t*)(w.dev + o_so),
                   (const double*)(w.dev + o_lv), (const uint32_t*)(w.dev + o_lo),
                   bias ? (const double*)(w.dev + o_bias) : nullptr,
                   nan_as_true && F ? (const uint8_t*)(w.dev + o_na) : nullptr, n_trees, F};
     double* d_out = (double*)(w.dev + o_out);
-    APPLY_TRY(hipMemcpyAsync(w.dev, h, chunked ? o_x : o_x + x_bytes, hipMemcpyHostToDevice, w.stream));
-    rc = chunked ? apply_chunks(w, features_fm, n, F, K, M, o_x, o_x, chunk, d_out)
-                 : launch_k(K, (const float*)(w.dev + o_x), n, n, M, d_out, n, w.stream);
+    const bool one_copy = pin_lv && pin_table;
+    APPLY_TRY(hipMemcpyAsync(w.dev, h, one_copy ? o_x + x_bytes : h_x, hipMemcpyHostToDevice, w.stream));
+    if (!pin_lv)
+        APPLY_TRY(hipMemcpyAsync(w.dev + o_lv, leaf_values, sizeof(double) * n_leaves * K, hipMemcpyHostToDevice, w.stream));
+    if (!one_copy && !chunked && x_bytes)
+        APPLY_TRY(hipMemcpyAsync(w.dev + o_x, pin_table ? (const void*)(h + h_x) : features_fm, x_bytes,
+                                 hipMemcpyHostToDevice, w.stream));
+    if (chunked) {
+        try {
+            rc = apply_chunks(w, features_fm, n, F, K, M, o_x, h_x, chunk, d_out);
+        } catch (const std::exception& e) {   // (before its threads are started)
+            rc = cbh_internal_fail(CBH_ERR_DEVICE, std::string("table upload: ") + e.what());
+        }
+    } else {
+        rc = launch_k(K, (const float*)(w.dev + o_x), n, n, M, d_out, n, w.stream);
+    }
     if (rc != CBH_OK) return rc;
     if (pin_out) {
-        unsigned char* ho = h + o_x + x_dev;
+        unsigned char* ho = h + h_out;
         APPLY_TRY(hipMemcpyAsync(ho, d_out, out_bytes, hipMemcpyDeviceToHost, w.stream));
         APPLY_TRY(hipStreamSynchronize(w.stream));
         std::memcpy(out, ho, out_bytes);

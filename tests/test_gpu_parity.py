@@ -1194,10 +1194,12 @@ def test_narrow_tile_fill_histograms(n, F, B, K, loss):
 
 
 @pytest.mark.parametrize("n,F,T,D,K", [(1, 1, 1, 1, 1), (65, 7, 5, 3, 3), (1024, 50, 30, 6, 1), (70_001, 50, 9, 9, 1),
-                                       (1_201, 3_000, 6, 4, 2), (200_000, 16, 11, 17, 1)])
+                                       (1_201, 3_000, 6, 4, 2), (200_000, 16, 11, 17, 1),
+                                       (113, 30_000, 4, 5, 1), (1_000, 5, 5, 18, 1)])
 def test_apply_oblivious_paths_match_reference(n, F, T, D, K):
     """Every route of a prediction call: a small table in one upload, a large one in pinned chunks
-    (over 12 MB; a last chunk that is no multiple of 64), features staged in LDS or, above 512 of
+    (over 12 MB; a last chunk that is no multiple of 64), one too wide for chunks and leaf values
+    past 8 MB from the caller's memory, features staged in LDS or, above 512 of
     them, read through the caches, trees of one to three groups of eight splits, absent features
     and NaN.  The sums are in tree order, so the result is bit-equal to the same order in f64.
     Two host threads predicting at once get the same."""
