@@ -398,6 +398,10 @@ def main():
     traffic, limiter = None, None   # (set below from the committed profile)
     fill_kernel = {0: "fill_kernel", 1: "fill_packed_kernel", 2: "fill_exact_kernel",
                    3: "fill_pkk_kernel", 4: "fill_pks_kernel", 5: "fill_packed_kernel"}[st["fill_mode"]]
+    # the exact fill's tiles: 8 features where the session's rule takes them (narrow_pays), else 32
+    narrow = st["fill_mode"] == 2 and (P["loss"] == "MultiClass" or n < 1 << 16 or n * F <= 1e6 * (51 + 0.615 * n_bins))
+    if narrow:
+        fill_kernel = "fill_narrow_kernel"
     traffic, limiter = _profile_facts(args.config, n, F, fill_kernel)
     names = {1: "config1: RMSE, no bootstrap, depth 6, 128 borders",
              2: ("config2: Logloss, Bayesian bootstrap T=1, depth 6, 254 GreedyLogSum borders selected on the "
@@ -430,7 +434,7 @@ def main():
                   f"u8 bins; int64 sums of rows rounded to {st['fill_pack_bits']}-bit fields of the tree's "
                   f"largest row (coarser than the reference's 2^-30); f64 scores"),
         "fill": {0: "generic 32-feature tiles (one 64-bit atomic per channel, full fixed-point scale)", 1: f"packed 64-feature tiles ({st['fill_pack_bits']}-bit rows)",
-                 2: "tiled exact 32-feature tiles (one 64-bit atomic per channel, full fixed-point scale)",
+                 2: f"tiled exact {8 if narrow else 32}-feature tiles (one 64-bit atomic per channel, full fixed-point scale)",
                  3: f"packed multi-channel 32-feature tiles (two channels per word, {st['fill_pack_bits']}-bit rows)",
                  4: f"packed multi-channel 32-feature tiles over sparse entries (a row per 16-lane DPP row, "
                     f"two channels per word, {st['fill_pack_bits']}-bit rows)",

@@ -216,9 +216,9 @@ struct cbh_session {
     bool count = false;
     bool int_w = true;                         // every object weight is an integer in [0, 2^20]
     uint32_t ex_sets = 3;                      // tiled: blocks in flight of the full loop
-    // narrow-tile exact fill (any K): tiles of kNtWords words, nt_ranges row ranges each
+    // narrow-tile exact fill (any K): tiles of kNtWords words
     bool narrow = false;
-    uint32_t nt_tiles = 0, nt_ranges = 1;
+    uint32_t nt_tiles = 0;
     bool nt_rm = false;                        // gathered levels read row-major words
     bool der_only = false;                     // PairLogitPairwise: the fill adds the der channel only
     // packed multi-channel fill (K > 1: two score channels per 64-bit word, NP = ceil(C/2) planes)
@@ -411,6 +411,17 @@ int validate_config(const cbh_config* cfg, uint32_t n_bins, uint64_t n, uint32_t
     if (n == 0 || F == 0) return fail(CBH_ERR_DEGENERATE, "empty dataset");
     if (n >= (1ull << 32)) return fail(CBH_DECLINED, "more than 2^32-1 rows");
     return CBH_OK;
+}
+
+// The level's finishing and scoring in one launch, or (lds == 0) in two.  One launch saves latency,
+// but its workgroups repeat the row scans and, at many parents, fill a CU's LDS alone, so from
+// 64 parents it has to get by with four rounds of the CUs.  Measured, us a level, one launch
+// against two: 1000 features x 129 bins 32 parents 73 / 87, 64 194 / 173, 128 369 / 283; 300 x 255
+// 64 parents (2.3 rounds) 103 / 110, 128 (4.7) 197 / 153.
+FinishPlan level_finish(const cbh_session* s, uint32_t level) {
+    FinishPlan pl = plan_finish(1u << level, s->K, s->F, s->B, s->cus, s->one_hot != nullptr);
+    if (s->K == 1 && level >= 6 && pl.blocks > 4u * s->cus) pl.lds = 0;
+    return pl;
 }
 
 int launch_zero(long long* p, size_t n, hipStream_t st) {
@@ -735,15 +746,31 @@ bool narrow_pays(uint64_t n, uint32_t F, uint32_t B) {
     return n < (1ull << 16) || (double)n * F <= 1e6 * (51.0 + 0.615 * B);
 }
 
-// Row ranges G of the narrow-tile exact fill.  A launch takes n / G rows a
-// workgroup at 0.75 C cycles each (6 cycles an LDS atomic of a wave) and flushes G images of
-// F B C cells at 1e11 cells/s (both measured): G balances the two, at most one round of the CUs
-// (half and twice that G measured 2-5% slower at 100k rows, the same at 500k and more).
-uint32_t narrow_ranges(const cbh_session* s, uint32_t cus, uint32_t C) {
-    const uint32_t nt = (s->W + kNtWords - 1) / kNtWords;
+// Few rows in many segments: a workgroup pays the latency and the flush of its LDS image for each
+// segment it meets, and many features leave the narrow tiles few ranges to spread the last level's
+// segments over, where the 32-feature tiles have four times as many.  load = segments a range x the
+// image's cells, against the rows (whose atomics the narrow tiles do faster).  Measured, us a
+// tree, these tiles against the others: 3000 x 1000 x 129 bins of depth 8 (load 8256) 1628 / 1126,
+// 3000 x 1000 x 255 of depth 6 (4080) 656 / 639, 5000 x 500 x 128, 6 channels, depth 7 (6144) 1379 /
+// 1090, 100k x 1000 x 129 of depth 8 (8256) 1638 / 1513; below the line 20k x 1000 x 65, 4
+// channels, depth 7 (4160) 848 / 1025, 3000 x 2000 x 33, 3 channels, depth 7 (3168) 684 / 736,
+// 60k x 300 x 255 of depth 8 (5440) 992 / 1002, 500k x 300 x 255 of depth 8 (10880) 1377 / 1457.
+bool narrow_spreads(const cbh_session* s) {
+    const uint32_t nt = (s->W + kNtWords - 1) / kNtWords, segs = s->depth >= 2 ? 1u << (s->depth - 2) : 1u;
+    const uint32_t G = std::max<uint32_t>(1, (uint32_t)s->cus / nt), C = s->pairwise ? 1u : (uint32_t)s->C;
+    return (double)segs / G * s->B * C <= 3500.0 + (double)s->n / 25.0;
+}
+
+// Row ranges G of the narrow-tile exact fill at a level of n_seg segments.  A launch takes n / G
+// rows a workgroup at 0.75 C cycles each (6 cycles an LDS atomic of a wave), about 6 us for each
+// segment past its first (the latency of its loads and of the flush), and flushes G images of F B C
+// cells at 1e11 cells/s (all measured): G balances them, at most one round of the CUs (half and
+// twice that G measured 2-5% slower at 100k rows, the same at 500k and more).
+uint32_t narrow_ranges(const cbh_session* s, uint32_t C, uint32_t n_seg) {
     const double row_us = 0.375 * C * kNtWords / 2400.0, flush_us = (double)s->F * s->B * C * 1e-5;
-    const double best = std::sqrt((double)s->n * row_us / flush_us);
-    return std::max<uint32_t>(1, std::min<uint32_t>(std::max<uint32_t>(1, cus / nt), (uint32_t)best));
+    const double best = std::sqrt(((double)s->n * row_us + 6.0 * (n_seg - 1)) / flush_us);
+    const uint32_t cap = std::max<uint32_t>(1, (uint32_t)s->cus / s->nt_tiles);
+    return std::max<uint32_t>(1, (uint32_t)std::min<double>(cap, best));
 }
 
 template <int C>
@@ -754,7 +781,7 @@ int set_narrow_attr(size_t lds) {
 }
 
 // Takes the narrow-tile exact fill when its tiles fit and its buffers stay within 32-bit offsets.
-int plan_narrow_fill(cbh_session* s, uint32_t cus, bool& taken) {
+int plan_narrow_fill(cbh_session* s, bool& taken) {
     taken = false;
     const uint32_t C = s->pairwise ? 1u : s->C;
     constexpr uint32_t TW = kNtWords;
@@ -762,7 +789,6 @@ int plan_narrow_fill(cbh_session* s, uint32_t cus, bool& taken) {
     if (lds > kNarrowLdsMax || s->n * 8ull * s->C >= (1ull << 31) || s->n * 16ull >= (1ull << 31)) return CBH_OK;
     CHECK(with_k((int)s->K, [&](auto kc) { return set_narrow_attr<decltype(kc)::value + 1>(narrow_lds(s->B, s->C)); }));
     if (C == 1) CHECK(set_narrow_attr<1>(lds));
-    s->nt_ranges = narrow_ranges(s, cus, C);
     s->narrow = true;
     s->nt_tiles = (s->W + TW - 1) / TW;
     s->der_only = s->pairwise;
@@ -781,10 +807,11 @@ int plan_narrow_fill(cbh_session* s, uint32_t cus, bool& taken) {
     return CBH_OK;
 }
 
-// Fill plan.  The default: K == 1 with integer score weights from 2^22 rows the count-packed
-// fill, else from 2^16 rows (2^20 with pairs) the tiled exact fill (which visits every bin: its
-// lanes add to distinct features, so a dominant bin does not serialize them); K > 1 from 500000
-// rows the packed multi-channel fill; otherwise the generic fill.  CBH_FILL (a measurement and
+// Fill plan.  The default: K == 1 the narrow-tile exact fill where it pays (narrow_pays,
+// narrow_spreads), else with integer score weights from 2^22 rows the count-packed fill, else from
+// 2^16 rows (2^20 with pairs) the tiled exact fill (which visits every bin: its lanes add to
+// distinct features, so a dominant bin does not serialize them); K > 1 from 500000 rows the packed
+// multi-channel fill, else the narrow-tile fill; otherwise the generic fill.  CBH_FILL (a measurement and
 // test knob) forces one: =generic the generic fill (any K), =tiled the tiled exact fill (K == 1),
 // =count the count-packed fill (K == 1, integer score weights), =packed the rounded packed fill
 // (K == 1: 18-bit rows) or the packed multi-channel fill (K > 1).
@@ -792,17 +819,15 @@ int plan_fill_mode(cbh_session* s) {
     s->packed = s->tiled = s->pkk = s->count = false;
     const char* e = std::getenv("CBH_FILL");
     const std::string v = e ? e : "";
-    int cus_n = 0;
-    HIP_TRY(hipDeviceGetAttribute(&cus_n, hipDeviceAttributeMultiprocessorCount, s->device));
     bool narrow_taken = false;
     if (s->K > 1) {
         if (v.empty() || v == "packed") CHECK(plan_pkk(s, v));
-        if (!s->pkk && v.empty()) CHECK(plan_narrow_fill(s, (uint32_t)cus_n, narrow_taken));
+        if (!s->pkk && v.empty() && narrow_spreads(s)) CHECK(plan_narrow_fill(s, narrow_taken));
         return CBH_OK;
     }
     if (v == "generic") return CBH_OK;
-    if (v.empty() && narrow_pays(s->n, s->F, s->B)) {
-        CHECK(plan_narrow_fill(s, (uint32_t)cus_n, narrow_taken));
+    if (v.empty() && narrow_pays(s->n, s->F, s->B) && narrow_spreads(s)) {
+        CHECK(plan_narrow_fill(s, narrow_taken));
         if (narrow_taken) return CBH_OK;
     }
     // integer score weights: no per-row sample beyond Bernoulli's keep mask, integer object
@@ -1297,9 +1322,9 @@ int session_open(const cbh_config* cfg, const double* weight, uint64_t n, uint32
     const bool chain_ok = s->K > 1 && s->score_chain && s->cfg.score_function <= CBH_SCORE_L2 && s->max_cand <= 64;
     s->fuse_finish = !s->pairwise && !chain_ok;
     for (uint32_t l = 0; l < s->depth && s->fuse_finish; ++l) {
-        const FinishPlan pl = plan_finish(1u << l, s->K, F, n_bins, s->cus, any_oh);
-        if (pl.lds == 0) s->fuse_finish = false;
-        if (pl.n_parts > 1) s->raw_alt = 1;
+        const FinishPlan pl = level_finish(s.get(), l);
+        if (pl.lds == 0 && s->K > 1) s->fuse_finish = false;
+        if (pl.lds != 0 && pl.n_parts > 1) s->raw_alt = 1;
     }
     if (!s->fuse_finish) s->raw_alt = 0;
     for (uint32_t k = 0; k <= s->raw_alt; ++k) {
@@ -1683,12 +1708,16 @@ int enqueue_prepare(cbh_session* s, const SampleParams& smp, bool use_host_sampl
                           {(uint32_t)(group_count_off(s->n_groups_part, s->depth - 1) + 1) / 2,
                            n_leaves * (uint32_t)leaf_cells<K>(), s->pairwise ? n_leaves * n_leaves : 0u,
                            s->use_skip ? ((uint32_t)s->C << (s->depth - 1)) + s->C : 0u}};
-    prepare_kernel<K><<<grid_for(n, 256, kPrepBlocks), 256, 0, st>>>(
+    // the raw rows of the last level, where no level after it clears them: a few stores a thread also
+    // where the rows are few (3000 x 1000, depth 8: 168 us on the rows' own 12 workgroups)
+    const FinishPlan lastf = level_finish(s, s->depth - 1);
+    const size_t n_zraw = s->raw_alt && lastf.lds != 0 && lastf.n_parts > 1 ? s->raw_cells : 0;
+    prepare_kernel<K><<<grid_for(std::max<uint64_t>(n, n_zraw / 8), 256, kPrepBlocks), 256, 0, st>>>(
         n, loss, s->approx, s->target, s->weight, s->leaf,
         apply_prev && !s->ranking ? s->leaf_scaled : nullptr,   // a pair loss applied them above
         smp, s->jt(), use_host_sample ? s->host_sample : nullptr, s->sstat, newton, s->slots,
         s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, clear,
-        s->raw_alt ? s->raw[(s->depth - 1) & 1] : nullptr, s->raw_alt ? s->raw_cells : 0);
+        s->raw[(s->depth - 1) & s->raw_alt], n_zraw);
     HIP_TRY(hipGetLastError());
     return s->stage_end();
 }
@@ -1724,6 +1753,7 @@ int enqueue_tree(cbh_session* s) {
 
     const size_t per_leaf = (size_t)s->F * s->B * C;
     const uint32_t NB = s->n_part_blocks;
+    uint32_t prev_parts = 1;   // workgroups a feature of the level before's finishing
     for (uint32_t level = 0; level < s->depth; ++level) {
         long long* cur = s->hist[level & 1];
         long long* par = s->hist[(level + 1) & 1];
@@ -1762,14 +1792,15 @@ int enqueue_tree(cbh_session* s) {
                 s->trows, s->W, n, lidx, lplan, s->spack, s->sseq, s->pk_gath.tiles16, s->F, s->B,
                 s->pk_gath.ranges, 0u, raw, 0u, s->pk_rm_sh ? s->rows : nullptr, s->pk_rm_sh, s->scales);
         else if (s->narrow) {
-            const unsigned blocks = 8 * ((s->nt_tiles * s->nt_ranges + 7) / 8);
+            const uint32_t ranges = narrow_ranges(s, s->der_only ? 1u : (uint32_t)C, n_seg);
+            const unsigned blocks = 8 * ((s->nt_tiles * ranges + 7) / 8);
             const uint32_t rb = 4u * s->Ws;
             auto launch = [&](auto cc) {
                 constexpr int CF = decltype(cc)::value;   // channels filled
                 const size_t lds = narrow_lds(s->B, CF);
                 (level == 0 ? fill_narrow_kernel<CF, false> : fill_narrow_kernel<CF, true>)<<<blocks, kNtThreads, lds, st>>>(
                     s->trows, s->W, n, lidx, lplan, s->sstat, s->C, (const double*)s->sseq, s->nt_tiles, s->F, s->B,
-                    s->nt_ranges, raw, level > 0 && s->nt_rm ? s->rows : nullptr, rb, s->scales, s->slots, s->bounds);
+                    ranges, raw, level > 0 && s->nt_rm ? s->rows : nullptr, rb, s->scales, s->slots, s->bounds);
             };
             if (s->der_only) launch(std::integral_constant<int, 1>{});
             else launch(std::integral_constant<int, C>{});
@@ -1864,10 +1895,13 @@ int enqueue_tree(cbh_session* s) {
         }
         // ---- histogram finishing: dominant bins, prefix form, siblings; K = 1 with the scoring ----
         const bool last = level + 1 == s->depth;
-        const bool finish = s->fuse_finish;
+        const FinishPlan pl = level_finish(s, level);
+        const bool finish = s->fuse_finish && pl.lds != 0;
         uint32_t parts = 1;   // best entries a feature
         if (!finish) {
             CHECK(s->stage_begin(kStDerive));
+            if (prev_parts > 1)   // left by the level before, whose finishing had several readers a row
+                CHECK(launch_zero(s->raw[(level - 1) & s->raw_alt], per_leaf * std::max(1u, n_seg / 2), st));
             // (PairLogitPairwise fills and reads the der channel only)
             const bool der_only = s->pairwise && !s->packed && !s->count && (!s->tiled || s->der_only) && !s->use_skip;
             const uint32_t CU = der_only ? 1u : (uint32_t)C;
@@ -1904,7 +1938,6 @@ int enqueue_tree(cbh_session* s) {
         } else if (finish) {
             // (the last level's rows are read by nothing after it)
             const int keep = !last || s->hist_cap ? 1 : 0;
-            const FinishPlan pl = plan_finish(n_leaves, K, s->F, s->B, s->cus, s->one_hot != nullptr);
             parts = pl.n_parts;
             finish_score_kernel<K><<<pl.blocks, kFinishThreads, pl.lds, st>>>(
                 raw, cur, lplan, n_seg, level > 0 ? par : nullptr, n_leaves, s->F, s->B, pl.nf, pl.m, pl.n_parts, pl.nt,
@@ -1937,7 +1970,7 @@ int enqueue_tree(cbh_session* s) {
                         sfn, s->best_score, s->best_bin, s->ctr_n ? s->fweight : nullptr, s->chain_spin,
                         &s->bounds->device_err, nf);
             }
-        } else if constexpr (K > 1) {   // (K = 1 always finishes and scores in one launch)
+        } else {
             if (s->max_cand <= 64)
                 score_kernel<K, 1><<<s->F, 64, 0, st>>>(cur, n_leaves, s->F, s->B, s->n_cand, s->one_hot,
                                                    s->scales, s->l2, sfn, s->best_score, s->best_bin,
@@ -1955,6 +1988,7 @@ int enqueue_tree(cbh_session* s) {
         if (s->hist_cap)   // the level's histograms as the scorer reads them (inspection only)
             HIP_TRY(hipMemcpyAsync(s->hist_cap + s->hist_cap_off[level], cur, sizeof(long long) * per_leaf * n_leaves,
                                    hipMemcpyDeviceToDevice, st));
+        prev_parts = parts;
         const bool fuse_argmax = s->F * parts <= kArgmaxFuse;
         if (!fuse_argmax) {
             argmax_kernel<<<1, 1024, 0, st>>>(s->best_score, s->best_bin, s->pairwise ? nullptr : s->one_hot, s->F,

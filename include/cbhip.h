@@ -219,8 +219,8 @@ typedef struct {
     uint32_t fill_mode;           /* 0: generic fill (32-feature tiles, one exact 64-bit atomic per channel,
                                      any K); 1: rounded packed fill (K = 1, 64-feature tiles, both channels
                                      rounded to 18-bit rows in one 64-bit atomic); 2: tiled exact fill (K = 1,
-                                     32-feature tiles, one exact 64-bit atomic per channel, DPP-broadcast
-                                     statistics); 3: packed multi-channel fill (K > 1, 32-feature tiles, two
+                                     32-feature tiles, or any K, 8-feature tiles; one exact 64-bit atomic
+                                     per channel, DPP-broadcast statistics); 3: packed multi-channel fill (K > 1, 32-feature tiles, two
                                      channels rounded to 20-bit rows per 64-bit atomic); 4: the same cells
                                      over sparse entries (a row per 16-lane DPP row, one lane per
                                      non-dominant (feature, bin)); 5: count-packed fill (K = 1, integer

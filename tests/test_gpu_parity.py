@@ -1228,3 +1228,24 @@ def test_apply_oblivious_paths_match_reference(n, F, T, D, K):
         for got in ex.map(lambda _: cb.apply_oblivious(x, sf, sb, so, lv, lo, approx_dim=K, bias=bias, nan_as_true=na),
                           range(4)):
             assert np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("n,F,borders,depth", [(1_500, 300, 254, 8), (900, 400, 128, 8), (1_200, 100, 254, 7),
+                                               (700, 1_100, 32, 7)])
+def test_deep_trees_over_few_rows(n, F, borders, depth):
+    """Deep trees over few rows and many features: levels of 64 and 128 parents finish and score in one
+    launch or in two (more than four rounds of workgroups), the raw rows that several workgroups of a
+    feature read are cleared by the next level's launch, by its own, or by the next tree's prepare,
+    and the fill goes back to the generic one where the narrow tiles meet too many segments.  Three
+    trees, so that a cell left over from one shows in the next; splits equal the oracle's."""
+    bins, nb, y, w = datagen.random_case(n + F, n, F, max_borders=borders)
+    params = dict(loss="RMSE", score="Cosine", leaf_method="Gradient", bootstrap_type="No", depth=depth,
+                  learning_rate=0.3, l2_leaf_reg=3.0, random_seed=1)
+    exp = O.train(bins, nb, y, iterations=3, weight=w, **params)
+    tr = cb.Trainer(bins, int(nb.max()) + 1, y, weight=w, real_folds=nb + 1, **params)
+    try:
+        splits, leaves = tr.fit(3)
+    finally:
+        tr.close()
+    assert np.array_equal(splits, exp["splits"])
+    _close(leaves, exp["leaf_values"])
