@@ -3882,25 +3882,29 @@ __device__ inline int cholesky_solve_dev(int k, double* a, const double* b, doub
     return 1;
 }
 
-// Leaf values (leaf.rs:161-335): one thread per leaf.  raw[leaf][d] unscaled, scaled =
-// raw * learning_rate (NormalizeLeafValues, boosting.rs:2879-2881).
 // The tree's results to the host: the device block's words into its pinned mirror (a copy node
-// costs twice the kernel's launch).
-__device__ __forceinline__ void publish(const uint4* __restrict__ src, uint4* __restrict__ host, uint32_t n16) {
-    for (uint32_t i = threadIdx.x; i < n16; i += blockDim.x) host[i] = src[i];
+// costs twice the kernel's launch).  The block holds doubles and records that the same launch may have
+// stored, so src is not __restrict__ and its words are copied as bytes.
+__device__ __forceinline__ void publish(const uint4* src, uint4* __restrict__ host, uint32_t n16) {
+    for (uint32_t i = threadIdx.x; i < n16; i += blockDim.x) {
+        uint4 v;
+        __builtin_memcpy(&v, src + i, sizeof(v));
+        host[i] = v;
+    }
 }
-static __global__ __launch_bounds__(256) void publish_kernel(const uint4* __restrict__ src, uint4* __restrict__ host,
-                                                             uint32_t n16) {
+static __global__ __launch_bounds__(256) void publish_kernel(const uint4* src, uint4* __restrict__ host, uint32_t n16) {
     publish(src, host, n16);
 }
 
-// K == 1: one workgroup of 256 threads (at most 256 leaves), which then publishes the results
-// (raw is part of the block).
+// Leaf values (leaf.rs:161-335): one thread per leaf.  raw[leaf][d] unscaled, scaled =
+// raw * learning_rate (NormalizeLeafValues, boosting.rs:2879-2881).  K == 1: one workgroup of 256
+// threads (at most 256 leaves), which then publishes the results: raw lies inside out's block, so
+// neither is __restrict__ (the compiler could otherwise read the block ahead of the stores).
 template <int K>
 static __global__ void leaf_values_kernel(const long long* __restrict__ sums, const Scales* __restrict__ sc,
                                    uint32_t n_leaves, int newton, double l2, double lr,
-                                   double* __restrict__ raw, double* __restrict__ scaled,
-                                   const uint4* __restrict__ out /* nullable: nothing to publish */,
+                                   double* raw, double* __restrict__ scaled,
+                                   const uint4* out /* nullable: nothing to publish */,
                                    uint4* __restrict__ host, uint32_t n16) {
     constexpr int CL = leaf_cells<K>();
     const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
