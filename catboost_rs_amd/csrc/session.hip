@@ -104,6 +104,8 @@ int cbh_internal_ctr_bins(const cbh_device_ctr_column* cols, uint32_t m, const u
 int cbh_internal_quantize(const float* d_col, uint64_t n, const double* d_borders, uint32_t nb, uint8_t* d_out,
                           hipStream_t st);  // borders.hip
 
+constexpr uint32_t kNoLevel = 0xFFFFFFFFu;
+
 struct cbh_session {
     cbh_config cfg{};
     std::vector<uint8_t> one_hot_host;
@@ -282,6 +284,10 @@ struct cbh_session {
     // per-tree launch sequence after prepare, recorded once and replayed
     hipGraphExec_t tree_graph = nullptr;
     bool graph_off = false;          // recording failed once: stay eager
+    // a tree was begun and has not ended: until its last kernels have run, the raw rows and the bound
+    // slots hold its sums, which only those kernels clear
+    bool dirty = false;
+    uint32_t fail_level = kNoLevel;  // a test's forced failure (cbh_internal_fail_level)
     // the per-tree results (splits, plans, bounds, raw leaves) live in one device block, which the
     // tree's last kernel writes to its pinned mirror; the pointers below are views into the blocks
     unsigned char* out_dev = nullptr;
@@ -1696,6 +1702,7 @@ int enqueue_prepare(cbh_session* s, const SampleParams& smp, bool use_host_sampl
         if (apply_prev) {
             apply_leaves_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(s->approx, s->leaf, s->leaf_scaled, n);
             HIP_TRY(hipGetLastError());
+            s->pending = false;
         }
         pairlogit_row_ders_kernel<<<grid_for(n, 256), 256, 0, st>>>(n, s->comp_off, s->comp_win, s->comp_los,
                                                                   s->comp_w, s->los_off, s->los_idx, s->approx,
@@ -1719,6 +1726,7 @@ int enqueue_prepare(cbh_session* s, const SampleParams& smp, bool use_host_sampl
         s->ranking ? s->ext_der : nullptr, s->ranking ? s->score_w : nullptr, clear,
         s->raw[(s->depth - 1) & s->raw_alt], n_zraw);
     HIP_TRY(hipGetLastError());
+    s->pending = false;   // (applied, also if the tree does not end)
     return s->stage_end();
 }
 
@@ -1755,6 +1763,7 @@ int enqueue_tree(cbh_session* s) {
     const uint32_t NB = s->n_part_blocks;
     uint32_t prev_parts = 1;   // workgroups a feature of the level before's finishing
     for (uint32_t level = 0; level < s->depth; ++level) {
+        if (level == s->fail_level) return fail(CBH_ERR_DEVICE, "forced failure");
         long long* cur = s->hist[level & 1];
         long long* par = s->hist[(level + 1) & 1];
         const uint32_t n_leaves = 1u << level;
@@ -2025,6 +2034,7 @@ int enqueue_tree(cbh_session* s) {
                                                                       s->F - s->ctr_n, s->ctr_avg);
         HIP_TRY(hipGetLastError());
     }
+    if (s->depth == s->fail_level) return fail(CBH_ERR_DEVICE, "forced failure");
     CHECK(s->stage_begin(kStLeaf));
     const uint32_t n_leaves = 1u << s->depth;
     const uint32_t CL = (uint32_t)leaf_cells<K>();
@@ -2110,17 +2120,25 @@ int grow_impl(cbh_session* s, const SampleParams& smp, bool use_host_sample,
         s->pin_ctr_used[s->ctr_n] = ctr_all_used(s) ? 1 : 0;   // then no phantom count is needed
         HIP_TRY(hipMemcpyAsync(s->ctr_used_dev, s->pin_ctr_used, s->ctr_n + 1, hipMemcpyHostToDevice, st));
     }
-    const bool replay = (s->pending || s->tree_graph) && !s->cfg.profile && !s->graph_off && ctr_static && !s->hist_cap;
+    const bool replay = (s->pending || s->tree_graph) && !s->cfg.profile && !s->graph_off && ctr_static && !s->hist_cap &&
+                        s->fail_level == kNoLevel;
     if (replay && !s->tree_graph) record_tree<K>(s);
+    if (s->dirty) {   // the tree before ended in an error: what its kernels had added goes
+        for (uint32_t k = 0; k <= s->raw_alt; ++k) CHECK(launch_zero(s->raw[k], s->raw_cells, st));
+        CHECK(launch_zero((long long*)s->slots, (size_t)kBoundSlots * kPartials, st));
+        s->timer_used = 0;
+    }
+    s->dirty = true;
     CHECK(enqueue_prepare<K>(s, smp, use_host_sample));
     if (replay && s->tree_graph) {
         HIP_TRY(hipGraphLaunch(s->tree_graph, st));
     } else {
         CHECK(enqueue_tree<K>(s));
     }
-    s->pending = true;
     if (s->overlap_fn) s->overlap_fn(s->overlap_arg);   // host work while the tree grows
     HIP_TRY(hipStreamSynchronize(st));
+    s->dirty = false;
+    s->pending = true;
     const size_t n_leaves = (size_t)1 << s->depth;
     splits_out.assign(s->pin_splits, s->pin_splits + s->depth);
     plans_out.assign(s->pin_plans, s->pin_plans + s->depth);
@@ -2477,6 +2495,12 @@ void cbh_internal_set_overlap(cbh_session* s, void (*fn)(void*), void* arg) {
     if (!s) return;
     s->overlap_fn = fn;
     s->overlap_arg = arg;
+}
+
+// Tests: the session's next trees end with an error on the host before they launch this level (the
+// depth: before the leaf values); any larger level ends that.
+void cbh_internal_fail_level(cbh_session* s, uint32_t level) {
+    if (s) s->fail_level = level <= s->depth ? level : kNoLevel;
 }
 
 int cbh_session_set_profile(cbh_session* s, int32_t on) {

@@ -1249,3 +1249,54 @@ def test_deep_trees_over_few_rows(n, F, borders, depth):
         tr.close()
     assert np.array_equal(splits, exp["splits"])
     _close(leaves, exp["leaf_values"])
+
+
+# ------------------------------------------------------------------ a tree that ends in an error
+@pytest.mark.parametrize("loss,n,F,B,K,depth", [
+    ("RMSE", 3_000, 12, 33, 1, 4),           # one reader a raw row
+    ("Logloss", 2_000, 300, 255, 1, 5),      # several readers a raw row: two raw buffers
+    ("MultiClass", 4_000, 9, 20, 3, 4), ("PairLogit", 2_000, 10, 40, 1, 4), ("PairLogitPairwise", 2_000, 10, 40, 1, 4)])
+def test_session_goes_on_after_a_failed_tree(loss, n, F, B, K, depth):
+    """Trees that end with an error on the host (forced after the first kernels, between two levels
+    and before the leaf values) leave nothing behind: the same tree grown again, and the next,
+    are bit-equal to those of a session that never failed, as is the approximant read between."""
+    g = np.random.default_rng(n + F)
+    bins = g.integers(0, B, (F, n)).astype(np.uint8)
+    y = g.integers(0, max(K, 2), n).astype(np.float64) + (g.standard_normal(n) if loss == "RMSE" else 0.0)
+    fam = None
+    if loss.startswith("PairLogit"):
+        a, b = np.arange(0, n, 2), np.arange(1, n, 2)
+        fam = (np.arange(0, n + 1, 10, dtype=np.uint32), np.where(y[a] >= y[b], a, b).astype(np.uint32),
+               np.where(y[a] >= y[b], b, a).astype(np.uint32))
+    fail_level = cb.load().cbh_internal_fail_level
+    fail_level.argtypes, fail_level.restype = [C.c_void_p, C.c_uint32], None
+
+    def grow(failures):
+        be = cb.HipBackend()
+        assert be.begin_device_training(loss, depth, True, 1, "Cosine", bins, None, n, F, B, 0.3, 3.0, approx_dim=K,
+                                        leaf_method="Newton" if K > 1 else "Gradient",
+                                        real_folds=np.full(F, B, np.uint32))
+        out = []
+        try:
+            for it in range(4):
+                args = dict(target=y, family=fam) if it == 0 else {}
+                for level in failures.get(it, ()):
+                    fail_level(be._s, level)
+                    with pytest.raises(cb.CbhError, match="forced"):
+                        be.grow_tree_on_device(**args)
+                    fail_level(be._s, depth + 1)
+                    if level == 1:   # the trees before are applied, once
+                        out.append(be.read_approx())
+                if it in (1, 3) and not failures:
+                    out.append(be.read_approx())
+                t = be.grow_tree_on_device(want_leaf_of=True, **args)
+                out += [np.array(t["splits"]), t["leaf_values"], t["leaf_of"], t["scores"]]
+            out.append(be.read_approx())
+        finally:
+            be.end_device_training()
+        return out
+
+    plain, failed = grow({}), grow({0: (0,), 1: (depth, 1), 2: (2,), 3: (1, 3)})
+    assert len(plain) == len(failed)
+    for x, z in zip(plain, failed):
+        assert np.array_equal(x, z)
