@@ -13,17 +13,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
 #include "../../include/cbhip.h"
 #include "common.hpp"
+#include "copy_threads.hpp"
 
 int cbh_internal_fail(int code, const std::string& msg);  // session.hip
 
@@ -311,45 +310,16 @@ int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, ui
     for (auto& e : w.ev)
         if (!e) APPLY_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (!w.copy) APPLY_TRY(hipStreamCreateWithFlags(&w.copy, hipStreamNonBlocking));
-    const unsigned want = copy_threads();
-    // chunk c may be filled once `open` is past it; `done[c]` counts the threads that have copied
-    // their features of it.  `threads` is how many there are, 0 until all have been started; the
-    // calling thread copies when none could be.
-    std::atomic<unsigned> threads{0};
-    std::atomic<uint64_t> open{std::min<uint64_t>(2, n_chunks)};
-    std::vector<std::atomic<uint32_t>> done(n_chunks);
-    for (auto& d : done) d.store(0, std::memory_order_relaxed);
-    std::atomic<bool> stop{false};
     auto copy_chunk = [&](uint64_t c, uint32_t first, uint32_t step) {
         const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
         float* dst = (float*)(w.pin + pin_x + (c % 3) * cbytes);
         for (uint32_t f = first; f < F; f += step)
             std::memcpy(dst + (size_t)f * m, features + (size_t)f * n + o0, sizeof(float) * m);
     };
-    auto copy = [&](unsigned t) {
-        unsigned T;
-        while ((T = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
-        for (uint64_t c = 0; c < n_chunks; ++c) {
-            while (open.load(std::memory_order_acquire) <= c) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                std::this_thread::yield();
-            }
-            copy_chunk(c, t, T);
-            done[c].fetch_add(1, std::memory_order_release);
-        }
-    };
-    std::vector<std::thread> pool;
+    cbh::CopyThreads<decltype(copy_chunk)> threads(copy_threads(), n_chunks, std::min<uint64_t>(2, n_chunks), copy_chunk);
     int rc = CBH_OK;
-    pool.reserve(want);
-    try {
-        for (unsigned t = 0; t < want; ++t) pool.emplace_back(copy, t);
-    } catch (const std::system_error&) {   // no more threads: those there are take all of it
-    }
-    const unsigned T = (unsigned)pool.size();
-    threads.store(T, std::memory_order_release);
     for (uint64_t c = 0; c < n_chunks && rc == CBH_OK; ++c) {
-        if (T == 0) copy_chunk(c, 0, 1);   // (its buffer is free: waited for below, two chunks ago)
-        while (done[c].load(std::memory_order_acquire) < T) std::this_thread::yield();
+        threads.wait(c);
         const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
         const size_t b = (c % 3) * cbytes;
         float* dx = (float*)(w.dev + dev_x + b);
@@ -365,11 +335,9 @@ int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, ui
             if (c >= 1 && hipEventSynchronize(w.ev[(c - 1) % 3]) != hipSuccess)
                 rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
             else
-                open.store(c + 3, std::memory_order_release);
+                threads.open(c + 3);
         }
     }
-    stop.store(true);
-    for (auto& th : pool) th.join();
     return rc;
 }
 
@@ -456,7 +424,7 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
     if (chunked) {
         try {
             rc = apply_chunks(w, features_fm, n, F, K, M, o_x, h_x, chunk, d_out);
-        } catch (const std::exception& e) {   // (before its threads are started)
+        } catch (const std::exception& e) {   // (its threads are joined)
             rc = cbh_internal_fail(CBH_ERR_DEVICE, std::string("table upload: ") + e.what());
         }
     } else {
