@@ -1,7 +1,9 @@
 // Host threads that copy a table chunk by chunk while the caller passes the finished chunks on.
 #pragma once
 #include <atomic>
+#include <condition_variable>
 #include <cstdint>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -12,6 +14,10 @@ namespace cbh {
 // it.  Threads that cannot be started, for whatever reason, are done without: those there take all
 // of it, the caller if there is none.  The destructor ends and joins them wherever they are, so an
 // exception on the caller's side leaves no thread behind.
+//
+// A wait gives way kYields times, then blocks.  Waits that only gave way kept eight threads and the
+// caller running for the whole call: 500k x 100, 500 trees 36 ms of CPU time in a call of 4.70 ms, 16 ms
+// in 4.66 ms this way; 100k x 40 0.61 ms both ways (blocking at once: 0.67 ms, the wake-ups).
 template <class Copy>
 class CopyThreads {
   public:
@@ -22,42 +28,63 @@ class CopyThreads {
             for (unsigned t = 0; t < want; ++t) pool_.emplace_back([this, t] { work(t); });
         } catch (...) {
         }
-        count_.store((unsigned)pool_.size(), std::memory_order_release);
+        count_ = (unsigned)pool_.size();
         started_.store(true, std::memory_order_release);
     }
     CopyThreads(const CopyThreads&) = delete;
     CopyThreads& operator=(const CopyThreads&) = delete;
     ~CopyThreads() {
-        stop_.store(true);
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            stop_ = true;
+        }
+        opened_.notify_all();
         for (auto& t : pool_) t.join();
     }
 
     // Chunks below n may be filled.
-    void open(uint64_t n) { open_.store(n, std::memory_order_release); }
+    void open(uint64_t n) {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            open_ = n;
+        }
+        opened_.notify_all();
+    }
 
     // Returns once chunk c, which has to be open, is copied.
     void wait(uint64_t c) {
-        const unsigned T = count_.load(std::memory_order_relaxed);
-        if (T == 0) copy_(c, 0, 1);
-        while (done_[c].load(std::memory_order_acquire) < T) std::this_thread::yield();
+        if (count_ == 0) copy_(c, 0, 1);
+        await(copied_, [&] { return done_[c] >= count_; });
     }
 
   private:
+    static constexpr int kYields = 100;
+    template <class Ready>
+    void await(std::condition_variable& cv, Ready ready) {
+        for (int k = 0; k < kYields; ++k) {
+            if (ready()) return;
+            std::this_thread::yield();
+        }
+        std::unique_lock<std::mutex> lock(mu_);
+        cv.wait(lock, ready);
+    }
     void work(unsigned t) {
-        while (!started_.load(std::memory_order_acquire)) std::this_thread::yield();
-        const unsigned T = count_.load(std::memory_order_acquire);
+        while (!started_.load(std::memory_order_acquire)) std::this_thread::yield();   // (while the others start)
         for (uint64_t c = 0; c < done_.size(); ++c) {
-            while (open_.load(std::memory_order_acquire) <= c) {
-                if (stop_.load(std::memory_order_relaxed)) return;
-                std::this_thread::yield();
+            await(opened_, [&] { return stop_ || open_ > c; });
+            if (stop_) return;
+            copy_(c, t, count_);
+            if (done_[c].fetch_add(1) + 1 == count_) {
+                { std::lock_guard<std::mutex> lock(mu_); }   // (a caller between its look and its wait)
+                copied_.notify_one();
             }
-            copy_(c, t, T);
-            done_[c].fetch_add(1, std::memory_order_release);
         }
     }
 
     Copy copy_;
-    std::atomic<unsigned> count_{0};
+    std::mutex mu_;
+    std::condition_variable opened_, copied_;
+    unsigned count_ = 0;
     std::atomic<bool> started_{false}, stop_{false};
     std::atomic<uint64_t> open_;
     std::vector<std::atomic<uint32_t>> done_;

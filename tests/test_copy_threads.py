@@ -62,17 +62,62 @@ int main() {
 """
 
 
-def test_copy_threads_survive_failed_starts(tmp_path):
-    """A thread that cannot be started (its allocation fails) costs neither the call nor the process:
-    the table is copied once by those there, by the caller if there is none, and a caller that
-    breaks off with an exception in the middle leaves no thread behind."""
+WAITING = r"""
+#include <chrono>
+#include <cstdio>
+#include <ctime>
+
+#include "copy_threads.hpp"
+
+static double cpu() {
+    timespec t;
+    clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t);
+    return t.tv_sec + 1e-9 * t.tv_nsec;
+}
+
+int main() {
+    std::atomic<int> copies{0};
+    auto slow = [&](uint64_t c, uint32_t, uint32_t) {   // chunk 1: the caller waits for its threads
+        if (c == 1) std::this_thread::sleep_for(std::chrono::milliseconds(400));
+        ++copies;
+    };
+    const double t0 = cpu();
+    {
+        cbh::CopyThreads<decltype(slow)> threads(4, 3, 2, slow);
+        threads.wait(0);
+        threads.wait(1);
+        std::this_thread::sleep_for(std::chrono::milliseconds(400));   // its threads wait for chunk 2
+        threads.open(3);
+        threads.wait(2);
+    }
+    std::printf("%d copies, %.3f\n", copies.load(), cpu() - t0);
+    return 0;
+}
+"""
+
+
+def _run(tmp_path, program):
     cxx = shutil.which("g++")
     if not cxx:
         pytest.skip("no host compiler")
     src, exe = tmp_path / "t.cpp", tmp_path / "t"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-pthread", "-I",
                     os.path.join(ROOT, "catboost_rs_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
-    assert r.stdout == "11 whole, 4 refused\n"
+    return r.stdout
+
+
+def test_waiting_threads_sleep(tmp_path):
+    """400 ms in which the caller waits for its threads and 400 ms in which they wait for it: threads
+    that only gave way would run for 0.4 s of CPU time or more in each, sleeping ones for almost none."""
+    copies, cpu = _run(tmp_path, WAITING).split(" copies, ")
+    assert copies == "12" and float(cpu) < 0.2
+
+
+def test_copy_threads_survive_failed_starts(tmp_path):
+    """A thread that cannot be started (its allocation fails) costs neither the call nor the process:
+    the table is copied once by those there, by the caller if there is none, and a caller that
+    breaks off with an exception in the middle leaves no thread behind."""
+    assert _run(tmp_path, PROGRAM) == "11 whole, 4 refused\n"
