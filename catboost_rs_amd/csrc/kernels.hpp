@@ -3353,6 +3353,8 @@ static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __res
 //   split_count: the level's argmax, then leaf |= pass << level for every row; counts of sampled
 //                rows per new leaf of every wave (cnt[wave][leaf]) and of every group of
 //                kGroupBlocks workgroups (gcnt[group][leaf], added atomically)
+//   group_scan:  (many rows in many leaves: scan_groups) the group counts to the rows of the groups
+//                before, and the leaf totals
 //   compact:     leaf totals and the rows before this workgroup from the group counts and its
 //                own group's wave counts; the plan (smaller child per parent, ties -> the TRUE
 //                child, tree.rs:1109, and the segment offsets of the next fill) from the totals;
@@ -3361,7 +3363,8 @@ static __global__ __launch_bounds__(1024) void argmax_kernel(const double* __res
 //                and mbcnt, across waves from per-wave counts in LDS.
 // A dependent launch costs 4.6-5.7 us whatever it does, so the argmax (a workgroup over F scores)
 // and the scan of the counts ride in the kernels that need their results: each workgroup of
-// split_count repeats the argmax, each workgroup of compact sums the counts before it.
+// split_count repeats the argmax, each workgroup of compact sums the counts before it (while those
+// are few).
 // ---------------------------------------------------------------------------------
 // Rows per wave (4 waves a workgroup): PR = 1024 keeps the counts few at many rows, 256 shortens
 // the waves' chains (a row a lane at a time) where workgroups are too few to fill the chip.
@@ -3369,7 +3372,7 @@ constexpr uint32_t kPartSmall = 256, kPartLarge = 1024;
 constexpr uint64_t kPartSmallMaxRows = 1u << 20;
 inline uint32_t part_wave_rows(uint64_t n) { return n <= kPartSmallMaxRows ? kPartSmall : kPartLarge; }
 // Workgroups a group of the counts covers: compact reads groups + 4 kGroupBlocks counts per leaf
-// (10M rows: 153 + 64), and a group count takes kGroupBlocks atomics on one address (about 66 ns
+// (10M rows: 153 + 64; of many groups' counts its own one's, after a scan), and a group count takes kGroupBlocks atomics on one address (about 66 ns
 // each, one after another, 1 us in all).
 constexpr uint32_t kGroupBlocks = 16;
 __host__ __device__ inline uint32_t part_groups(uint32_t n_blocks) { return (n_blocks + kGroupBlocks - 1) / kGroupBlocks; }
@@ -3461,6 +3464,40 @@ static __global__ __launch_bounds__(256) void split_count_kernel(
     }
 }
 
+// Group counts [group][leaf] to the rows of the groups before, and every leaf's total: a workgroup a
+// leaf, 1024 groups at a time (latency: a load, a scan and a barrier each, two rounds at 120M rows).
+constexpr uint32_t kScanThreads = 1024;
+static __global__ __launch_bounds__(kScanThreads) void group_scan_kernel(uint32_t* __restrict__ gcnt, uint32_t n_groups,
+                                                                         uint32_t n_new, uint32_t* __restrict__ totals) {
+    constexpr uint32_t NW = kScanThreads / 64;
+    __shared__ uint32_t sums[2][NW];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    uint32_t run = 0, buf = 0;
+    for (uint32_t g0 = 0; g0 < n_groups; g0 += kScanThreads, buf ^= 1u) {   // workgroup-uniform
+        const uint32_t g = g0 + threadIdx.x;
+        uint32_t* at = gcnt + (size_t)g * n_new + blockIdx.x;
+        const uint32_t v = g < n_groups ? *at : 0u;
+        uint32_t inc = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = __shfl_up(inc, o, 64);
+            if (lane >= (uint32_t)o) inc += u;
+        }
+        if (lane == 63) sums[buf][wave] = inc;
+        __syncthreads();   // (the other buffer's readers pass it only after reading it)
+        uint32_t before = run, all = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < NW; ++w) {
+            const uint32_t t = sums[buf][w];
+            before += w < wave ? t : 0u;
+            all += t;
+        }
+        if (g < n_groups) *at = before + inc - v;
+        run += all;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
+
 // Stable compaction of the rows of every directly built child into idx (grouped by parent in
 // plan order, object order inside each group).  Each wave walks its own rows with per-leaf
 // running offsets in its LDS slice (seeded from the scanned per-wave counts), so the loop
@@ -3478,6 +3515,7 @@ template <int SPW, uint32_t PR>
 static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __restrict__ leaf, uint64_t n,
                                                       uint32_t level, const uint32_t* __restrict__ cnt,
                                                       const uint32_t* __restrict__ gcnt, uint32_t n_groups,
+                                                      const uint32_t* __restrict__ totals /* nullable: not scanned */,
                                                       LevelPlan* __restrict__ plan,
                                                       uint32_t* __restrict__ idx,
                                                       const unsigned long long* __restrict__ sp_in,
@@ -3509,11 +3547,18 @@ static __global__ __launch_bounds__(256) void compact_kernel(const uint16_t* __r
         const uint32_t w0 = group * kGroupBlocks * 4, w1 = blockIdx.x * 4;   // its group's waves before this block
         uint32_t t = 0, p = 0;
         const uint32_t cells = n_groups * n_new, before = group * n_new;
+        if (totals) {   // gcnt holds the rows before each group
+            if (threadIdx.x < n_new) {
+                t = totals[threadIdx.x];
+                p = gcnt[before + threadIdx.x];
+            }
+        } else {
 #pragma unroll 4
-        for (uint32_t i = threadIdx.x; i < cells; i += 256) {
-            const uint32_t v = gcnt[i];
-            t += v;
-            p += i < before ? v : 0u;
+            for (uint32_t i = threadIdx.x; i < cells; i += 256) {
+                const uint32_t v = gcnt[i];
+                t += v;
+                p += i < before ? v : 0u;
+            }
         }
         const uint32_t* own = cnt + (size_t)w0 * n_new;
         const uint32_t own_cells = (w1 - w0) * n_new;

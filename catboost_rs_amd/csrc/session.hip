@@ -139,6 +139,7 @@ struct cbh_session {
     size_t hist_cells_max = 0, raw_cells = 0;
     uint32_t* cnt = nullptr;         // partition: row counts [wave][leaf] of the level
     uint32_t* gcnt = nullptr;        // [level][group][leaf], cleared once per tree
+    uint32_t* totals = nullptr;      // [leaf] of the level, where the group counts are scanned
     uint32_t n_part_blocks = 0, n_groups_part = 0, part_rows = kPartLarge;   // rows per wave
     LevelPlan* plans = nullptr;   // [depth]
     SplitRec* splits = nullptr;   // [depth]
@@ -308,7 +309,7 @@ struct cbh_session {
     void release() {
         dfree(rows); dfree(cols); dfree(weight); dfree(target); dfree(approx); dfree(sstat);
         dfree(host_sample); dfree(leaf); dfree(idx); dfree(hist[0]); dfree(hist[1]); dfree(raw[0]); dfree(raw[1]); dfree(cnt);
-        dfree(gcnt); dfree(best_score);
+        dfree(gcnt); dfree(totals); dfree(best_score);
         dfree(best_bin); dfree(n_cand); dfree(one_hot); dfree(scales);
         dfree(leaf_sums); dfree(leaf_scaled); dfree(jump);
         dfree(out_dev);
@@ -430,6 +431,16 @@ FinishPlan level_finish(const cbh_session* s, uint32_t level) {
     return pl;
 }
 
+// Whether a level's group counts are scanned in a launch of their own.  Without it every workgroup of
+// compact reads all of them, which grows with the square of the rows (and with the leaves): the line
+// is the bytes so read that take as long as the launch.  Measured, us a tree of depth 8 over 4
+// features, every level scanned / none: 3M rows 573 / 568, 6M 909 / 919, 10M 1423 / 1447, 24M 2963 /
+// 3070, 60M 7662 / 8201, 120M 14933 / 17379; by this line 565, 906, 1425, 2980, 7675, 15010.
+constexpr uint64_t kScanBytes = 64ull << 20;
+bool scan_groups(const cbh_session* s, uint32_t level) {
+    return (uint64_t)s->n_part_blocks * s->n_groups_part * (2u << level) * sizeof(uint32_t) > kScanBytes;
+}
+
 int launch_zero(long long* p, size_t n, hipStream_t st) {
     zero_i64_kernel<<<grid_for(n, 256, 8192), 256, 0, st>>>(p, n);
     HIP_TRY(hipGetLastError());
@@ -458,6 +469,7 @@ int session_alloc(cbh_session* s) {
     CHECK(dalloc(&s->cnt, ((size_t)s->n_part_blocks * 4) << (s->depth - 1)));
     s->n_groups_part = part_groups(s->n_part_blocks);
     CHECK(dalloc(&s->gcnt, group_count_off(s->n_groups_part, s->depth - 1) + 2));
+    CHECK(dalloc(&s->totals, (size_t)1 << (s->depth - 1)));
     {   // one block for the per-tree results, sections 256-byte aligned
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         const size_t o_plans = up(sizeof(SplitRec) * s->depth);
@@ -2015,13 +2027,19 @@ int enqueue_tree(cbh_session* s) {
                                  s->pairwise ? nullptr : s->one_hot, s->F, parts, level, s->leaf, s->cnt, gcnt);
         HIP_TRY(hipGetLastError());
         if (!last) {
+            const bool scan = scan_groups(s, level);
+            if (scan) {
+                group_scan_kernel<<<2u << level, kScanThreads, 0, st>>>(gcnt, s->n_groups_part, 2u << level, s->totals);
+                HIP_TRY(hipGetLastError());
+            }
             // beside the index: the listed row's packed statistic, or both f64 score channels
             const int spw = s->packed || s->count ? 1 : s->tiled && s->sseq ? 2 : 0;
             const unsigned long long* sp = spw == 1 ? s->spack : spw == 2 ? (const unsigned long long*)s->sstat : nullptr;
             (spw == 1   ? (small ? compact_kernel<1, kPartSmall> : compact_kernel<1, kPartLarge>)
              : spw == 2 ? (small ? compact_kernel<2, kPartSmall> : compact_kernel<2, kPartLarge>)
                         : (small ? compact_kernel<0, kPartSmall> : compact_kernel<0, kPartLarge>))
-                <<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, s->n_groups_part, s->plans + level, s->idx, sp,
+                <<<NB, 256, 0, st>>>(s->leaf, n, level, s->cnt, gcnt, s->n_groups_part, scan ? s->totals : nullptr,
+                                     s->plans + level, s->idx, sp,
                                      spw ? s->sseq : nullptr);
             HIP_TRY(hipGetLastError());
         }

@@ -1251,6 +1251,40 @@ def test_deep_trees_over_few_rows(n, F, borders, depth):
     _close(leaves, exp["leaf_values"])
 
 
+@pytest.mark.parametrize("n,F,depth", [(6_100_003, 2, 8), (12_000_001, 2, 8), (70_000_001, 1, 3)])
+def test_partition_with_scanned_group_counts(n, F, depth):
+    """Many rows in many leaves: the partition's group counts are scanned in a launch of their own (at
+    6.1M rows at the deepest level only, at 12M at the three deepest, at 70M at every level and in two
+    rounds of 1024 groups), those of the other levels are summed by every workgroup.  Every level's
+    histogram equals the sums over the rows of its leaves, cell by cell, to the fixed-point step."""
+    B = 23
+    g = np.random.default_rng(n)
+    bins = g.integers(0, B, (F, n), dtype=np.uint8)
+    bins[-1] = np.minimum(bins[-1], bins[0])   # leaves of unlike sizes
+    y = bins[0] * 0.25 - (bins[-1] % 5) + g.standard_normal(n)
+    be = cb.HipBackend()
+    assert be.begin_device_training("RMSE", depth, True, 1, "Cosine", bins, None, n, F, B, 0.1, 3.0,
+                                    real_folds=np.full(F, B, np.uint32))
+    try:
+        be.capture_hists()
+        t = be.grow_tree_on_device(target=y, want_leaf_of=True)
+        hists = [be.level_hist(l, F, B) for l in range(depth)]
+    finally:
+        be.end_device_training()
+    leaf = np.zeros(n, np.int64)
+    for level, (f, b, _) in enumerate(t["splits"]):
+        for ft in range(F):
+            cell = leaf * B + bins[ft]
+            cnt = np.bincount(cell, minlength=B << level).reshape(-1, B)
+            der = np.bincount(cell, weights=y, minlength=B << level).reshape(-1, B)
+            assert np.array_equal(hists[level][:, ft, :, 1], cnt)
+            # a row is rounded to 2^-61 of the channel's sum, the f64 sums here to n 2^-53 of it; the
+            # counts have told a misplaced row by then
+            assert np.abs(hists[level][:, ft, :, 0] - der).max() <= np.abs(y).sum() * n * 2.0**-53
+        leaf |= (bins[f] > b).astype(np.int64) << level
+    assert np.array_equal(leaf, t["leaf_of"])
+
+
 # ------------------------------------------------------------------ a tree that ends in an error
 @pytest.mark.parametrize("loss,n,F,B,K,depth", [
     ("RMSE", 3_000, 12, 33, 1, 4),           # one reader a raw row
