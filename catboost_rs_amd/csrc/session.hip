@@ -754,29 +754,43 @@ int plan_pkk(cbh_session* s, const std::string& v) {
     return CBH_OK;
 }
 
-// The narrow tiles against the 32-feature tiles (K == 1): they save about 0.12 B + 10 us of
-// flushing and latency a level and read rows and statistics four times as often, 0.195 us a level
-// per million (row, feature).  Measured, us a tree of depth 6, narrow against 32-feature: 255
-// bins 1M x 50 415 / 603, 2M x 100 824 / 828, 4M x 50 935 / 953, 1M x 200 820 / 799, 4M x 200 2386 /
-// 1637; 33 bins 1M x 50 345 / 371, 4M x 50 886 / 750.  Below 2^16 rows the 32-feature tiles are
-// not planned.
-bool narrow_pays(uint64_t n, uint32_t F, uint32_t B) {
-    return n < (1ull << 16) || (double)n * F <= 1e6 * (51.0 + 0.615 * B);
-}
-
-// Few rows in many segments: a workgroup pays the latency and the flush of its LDS image for each
-// segment it meets, and many features leave the narrow tiles few ranges to spread the last level's
-// segments over, where the 32-feature tiles have four times as many.  load = segments a range x the
-// image's cells, against the rows (whose atomics the narrow tiles do faster).  Measured, us a
-// tree, these tiles against the others: 3000 x 1000 x 129 bins of depth 8 (load 8256) 1628 / 1126,
-// 3000 x 1000 x 255 of depth 6 (4080) 656 / 639, 5000 x 500 x 128, 6 channels, depth 7 (6144) 1379 /
-// 1090, 100k x 1000 x 129 of depth 8 (8256) 1638 / 1513; below the line 20k x 1000 x 65, 4
-// channels, depth 7 (4160) 848 / 1025, 3000 x 2000 x 33, 3 channels, depth 7 (3168) 684 / 736,
-// 60k x 300 x 255 of depth 8 (5440) 992 / 1002, 500k x 300 x 255 of depth 8 (10880) 1377 / 1457.
-bool narrow_spreads(const cbh_session* s) {
+// Cells a workgroup of the narrow tiles flushes at the last level: the segments it meets (a few row
+// ranges over many features leave each many) x the cells of its image a feature.
+double narrow_load(const cbh_session* s) {
     const uint32_t nt = (s->W + kNtWords - 1) / kNtWords, segs = s->depth >= 2 ? 1u << (s->depth - 2) : 1u;
     const uint32_t G = std::max<uint32_t>(1, (uint32_t)s->cus / nt), C = s->pairwise ? 1u : (uint32_t)s->C;
-    return (double)segs / G * s->B * C <= 3500.0 + (double)s->n / 25.0;
+    return (double)segs / G * s->B * C;
+}
+
+// Whether the narrow tiles are the faster ones: against the 32-feature tiles from 2^16 rows (2^20 with
+// pairs) at K = 1, else against the generic fill.
+//
+// Against the 32-feature tiles they save about 0.12 B + 10 us of flushing and latency a level and
+// read rows and statistics four times as often, 0.195 us a level per million (row, feature); the more
+// segments a workgroup meets, the less they save.  Measured, us a tree of depth 6, narrow /
+// 32-feature: 255 bins 1M x 50 413 / 596, x 170 762 / 813, x 200 866 / 807, 4M x 45 948 / 962, x 50
+// 991 / 977; 129 bins 1M x 110 532 / 587, x 200 795 / 678, 300k x 400 580 / 599, 200k x 600 648 / 634; 65 bins
+// 2M x 40 490 / 508, 1M x 90 462 / 440; 33 bins 1M x 60 355 / 381, x 70 394 / 380; deeper: 70k x 1000 x
+// 255, depth 7 1323 / 1450, depth 8 2327 / 2420, 200k x 600 x 255, depth 8 1754 / 1832, 100k x 1000 x
+// 129, depth 8 1484 / 1434, 100k x 1500 x 255 1336 / 1235.  From 2^22 rows few segments are met and the
+// line is a little higher: 8M x 25 x 255, sampled 1416 / 1402, unsampled (the count-packed fill instead,
+// whose rows are rounded coarser) 1376 / 1312, 8M x 16 x 129 1163 / 1137, 5M x 20 x 255 858 / 894.
+//
+// Against the generic fill they lose where few rows meet many segments: a workgroup pays the latency
+// and the flush of its image for each.  Measured, narrow / generic: K = 1 3000 x 1000 x 129, depth 8 (load
+// 8256) 1143 / 1043, depth 7 (4128) 650 / 632, 30k x 500 x 255, depth 8 (8160) 1233 / 1191, 60k x 1000 x
+// 255, depth 7 (8160) 1289 / 1228; 60k x 300 x 255, depth 8 (5440) 941 / 961, 10k x 400 x 129, depth 8 (3302)
+// 629 / 652.  K > 1, whose generic fill has the more to flush: 8000 x 1000 x 33, 4 channels, depth 8
+// (4224) 852 / 819, 5000 x 500 x 128, 6, depth 7 (6144) 1016 / 992, 3000 x 2000 x 33, 3, depth 7 (3168)
+// 677 / 640, 30k x 2000 x 17, 8, depth 8 (8704) 1815 / 1622; 50k x 500 x 128, 6, depth 7 (6144) 1120 /
+// 1215, 30k x 1000 x 65, 4, depth 8 (8320) 1467 / 1540, 20k x 1000 x 65, 4, depth 7 (4160) 836 / 940.
+bool narrow_pays(const cbh_session* s) {
+    const double n = (double)s->n, nf = n * s->F, load = narrow_load(s);
+    if (s->K > 1) return load <= 2500.0 + n / 5.0;
+    if (s->n < (1ull << 16)) return load <= 3500.0 + n / 25.0;
+    if (s->ranking && s->n < (1ull << 20)) return nf <= 1e6 * (51.0 + 0.615 * s->B) && load <= 3500.0 + n / 25.0;
+    if (s->n >= (1ull << 22)) return nf <= 1e6 * (51.0 + 0.615 * s->B);
+    return nf <= 1e6 * (46.0 + 0.6 * s->B) * (1.0 - load / 30000.0);
 }
 
 // Row ranges G of the narrow-tile exact fill at a level of n_seg segments.  A launch takes n / G
@@ -825,8 +839,8 @@ int plan_narrow_fill(cbh_session* s, bool& taken) {
     return CBH_OK;
 }
 
-// Fill plan.  The default: K == 1 the narrow-tile exact fill where it pays (narrow_pays,
-// narrow_spreads), else with integer score weights from 2^22 rows the count-packed fill, else from
+// Fill plan.  The default: K == 1 the narrow-tile exact fill where it pays (narrow_pays), else
+// with integer score weights from 2^22 rows the count-packed fill, else from
 // 2^16 rows (2^20 with pairs) the tiled exact fill (which visits every bin: its lanes add to
 // distinct features, so a dominant bin does not serialize them); K > 1 from 500000 rows the packed
 // multi-channel fill, else the narrow-tile fill; otherwise the generic fill.  CBH_FILL (a measurement and
@@ -840,11 +854,11 @@ int plan_fill_mode(cbh_session* s) {
     bool narrow_taken = false;
     if (s->K > 1) {
         if (v.empty() || v == "packed") CHECK(plan_pkk(s, v));
-        if (!s->pkk && v.empty() && narrow_spreads(s)) CHECK(plan_narrow_fill(s, narrow_taken));
+        if (!s->pkk && v.empty() && narrow_pays(s)) CHECK(plan_narrow_fill(s, narrow_taken));
         return CBH_OK;
     }
     if (v == "generic") return CBH_OK;
-    if (v.empty() && narrow_pays(s->n, s->F, s->B) && narrow_spreads(s)) {
+    if (v.empty() && narrow_pays(s)) {
         CHECK(plan_narrow_fill(s, narrow_taken));
         if (narrow_taken) return CBH_OK;
     }

@@ -1251,6 +1251,29 @@ def test_deep_trees_over_few_rows(n, F, borders, depth):
     _close(leaves, exp["leaf_values"])
 
 
+@pytest.mark.parametrize("n,F,B,K,depth", [(66_001, 600, 255, 1, 8), (30_001, 1_000, 65, 3, 8)])
+def test_deep_trees_over_many_features_equal_the_generic_fill(n, F, B, K, depth, monkeypatch):
+    """Deep trees whose narrow-tile workgroups meet many segments each (21 and 32 at the last level):
+    the sums are exact integers at the same scales, so two trees are bit-equal to the generic fill's."""
+    g = np.random.default_rng(n)
+    bins = g.integers(0, B, (F, n), dtype=np.uint8)
+    y = g.integers(0, K, n).astype(np.float64) if K > 1 else bins[3] * 0.1 + g.standard_normal(n)
+    out = []
+    for fill in ("", "generic"):
+        monkeypatch.setenv("CBH_FILL", fill)
+        tr = cb.Trainer(bins, B, y, loss="MultiClass" if K > 1 else "RMSE", depth=depth, approx_dim=K,
+                        leaf_method="Newton" if K > 1 else "Gradient", bootstrap_type="No", learning_rate=0.3,
+                        real_folds=np.full(F, B, np.uint32))
+        try:
+            assert tr.stats()["fill_mode"] == (0 if fill else 2)
+            splits, leaves = tr.fit(2)
+            out.append((splits, leaves, tr.approx()))
+        finally:
+            tr.close()
+    for x, z in zip(*out):
+        assert np.array_equal(x, z)
+
+
 @pytest.mark.parametrize("n,F,depth", [(6_100_003, 2, 8), (12_000_001, 2, 8), (70_000_001, 1, 3)])
 def test_partition_with_scanned_group_counts(n, F, depth):
     """Many rows in many leaves: the partition's group counts are scanned in a launch of their own (at
