@@ -74,6 +74,22 @@ def _profile_facts(config, n, F, kernel):
     return round((float(m.group(1)) + float(m.group(2))) * 1e9), (lim.group(1).strip() if lim else None)
 
 
+def _fill_kernel(st):
+    """(kernel, what it does) of a session's fill, by its stats."""
+    bits = st["fill_pack_bits"]
+    narrow = st["fill_mode"] == 2 and st["fill_tile"] == 8
+    return {0: ("fill_kernel", f"generic {st['fill_tile']}-feature tiles (one 64-bit atomic per channel, full fixed-point scale)"),
+            1: ("fill_packed_kernel", f"packed 64-feature tiles ({bits}-bit rows)"),
+            2: ("fill_narrow_kernel" if narrow else "fill_exact_kernel",
+                f"tiled exact {st['fill_tile']}-feature tiles (one 64-bit atomic per channel, full fixed-point scale)"),
+            3: ("fill_pkk_kernel", f"packed multi-channel 32-feature tiles (two channels per word, {bits}-bit rows)"),
+            4: ("fill_pks_kernel", f"packed multi-channel 32-feature tiles over sparse entries (a row per 16-lane DPP "
+                                   f"row, two channels per word, {bits}-bit rows)"),
+            5: ("fill_packed_kernel",
+                "count-packed 64-feature tiles (der at >= 2^-30 and the integer weight in one 64-bit atomic)"),
+            }[st["fill_mode"]]
+
+
 def _lds_rates():
     probe = os.path.join(ROOT, "catboost_rs_amd", "lds_atomic_rate")
     if not os.path.exists(probe):
@@ -396,12 +412,7 @@ def main():
             log(f"cpu: {P['iterations']} trees in {one:.1f}s on 1 thread")
 
     traffic, limiter = None, None   # (set below from the committed profile)
-    fill_kernel = {0: "fill_kernel", 1: "fill_packed_kernel", 2: "fill_exact_kernel",
-                   3: "fill_pkk_kernel", 4: "fill_pks_kernel", 5: "fill_packed_kernel"}[st["fill_mode"]]
-    # the exact fill's tiles: 8 features where the session's rule takes them (narrow_pays), else 32
-    narrow = st["fill_mode"] == 2 and (P["loss"] == "MultiClass" or n < 1 << 16 or n * F <= 1e6 * (51 + 0.615 * n_bins))
-    if narrow:
-        fill_kernel = "fill_narrow_kernel"
+    fill_kernel, fill_text = _fill_kernel(st)
     traffic, limiter = _profile_facts(args.config, n, F, fill_kernel)
     names = {1: "config1: RMSE, no bootstrap, depth 6, 128 borders",
              2: ("config2: Logloss, Bayesian bootstrap T=1, depth 6, 254 GreedyLogSum borders selected on the "
@@ -433,13 +444,7 @@ def main():
                   if st["fill_mode"] == 5 else
                   f"u8 bins; int64 sums of rows rounded to {st['fill_pack_bits']}-bit fields of the tree's "
                   f"largest row (coarser than the reference's 2^-30); f64 scores"),
-        "fill": {0: "generic 32-feature tiles (one 64-bit atomic per channel, full fixed-point scale)", 1: f"packed 64-feature tiles ({st['fill_pack_bits']}-bit rows)",
-                 2: f"tiled exact {8 if narrow else 32}-feature tiles (one 64-bit atomic per channel, full fixed-point scale)",
-                 3: f"packed multi-channel 32-feature tiles (two channels per word, {st['fill_pack_bits']}-bit rows)",
-                 4: f"packed multi-channel 32-feature tiles over sparse entries (a row per 16-lane DPP row, "
-                    f"two channels per word, {st['fill_pack_bits']}-bit rows)",
-                 5: "count-packed 64-feature tiles (der at >= 2^-30 and the integer weight in one 64-bit atomic)",
-                 }[st["fill_mode"]],
+        "fill": fill_text,
         "data": f"synthetic (seeded; datagen.config{args.config}{'_raw' if raw else ''})",
         "config": {"workload": names[args.config] + (f" (bootstrap overridden: {args.bootstrap})"
                                                      if args.bootstrap else ""),

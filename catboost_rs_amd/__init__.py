@@ -128,7 +128,7 @@ EXPORTS = ["cbh_session_begin", "cbh_session_begin_u8", "cbh_session_grow",
            "cbt_read_approx", "cbt_stats", "cbt_reset_stats", "cbt_bias", "cbt_close", "cbh_session_set_profile",
            "cbt_set_profile", "cbh_session_set_ctr", "cbt_set_ctr", "cbh_session_read_ctr_bins",
            "cbt_open_ctr", "cbh_hist_build_noalloc", "cbh_session_capture_hists", "cbh_session_level_hist",
-           "cbh_columns_from_rows"]
+           "cbh_columns_from_rows", "cbh_session_fill_tile", "cbt_fill_tile"]
 
 _lib = None
 
@@ -176,6 +176,8 @@ def load(path: str = LIB_PATH):
     L.cbt_step.argtypes = [P, P, P, P, P]
     L.cbt_read_approx.argtypes = [P, P]
     L.cbt_stats.argtypes = [P, C.POINTER(Stats)]
+    L.cbh_session_fill_tile.argtypes = L.cbt_fill_tile.argtypes = [P]
+    L.cbh_session_fill_tile.restype = L.cbt_fill_tile.restype = C.c_uint32
     L.cbt_reset_stats.argtypes = [P]
     L.cbt_reset_stats.restype = None
     L.cbt_bias.argtypes = [P]
@@ -594,7 +596,7 @@ class HipBackend:
     def stats(self):
         st = Stats()
         _check(load().cbh_session_stats(self._s, C.byref(st)))
-        return st.as_dict()
+        return dict(st.as_dict(), fill_tile=int(load().cbh_session_fill_tile(self._s)))
 
     def end_device_training(self):
         if self._s:
@@ -713,7 +715,7 @@ class Trainer:
     def stats(self):
         st = Stats()
         _check(load().cbt_stats(self._h, C.byref(st)))
-        return st.as_dict()
+        return dict(st.as_dict(), fill_tile=int(load().cbt_fill_tile(self._h)))
 
     def reset_stats(self):
         load().cbt_reset_stats(self._h)

@@ -287,6 +287,8 @@ int cbt_stats(const cbt_trainer* t, cbh_stats* out) {
     return cbh_session_stats(t->s, out);
 }
 
+uint32_t cbt_fill_tile(const cbt_trainer* t) { return t ? cbh_session_fill_tile(t->s) : 0; }
+
 void cbt_reset_stats(cbt_trainer* t) {
     if (t) cbh_session_reset_stats(t->s);
 }

@@ -2478,6 +2478,14 @@ int cbh_session_stats(const cbh_session* s, cbh_stats* out) {
     return CBH_OK;
 }
 
+uint32_t cbh_session_fill_tile(const cbh_session* s) {
+    if (!s) return 0;
+    if (s->narrow) return 4u * kNtWords;
+    if (s->packed || s->count) return 4u * kPackTileWords;
+    if (s->tiled) return 4u * kExTileWords;
+    return s->pkk ? 32u : 4u * s->tiles.tw;
+}
+
 void cbh_session_reset_stats(cbh_session* s) {
     if (!s) return;
     s->stats = cbh_stats{};

@@ -239,6 +239,11 @@ typedef struct {
 
 int cbh_session_stats(const cbh_session* s, cbh_stats* out);
 
+/* Features of a full tile of the session's fill (0 for a null session): tells the two tiled exact
+ * fills (fill_mode 2) apart, 8 or 32; 64 with fill_modes 1 and 5, 32 with 3 and 4, and with the
+ * generic fill as many as its LDS budget takes. */
+uint32_t cbh_session_fill_tile(const cbh_session* s);
+
 /* CTR columns of a session (DeviceCtrConfig, runtime.rs:1160-1230, for simple projections and
  * one learning permutation).  The LAST n_ctr features of the session are CTR columns built
  * under the structure (learning) permutation (cbh_ctr_columns).  They are scored after the
