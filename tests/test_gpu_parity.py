@@ -1199,7 +1199,7 @@ def test_narrow_tile_fill_histograms(n, F, B, K, loss):
 def test_apply_oblivious_paths_match_reference(n, F, T, D, K):
     """Every route of a prediction call: a small table in one upload, a large one in pinned chunks
     (over 12 MB; a last chunk that is no multiple of 64), one too wide for chunks and leaf values
-    past 8 MB from the caller's memory, features staged in LDS or, above 512 of
+    past 512 KiB from the caller's memory, features staged in LDS or, above 512 of
     them, read through the caches, trees of one to three groups of eight splits, absent features
     and NaN.  The sums are in tree order, so the result is bit-equal to the same order in f64.
     Two host threads predicting at once get the same."""
