@@ -196,10 +196,13 @@ int launch_k(uint32_t K, const float* x, uint64_t ld, uint64_t n, const Model& M
 }
 bool has_variant(uint32_t K) { return (K >= 1 && K <= 8) || K == 10 || K == 12 || K == 16; }
 
-// A call's buffers: a device block, a pinned block and a stream.  Allocating and freeing them per
+// A call's buffers: a device block, a pinned block and its streams.  Allocating and freeing them per
 // call (eight of each, each free a device synchronization) was most of a small call's time, so
-// up to kKeep idle workspaces are kept, each a call's own while it runs (any number of threads);
-// one that has grown past kKeepBytes is freed with its call, as are those above kKeep.
+// up to kKeep idle workspaces are kept, each a call's own while it runs (any number of threads).
+// A workspace whose block has grown past kKeepBytes loses the block with its call and keeps its streams
+// and the rest, as does one whose blocks would take the kept ones past kKeepTotal: freed whole and
+// made anew by each call, streams included, 10M x 1 (an 80 MB result) took 17.7 ms, 10.3 this way.  The
+// kept blocks go when an allocation fails.
 struct Workspace {
     int device = -1;
     hipStream_t stream = nullptr, copy = nullptr;   // copy: a large table's uploads, beside the kernels
@@ -209,41 +212,29 @@ struct Workspace {
     hipEvent_t ev[6] = {};   // of the three chunk buffers: uploaded, then read by the kernel
 
     void release() {
-        if (dev) (void)hipFree(dev);
-        if (pin) (void)hipHostFree(pin);
+        drop_dev();
+        drop_pin();
         for (auto& e : ev) {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
         }
         if (stream) (void)hipStreamDestroy(stream);
         if (copy) (void)hipStreamDestroy(copy);
-        copy = nullptr;
-        dev = pin = nullptr;
-        dev_cap = pin_cap = 0;
-        stream = nullptr;
+        copy = stream = nullptr;
     }
-    int grow(size_t need_dev, size_t need_pin) {
-        if (!stream) APPLY_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        if (need_dev > dev_cap) {
-            if (dev) (void)hipFree(dev);
-            dev = nullptr;
-            dev_cap = 0;
-            need_dev = std::max<size_t>(need_dev, 1 << 20);
-            APPLY_TRY(hipMalloc((void**)&dev, need_dev));
-            dev_cap = need_dev;
-        }
-        if (need_pin > pin_cap) {
-            if (pin) (void)hipHostFree(pin);
-            pin = nullptr;
-            pin_cap = 0;
-            need_pin = std::max<size_t>(need_pin, 1 << 20);
-            APPLY_TRY(hipHostMalloc((void**)&pin, need_pin, hipHostMallocDefault));
-            pin_cap = need_pin;
-        }
-        return CBH_OK;
+    void drop_dev() {
+        if (dev) (void)hipFree(dev);
+        dev = nullptr;
+        dev_cap = 0;
     }
+    void drop_pin() {
+        if (pin) (void)hipHostFree(pin);
+        pin = nullptr;
+        pin_cap = 0;
+    }
+    int grow(size_t need_dev, size_t need_pin);
 };
-constexpr size_t kKeep = 2, kKeepBytes = (size_t)64 << 20;
+constexpr size_t kKeep = 16, kKeepBytes = (size_t)64 << 20, kKeepTotal = (size_t)256 << 20;
 std::mutex g_ws_mu;
 std::vector<Workspace>& idle_workspaces() {
     static std::vector<Workspace>* v = [] {   // (never destroyed: no frees after the runtime has gone)
@@ -253,13 +244,45 @@ std::vector<Workspace>& idle_workspaces() {
     }();
     return *v;
 }
+// The idle workspaces' blocks are given back (to a call that found no memory).
+void drop_idle_blocks() {
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    for (Workspace& w : idle_workspaces()) {
+        w.drop_dev();
+        w.drop_pin();
+    }
+}
+int Workspace::grow(size_t need_dev, size_t need_pin) {
+    if (!stream) APPLY_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    if (need_dev > dev_cap) {
+        drop_dev();
+        need_dev = std::max<size_t>(need_dev, 1 << 20);
+        if (hipMalloc((void**)&dev, need_dev) != hipSuccess) {
+            (void)hipGetLastError();
+            drop_idle_blocks();
+            APPLY_TRY(hipMalloc((void**)&dev, need_dev));
+        }
+        dev_cap = need_dev;
+    }
+    if (need_pin > pin_cap) {
+        drop_pin();
+        need_pin = std::max<size_t>(need_pin, 1 << 20);
+        if (hipHostMalloc((void**)&pin, need_pin, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            drop_idle_blocks();
+            APPLY_TRY(hipHostMalloc((void**)&pin, need_pin, hipHostMallocDefault));
+        }
+        pin_cap = need_pin;
+    }
+    return CBH_OK;
+}
 struct Lease {
     Workspace ws;
     bool ok = false;   // the call went through: nothing is running on the stream
     explicit Lease(int device) {
         std::lock_guard<std::mutex> lock(g_ws_mu);
         auto& idle = idle_workspaces();
-        for (size_t k = 0; k < idle.size(); ++k)
+        for (size_t k = idle.size(); k-- > 0;)   // the one given back last
             if (idle[k].device == device) {
                 ws = idle[k];
                 idle.erase(idle.begin() + (long)k);
@@ -270,10 +293,19 @@ struct Lease {
     ~Lease() {
         if (!ok && ws.copy) (void)hipStreamSynchronize(ws.copy);
         if (!ok && ws.stream) (void)hipStreamSynchronize(ws.stream);
-        if (ok && ws.dev_cap <= kKeepBytes && ws.pin_cap <= kKeepBytes) {
+        if (ok) {
+            if (ws.dev_cap > kKeepBytes) ws.drop_dev();
+            if (ws.pin_cap > kKeepBytes) ws.drop_pin();
             std::lock_guard<std::mutex> lock(g_ws_mu);
-            if (idle_workspaces().size() < kKeep) {
-                idle_workspaces().push_back(ws);
+            auto& idle = idle_workspaces();
+            if (idle.size() < kKeep) {
+                size_t kept = ws.dev_cap + ws.pin_cap;
+                for (const Workspace& w : idle) kept += w.dev_cap + w.pin_cap;
+                if (kept > kKeepTotal) {
+                    ws.drop_dev();
+                    ws.drop_pin();
+                }
+                idle.push_back(ws);
                 return;
             }
         }

@@ -119,3 +119,23 @@ def test_predictions_with_leaf_values_either_side_of_the_pinned_size(stumps):
         exp += lv[lo[t] + leaf]
     got = cb.apply_oblivious(x, sf, sb, so, lv, lo, approx_dim=1)
     assert np.array_equal(np.asarray(got).reshape(-1), exp)
+
+
+def test_predictions_past_the_kept_sizes():
+    """A result of 72 MB loses its device block with the call, the calls after it and beside it (three host
+    threads, small and large) start from what is kept.  Equal bit by bit to the same sums on the host."""
+    from concurrent.futures import ThreadPoolExecutor
+    g = np.random.default_rng(9)
+    sf, sb = np.zeros(2, np.uint32), np.array([-0.5, 0.75])
+    so, lo, lv = np.array([0, 1, 2], np.uint32), np.array([0, 2, 4], np.uint32), np.array([0.1, 0.7, -0.3, 1.1])
+    big = g.standard_normal((1, 9_000_001), dtype=np.float32)
+
+    def one(n):
+        x = big[:, :n]
+        exp = np.where(x[0] > -0.5, 0.7, 0.1) + np.where(x[0] > 0.75, 1.1, -0.3)
+        got = np.asarray(cb.apply_oblivious(np.ascontiguousarray(x), sf, sb, so, lv, lo, approx_dim=1)).reshape(-1)
+        return np.array_equal(got, exp)
+
+    assert one(9_000_001) and one(100)
+    with ThreadPoolExecutor(3) as ex:
+        assert all(ex.map(one, [9_000_001, 63, 4_000_000, 1, 8_500_000, 70_000] * 2))
