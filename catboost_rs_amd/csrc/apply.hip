@@ -198,11 +198,12 @@ bool has_variant(uint32_t K) { return (K >= 1 && K <= 8) || K == 10 || K == 12 |
 
 // A call's buffers: a device block, a pinned block and its streams.  Allocating and freeing them per
 // call (eight of each, each free a device synchronization) was most of a small call's time, so
-// up to kKeep idle workspaces are kept, each a call's own while it runs (any number of threads).
-// A workspace whose block has grown past kKeepBytes loses the block with its call and keeps its streams
-// and the rest, as does one whose blocks would take the kept ones past kKeepTotal: freed whole and
-// made anew by each call, streams included, 10M x 1 (an 80 MB result) took 17.7 ms, 10.3 this way.  The
-// kept blocks go when an allocation fails.
+// up to kKeep idle workspaces are kept, each a call's own while it runs (any number of threads); one
+// more is freed with its call.  A block that has grown past kKeepBytes goes with its call, the streams
+// and the rest stay: freed whole and made anew by each call, 10M x 1 (an 80 MB result) took 17.7 ms, 10.3
+// this way.  The kept blocks go when an allocation fails.  Two are kept because streams that stay
+// share the few hardware queues as they were dealt: with 16 kept, calls of four threads on 50k x 50
+// took 230 to 320 us each from run to run, 235 with two.
 struct Workspace {
     int device = -1;
     hipStream_t stream = nullptr, copy = nullptr;   // copy: a large table's uploads, beside the kernels
@@ -234,7 +235,7 @@ struct Workspace {
     }
     int grow(size_t need_dev, size_t need_pin);
 };
-constexpr size_t kKeep = 16, kKeepBytes = (size_t)64 << 20, kKeepTotal = (size_t)256 << 20;
+constexpr size_t kKeep = 2, kKeepBytes = (size_t)64 << 20;
 std::mutex g_ws_mu;
 std::vector<Workspace>& idle_workspaces() {
     static std::vector<Workspace>* v = [] {   // (never destroyed: no frees after the runtime has gone)
@@ -299,12 +300,6 @@ struct Lease {
             std::lock_guard<std::mutex> lock(g_ws_mu);
             auto& idle = idle_workspaces();
             if (idle.size() < kKeep) {
-                size_t kept = ws.dev_cap + ws.pin_cap;
-                for (const Workspace& w : idle) kept += w.dev_cap + w.pin_cap;
-                if (kept > kKeepTotal) {
-                    ws.drop_dev();
-                    ws.drop_pin();
-                }
                 idle.push_back(ws);
                 return;
             }
