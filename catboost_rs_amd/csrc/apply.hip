@@ -61,13 +61,24 @@ constexpr uint32_t kApplyObj = 64, kApplyWaves = 8, kApplyTrees = 32;
 constexpr uint32_t kNoLeaf = 0xFFFFFFFFu;
 template <int K, bool kLds>
 __global__ __launch_bounds__(kApplyObj * kApplyWaves) void apply_oblivious_kernel(
-    const float* __restrict__ x /* value of feature f, object i at x[f * ld + i] */, uint64_t ld, uint64_t n, Model M,
+    const float* __restrict__ x /* value of feature f, object i at x[f * ld + i] */, uint64_t ld, uint64_t n,
+    uint32_t chunk /* 0, or a multiple of kApplyObj: the table comes in chunks of so many objects, */,
+    uint64_t cstride /* chunk c at x + c cstride, its values [F][objects of it] */, Model M,
     double* __restrict__ out /* [K][ldo] */, uint64_t ldo) {
     __shared__ uint32_t leaves[2][kApplyTrees][kApplyObj];
     extern __shared__ float xs[];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kApplyObj), lane = threadIdx.x % kApplyObj;
     const uint64_t obj = (uint64_t)blockIdx.x * kApplyObj + lane;
-    const uint64_t oc = obj < n ? obj : n - 1;
+    uint64_t oc = obj, end = n;
+    if (chunk) {   // (a workgroup's objects lie in one chunk)
+        const uint32_t c = blockIdx.x / (chunk / kApplyObj);
+        const uint64_t o0 = (uint64_t)c * chunk;
+        x += c * cstride;
+        oc = obj - o0;
+        end = n - o0 < chunk ? n - o0 : chunk;
+        ld = end;
+    }
+    if (oc >= end) oc = end - 1;
     if (kLds) {
 #pragma unroll 4
         for (uint32_t f = wave; f < M.F; f += kApplyWaves) xs[f * kApplyObj + lane] = x[(size_t)f * ld + oc];
@@ -163,32 +174,40 @@ __global__ __launch_bounds__(kApplyObj * kApplyWaves) void apply_oblivious_kerne
 constexpr size_t kApplyLdsMax = 128 * 1024;
 constexpr uint64_t kMaxBlocks = (uint64_t)1 << 22;
 
+struct Table {   // on the device: one block of leading dimension ld, or chunks (the kernel's arguments)
+    const float* x;
+    uint64_t ld;
+    uint32_t chunk;
+    uint64_t cstride;
+};
+
 template <int K>
-int launch(const float* x, uint64_t ld, uint64_t n, const Model& M, double* out, uint64_t ldo, hipStream_t st) {
+int launch(const Table& t, uint64_t n, const Model& M, double* out, uint64_t ldo, hipStream_t st) {
     const size_t lds = (size_t)M.F * kApplyObj * sizeof(float);
     const uint64_t blocks = (n + kApplyObj - 1) / kApplyObj;
-    if (blocks > kMaxBlocks) {   // (a launch holds fewer than 2^32 threads)
+    if (blocks > kMaxBlocks) {   // (a launch holds fewer than 2^32 threads; chunks are far smaller)
         const uint64_t n0 = kMaxBlocks * kApplyObj;
-        const int rc = launch<K>(x, ld, n0, M, out, ldo, st);
-        return rc != CBH_OK ? rc : launch<K>(x + n0, ld, n - n0, M, out + n0, ldo, st);
+        const int rc = launch<K>(t, n0, M, out, ldo, st);
+        return rc != CBH_OK ? rc : launch<K>(Table{t.x + n0, t.ld, 0, 0}, n - n0, M, out + n0, ldo, st);
     }
     const unsigned grid = (unsigned)blocks;
     if (lds <= kApplyLdsMax) {
         if (lds > 32 * 1024)
             APPLY_TRY(hipFuncSetAttribute((const void*)apply_oblivious_kernel<K, true>,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kApplyLdsMax));
-        apply_oblivious_kernel<K, true><<<grid, kApplyObj * kApplyWaves, lds, st>>>(x, ld, n, M, out, ldo);
+        apply_oblivious_kernel<K, true><<<grid, kApplyObj * kApplyWaves, lds, st>>>(t.x, t.ld, n, t.chunk, t.cstride, M,
+                                                                                    out, ldo);
     } else {
-        apply_oblivious_kernel<K, false><<<grid, kApplyObj * kApplyWaves, 0, st>>>(x, ld, n, M, out, ldo);
+        apply_oblivious_kernel<K, false><<<grid, kApplyObj * kApplyWaves, 0, st>>>(t.x, t.ld, n, t.chunk, t.cstride, M,
+                                                                                   out, ldo);
     }
     APPLY_TRY(hipGetLastError());
     return CBH_OK;
 }
 
-int launch_k(uint32_t K, const float* x, uint64_t ld, uint64_t n, const Model& M, double* out, uint64_t ldo,
-             hipStream_t st) {
+int launch_k(uint32_t K, const Table& t, uint64_t n, const Model& M, double* out, uint64_t ldo, hipStream_t st) {
     switch (K) {
-#define CASE(k) case k: return launch<k>(x, ld, n, M, out, ldo, st);
+#define CASE(k) case k: return launch<k>(t, n, M, out, ldo, st);
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(10) CASE(12) CASE(16)
 #undef CASE
         default: return cbh_internal_fail(CBH_ERR_UNSUPPORTED, "approx_dim " + std::to_string(K) + " has no apply variant");
@@ -330,10 +349,43 @@ constexpr size_t kChunkBytes = (size_t)6 << 20;   // of a table in pinned chunks
 // A large table in chunks of objects: the threads copy a chunk's runs of every feature into one of
 // three pinned buffers, which goes to its device buffer and through the kernel while the next one
 // fills (the runtime's own path for pageable memory copies with one thread: 200 MB in 7 ms).
+//
+// A kernel takes a group of chunks: one where the model takes less time than a chunk's upload (135 us),
+// three groups in flight, else as many as fill the CUs, two groups in flight.  A chunk of 100 features is
+// 245 workgroups, one a CU and bound by the latency of its trees (0.2 us each up to 8 splits): a
+// launch a chunk fell behind the uploads at large models, and behind one launch over the whole
+// table.  500k x 100, a launch a chunk / a group / one launch after the upload: 500 trees 4.6 / - / 9.5 ms,
+// 1000 6.9 / 4.9 / 11.0, 5000 30.3 / 16.6 / 23.8; 300k x 300, 3000 trees of depth 8 38.5 / 13.9 / 27.0.
+// (The three buffers' kernels on streams of their own gave the same where the streams had hardware
+// queues of their own, and nothing where they had not.)
+struct ChunkPlan {
+    uint64_t chunk, n_chunks;   // objects, a multiple of kApplyObj
+    uint32_t group, ring;       // chunks a launch, groups in flight
+    size_t cbytes;              // of a chunk's buffer
+};
+constexpr uint64_t kGroupWork = 800;    // trees and groups of 8 splits past which a launch takes several chunks
+constexpr uint32_t kGroupMax = 10;      // (60 MB)
+ChunkPlan plan_chunks(uint64_t n, uint32_t F, uint32_t n_trees, uint32_t n_splits, uint32_t cus) {
+    ChunkPlan p{};
+    p.chunk = kChunkBytes / (sizeof(float) * F) / kApplyObj * kApplyObj;
+    p.n_chunks = (n + p.chunk - 1) / p.chunk;
+    p.cbytes = align256(sizeof(float) * p.chunk * F);
+    p.group = 1;
+    p.ring = 3;
+    if ((uint64_t)n_trees + n_splits / 8 > kGroupWork) {
+        // workgroups a CU holds: 32 waves, and the objects' values in its LDS
+        const size_t lds = (size_t)F * kApplyObj * sizeof(float) + sizeof(uint32_t) * 2 * kApplyTrees * kApplyObj;
+        const uint32_t per_cu = lds <= kApplyLdsMax + 16 * 1024 ? std::max<uint32_t>(1, std::min<uint32_t>(4, 160 * 1024 / lds)) : 4u;
+        const uint64_t wgs = p.chunk / kApplyObj;
+        p.group = (uint32_t)std::min<uint64_t>({std::max<uint64_t>(1, (uint64_t)cus * per_cu / wgs), kGroupMax, p.n_chunks});
+        if (p.group > 1) p.ring = (uint32_t)std::min<uint64_t>(2, (p.n_chunks + p.group - 1) / p.group);
+    }
+    return p;
+}
 int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, uint32_t K, const Model& M, size_t dev_x,
-                 size_t pin_x, uint64_t chunk, double* d_out) {
-    const uint64_t n_chunks = (n + chunk - 1) / chunk;
-    const size_t cbytes = align256(sizeof(float) * chunk * F);
+                 size_t pin_x, const ChunkPlan& p, double* d_out) {
+    const uint64_t chunk = p.chunk, n_chunks = p.n_chunks;
+    const size_t cbytes = p.cbytes;
     for (auto& e : w.ev)
         if (!e) APPLY_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (!w.copy) APPLY_TRY(hipStreamCreateWithFlags(&w.copy, hipStreamNonBlocking));
@@ -348,16 +400,24 @@ int apply_chunks(Workspace& w, const float* features, uint64_t n, uint32_t F, ui
     for (uint64_t c = 0; c < n_chunks && rc == CBH_OK; ++c) {
         threads.wait(c);
         const uint64_t o0 = c * chunk, m = std::min(chunk, n - o0);
-        const size_t b = (c % 3) * cbytes;
-        float* dx = (float*)(w.dev + dev_x + b);
-        hipEvent_t up = w.ev[c % 3], read = w.ev[3 + c % 3];
-        if ((c >= 3 && hipStreamWaitEvent(w.copy, read, 0) != hipSuccess) ||   // chunk c - 3's kernel
-            hipMemcpyAsync(dx, w.pin + pin_x + b, sizeof(float) * m * F, hipMemcpyHostToDevice, w.copy) != hipSuccess ||
-            hipEventRecord(up, w.copy) != hipSuccess || hipStreamWaitEvent(w.stream, up, 0) != hipSuccess)
+        const uint64_t grp = c / p.group, slot = grp % p.ring, in = c - grp * p.group;   // its place on the device
+        float* dx = (float*)(w.dev + dev_x + slot * p.group * cbytes);
+        hipEvent_t up = w.ev[c % 3], read = w.ev[3 + slot];
+        if ((in == 0 && grp >= p.ring && hipStreamWaitEvent(w.copy, read, 0) != hipSuccess) ||   // the slot's last kernel
+            hipMemcpyAsync((unsigned char*)dx + in * cbytes, w.pin + pin_x + (c % 3) * cbytes, sizeof(float) * m * F,
+                           hipMemcpyHostToDevice, w.copy) != hipSuccess ||
+            hipEventRecord(up, w.copy) != hipSuccess)
             rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
-        if (rc == CBH_OK) rc = launch_k(K, dx, m, m, M, d_out + o0, n, w.stream);
-        if (rc == CBH_OK && hipEventRecord(read, w.stream) != hipSuccess)
-            rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+        if (rc == CBH_OK && (in + 1 == p.group || c + 1 == n_chunks)) {   // the group is on its way
+            const uint64_t g0 = grp * p.group * chunk;
+            if (hipStreamWaitEvent(w.stream, up, 0) != hipSuccess)
+                rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+            if (rc == CBH_OK)
+                rc = launch_k(K, Table{dx, m, in ? (uint32_t)chunk : 0u, cbytes / sizeof(float)}, o0 + m - g0, M,
+                              d_out + g0, n, w.stream);
+            if (rc == CBH_OK && hipEventRecord(read, w.stream) != hipSuccess)
+                rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
+        }
         if (rc == CBH_OK && c + 2 < n_chunks) {   // chunk c + 2 takes the buffer of chunk c - 1
             if (c >= 1 && hipEventSynchronize(w.ev[(c - 1) % 3]) != hipSuccess)
                 rc = cbh_internal_fail(CBH_ERR_DEVICE, "table upload failed");
@@ -412,17 +472,18 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
     // them would take longer than the runtime's copy)
     const bool big = x_bytes > 2 * kChunkBytes, chunked = big && kChunkBytes / (sizeof(float) * F) >= 64;
     const bool pin_table = !big, pin_lv = sizeof(double) * n_leaves * K <= kPinModel;
-    const uint64_t chunk = chunked ? kChunkBytes / (sizeof(float) * F) / 64 * 64 : n;
-    const size_t x_dev = chunked ? 3 * align256(sizeof(float) * chunk * F) : align256(x_bytes);
-    const size_t o_out = o_x + x_dev;
-    int dev = 0;
+    int dev = 0, cus = 0;
     APPLY_TRY(hipGetDevice(&dev));
+    if (chunked) APPLY_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const ChunkPlan plan = chunked ? plan_chunks(n, F, n_trees, n_splits, (uint32_t)cus) : ChunkPlan{};
+    const size_t x_dev = chunked ? plan.ring * plan.group * plan.cbytes : align256(x_bytes);
+    const size_t o_out = o_x + x_dev;
     Lease L(dev);
     Workspace& w = L.ws;
     const bool pin_out = out_bytes <= ((size_t)4 << 20);   // the kernel's results through pinned memory
     // the pinned block: the model's arrays and a small table laid out as on the device, so that they
     // go up in one copy, or the chunk buffers, then the results
-    const size_t h_x = pin_lv ? o_x : o_lv, h_out = h_x + (chunked || pin_table ? x_dev : 0);
+    const size_t h_x = pin_lv ? o_x : o_lv, h_out = h_x + (chunked ? 3 * plan.cbytes : pin_table ? x_dev : 0);
     int rc = w.grow(o_out + out_bytes, h_out + (pin_out ? out_bytes : 0));
     if (rc != CBH_OK) return rc;
     unsigned char* h = w.pin;
@@ -450,12 +511,12 @@ extern "C" int cbh_apply_oblivious(const float* features_fm, uint64_t n_objects,
                                  hipMemcpyHostToDevice, w.stream));
     if (chunked) {
         try {
-            rc = apply_chunks(w, features_fm, n, F, K, M, o_x, h_x, chunk, d_out);
+            rc = apply_chunks(w, features_fm, n, F, K, M, o_x, h_x, plan, d_out);
         } catch (const std::exception& e) {   // (its threads are joined)
             rc = cbh_internal_fail(CBH_ERR_DEVICE, std::string("table upload: ") + e.what());
         }
     } else {
-        rc = launch_k(K, (const float*)(w.dev + o_x), n, n, M, d_out, n, w.stream);
+        rc = launch_k(K, Table{(const float*)(w.dev + o_x), n, 0, 0}, n, M, d_out, n, w.stream);
     }
     if (rc != CBH_OK) return rc;
     if (pin_out) {

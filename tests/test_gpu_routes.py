@@ -139,3 +139,47 @@ def test_predictions_past_the_kept_sizes():
     assert one(9_000_001) and one(100)
     with ThreadPoolExecutor(3) as ex:
         assert all(ex.map(one, [9_000_001, 63, 4_000_000, 1, 8_500_000, 70_000] * 2))
+
+
+@pytest.mark.parametrize("n,T", [(2_100_000, 3), (3_900_001, 3), (5_600_000, 700)])
+def test_predictions_of_chunked_tables(n, T):
+    """A table in two, three and four chunks of 1.57M objects, their kernels on three streams: every chunk
+    sees the whole model and the results wait for every chunk, also where the kernels (700 trees) take
+    longer than the uploads.  One feature, so a tree's leaf follows from the value's place between
+    its borders; the sums are in tree order, equal bit by bit."""
+    g = np.random.default_rng(T)
+    x = g.standard_normal((1, n), dtype=np.float32)
+    sb = np.sort(g.standard_normal((T, 2)).astype(np.float32).astype(np.float64), axis=1).reshape(-1)
+    sf = np.zeros(2 * T, np.uint32)
+    so, lo = np.arange(0, 2 * T + 1, 2, dtype=np.uint32), np.arange(0, 4 * T + 1, 4, dtype=np.uint32)
+    lv = g.standard_normal(4 * T)
+    rows = np.unique(np.concatenate([g.integers(0, n, 60_000), np.arange(64), n - 1 - np.arange(64)])) if T > 100 else np.arange(n)
+    v = x[0, rows].astype(np.float64)
+    for _ in range(2):
+        got = np.asarray(cb.apply_oblivious(x, sf, sb, so, lv, lo, approx_dim=1)).reshape(-1)
+        exp = np.zeros(len(rows))
+        for t in range(T):
+            exp += lv[4 * t + (v > sb[2 * t]).astype(np.int64) + 2 * (v > sb[2 * t + 1])]
+        assert np.array_equal(got[rows], exp)
+
+
+@pytest.mark.parametrize("n,F,T", [(3_900_001, 1, 3), (100_001, 100, 3), (100_001, 100, 900), (94_080, 100, 900),
+                                   (40_001, 600, 900), (31_361, 250, 900)])
+def test_predictions_of_chunked_tables(n, F, T):
+    """Tables in pinned chunks of 6 MB: a launch a chunk at small models, one launch over several chunks at
+    large ones (three of 100 features, ten of 600 whose values are read through the caches, two of 250),
+    with a last group of one chunk, a last chunk of one object, or none left over, and device buffers
+    that are used again.  Sums in tree order, equal bit by bit."""
+    g = np.random.default_rng(n)
+    x = g.standard_normal((F, n), dtype=np.float32)
+    sf = g.integers(0, F, 2 * T).astype(np.uint32)
+    sb = g.standard_normal(2 * T).astype(np.float32).astype(np.float64)
+    so, lo = np.arange(0, 2 * T + 1, 2, dtype=np.uint32), np.arange(0, 4 * T + 1, 4, dtype=np.uint32)
+    lv = g.standard_normal(4 * T)
+    exp = np.zeros(n)
+    for t in range(T):
+        a, b = 2 * t, 2 * t + 1
+        exp += lv[4 * t + (x[sf[a]] > sb[a]).astype(np.int64) + 2 * (x[sf[b]] > sb[b])]
+    for _ in range(2):
+        got = np.asarray(cb.apply_oblivious(x, sf, sb, so, lv, lo, approx_dim=1)).reshape(-1)
+        assert np.array_equal(got, exp)
