@@ -1607,8 +1607,8 @@ static __global__ __launch_bounds__(kExThreads) void fill_exact_kernel(
 // width times a constant.  These tiles flush a quarter of what the 32-feature tiles do for the
 // same atomics (tiles of 16 features measured 3-8% slower a tree); they read a row's statistics
 // once per 8 features, which costs at many rows and features (narrow_pays).
-// 100k x 50, 129 bins: 22 -> 9 us dense, 15 -> 9 us gathered; 300k x 60, 128 bins, 6 channels: 43
-// (one atomic per channel over feature-major LDS) -> 21 us.
+// Kernel trace: 100k x 50, 129 bins: 22.0 -> 11.8 us dense, 14.8-16.6 -> 9.3-12.6 us gathered; 300k x 60, 128
+// bins, 6 channels: 69 (one atomic per channel over feature-major LDS) -> 34 us dense, 34-43 -> 21-28 us.
 //
 // LDS [bin][ch][16] of u64.  A 16-lane DPP row takes 8 rows a pass, lane 2 j + w word w of row j;
 // the 16 positions it covers in a block of 1024 are staged one per lane (the channels' f64
@@ -2722,8 +2722,8 @@ __global__ __launch_bounds__(64 * NW) void score_kernel(
 // feature (n_parts workgroups a feature).  The raw rows of its features become the prefix rows of
 // the built children and their siblings (as hist_prefix_kernel; a slice's workgroup scans the
 // whole row and writes its own slice), and its borders are scored from the copy it keeps in LDS.
-// As two launches the finishing cost 5-8 us a level of launch and memory latency, and the
-// scorer as much again to read the rows back.
+// Kernel trace, levels of 1 to 32 parents, finishing + scoring as two launches against this one: 100k x 50,
+// 129 bins 3.7-4.0 + 5.9-13.7 -> 5.9-11.4 us; 300k x 60, 128 bins, K = 5 4.6-6.1 + 18.4-60.4 -> 6.6-27.9 us.
 //
 // What bounds it is latency: the raw rows (added by other XCDs' atomics) and the parent's take
 // 1-2 us to come, so the rows of every channel are in flight together, spread over the waves;

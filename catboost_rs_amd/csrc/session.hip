@@ -784,10 +784,13 @@ double narrow_load(const cbh_session* s) {
 // (4224) 852 / 819, 5000 x 500 x 128, 6, depth 7 (6144) 1016 / 992, 3000 x 2000 x 33, 3, depth 7 (3168)
 // 677 / 640, 30k x 2000 x 17, 8, depth 8 (8704) 1815 / 1622; 50k x 500 x 128, 6, depth 7 (6144) 1120 /
 // 1215, 30k x 1000 x 65, 4, depth 8 (8320) 1467 / 1540, 20k x 1000 x 65, 4, depth 7 (4160) 836 / 940.
+// PairLogitPairwise fills one channel either way: 1M x 100 x 255 3147 / 3122, x 129 2253 / 2202; 1M x 60 x
+// 33 1083 / 1081, 500k x 50 x 255 1779 / 1804, 200k x 100 x 33 973 / 1015.
 bool narrow_pays(const cbh_session* s) {
     const double n = (double)s->n, nf = n * s->F, load = narrow_load(s);
     if (s->K > 1) return load <= 2500.0 + n / 5.0;
     if (s->n < (1ull << 16)) return load <= 3500.0 + n / 25.0;
+    if (s->pairwise && s->n < (1ull << 20) && nf > 60e6) return false;
     if (s->ranking && s->n < (1ull << 20)) return nf <= 1e6 * (51.0 + 0.615 * s->B) && load <= 3500.0 + n / 25.0;
     if (s->n >= (1ull << 22)) return nf <= 1e6 * (51.0 + 0.615 * s->B);
     return nf <= 1e6 * (46.0 + 0.6 * s->B) * (1.0 - load / 30000.0);

@@ -867,8 +867,8 @@ def test_fill_layouts_ragged_shapes_match_oracle(layout, F, B, K, monkeypatch):
 def test_config3_reduced_matches_oracle(loss, fill, monkeypatch):
     """Config 3 shape (groups of 20, ~10 pairs per group, 100 features, 254 borders, depth 6);
     PairLogit also through the packed fill (its weight channel holds the pairwise weights);
-    PairLogitPairwise through the generic fill of its der channel alone (auto, below 2^20 rows)
-    and through the tiled exact fill (both channels, its default from 2^20 rows)."""
+    PairLogitPairwise through the fill of its der channel alone that a session of this size takes (auto:
+    the narrow tiles) and through the tiled exact fill (both channels)."""
     if fill != "auto":
         monkeypatch.setenv("CBH_FILL", fill)
     d = datagen.config3(n_rows=20_000 if loss == "PairLogit" else 4_000, loss=loss)
