@@ -354,7 +354,7 @@ constexpr size_t kChunkBytes = (size_t)6 << 20;   // of a table in pinned chunks
 // three groups in flight, else as many as fill the CUs, two groups in flight.  A chunk of 100 features is
 // 245 workgroups, one a CU and bound by the latency of its trees (0.2 us each up to 8 splits): a
 // launch a chunk fell behind the uploads at large models, and behind one launch over the whole
-// table.  500k x 100, a launch a chunk / a group / one launch after the upload: 500 trees 4.6 / - / 9.5 ms,
+// table.  500k x 100, a launch a chunk / a group / one launch after the upload: 500 trees 4.6 / 4.6 / 9.5 ms,
 // 1000 6.9 / 4.9 / 11.0, 5000 30.3 / 16.6 / 23.8; 300k x 300, 3000 trees of depth 8 38.5 / 13.9 / 27.0.
 // (The three buffers' kernels on streams of their own gave the same where the streams had hardware
 // queues of their own, and nothing where they had not.)
