@@ -11,7 +11,9 @@
 //   leaf   u16 [n]         leaf index, bit 15 set for rows outside the score sample
 //   idx    u32 [<= n]      row ids of the directly built children, grouped by parent leaf,
 //                          ascending row order inside each group (stable partition)
-//   hist   i64 [2^l][K+1][F][B]  exact fixed-point histograms of level l (channel planes)
+//   raw    i64 [2^(l-1)][K+1][F][B]  the fill's sums of level l's directly built children, cleared by
+//                          their reader (channel planes)
+//   hist   i64 [2^l][K+1][F][B]  exact fixed-point histograms of level l, prefix sums over bins
 #pragma once
 #include <algorithm>
 
@@ -236,7 +238,7 @@ __device__ __forceinline__ void sample_row(const SampleParams& smp, const JumpTa
 // ---------------------------------------------------------------------------------
 // Per-tree preparation: apply the previous tree (approx += lr * leaf), derivatives,
 // bootstrap sample, score channels, leaf flags, and per-block partial bounds for the
-// fixed-point scales (summed deterministically by scales_kernel).
+// fixed-point scales (summed deterministically by wave_scales).
 // ---------------------------------------------------------------------------------
 constexpr int kPrepBlocks = 2048;
 constexpr int kPartials = 8;   // per slot: 4 bounds, sampled rows, 2 maxima, 1 spare
@@ -499,7 +501,7 @@ static __global__ void quantize_stats_kernel(double* __restrict__ sstat, uint64_
 // ---------------------------------------------------------------------------------
 // Histogram fill.  One workgroup = (feature tile, row range); it accumulates
 // round(v * 2^S) of its rows into an LDS histogram of its feature tile with 64-bit integer
-// LDS atomics, then flushes non-zero cells into the level histogram with 64-bit global
+// LDS atomics, then flushes non-zero cells into the level's raw rows with 64-bit global
 // atomics (integer adds: any order gives the same bits).  The blockIdx -> (tile, range)
 // map keeps all tiles of a range on one XCD (blocks are dealt to the 8 XCDs round-robin),
 // so the rows a range reads are fetched into that XCD's L2 once and shared by its tiles.
@@ -728,7 +730,7 @@ static __global__ __launch_bounds__(1024) void fill_kernel(
 // kPackIterRows rows; atomics of threads already in the next period may land before the swap,
 // so at most R = 2 * swap_every * kPackIterRows rows fall between two swaps of a cell, and
 // pack_bits = 31 - log2(R) keeps every field sum within R * (2^pack_bits - 1) < 2^31.  The
-// swapped words are decoded into int64 registers, which flush to the level histogram at
+// swapped words are decoded into int64 registers, which flush to the level's raw rows at
 // segment ends.  Every sum stays an exact integer (order-free, reproducible); only the per-row
 // quantization step is coarser than the two-atomic fill's (2^-pack_bits of the largest row
 // instead of 2^-61 of the sum).
@@ -1194,7 +1196,7 @@ static __global__ __launch_bounds__(kPackThreads) void fill_packed_kernel(
 // (round(v * 2^S), S = 61 - ceil(log2 sum|v|) per channel, 2^-37 at config 2), one 64-bit LDS
 // atomic per (row, feature, channel).  The LDS cells are exact int64 sums: nothing is rounded
 // beyond the per-row quantization, no cell is swapped, and the tile flushes straight from LDS to
-// the level histogram at segment ends.
+// the level's raw rows at segment ends.
 //
 // Tiles of 32 features (8 words); LDS [bin][ch][32] of u64, 512 bytes per bin, the weight cell
 // of a column 256 bytes past its der cell (one immediate offset apart).  A 16-lane DPP row
@@ -1798,7 +1800,7 @@ static __global__ __launch_bounds__(kNtThreads) void fill_narrow_kernel(
 // kPkkSwapBlocks blocks of kPkkBlockRows rows; atomics of threads already in the next period
 // may land before the swap, so at most R = 2 * kPkkSwapBlocks * kPkkBlockRows rows fall between
 // two swaps of a cell and R * (2^kPkkBits - 1) < 2^31.  The swapped fields are added to int64
-// registers, flushed to the level histogram at segment ends: every sum is an exact integer of
+// registers, flushed to the level's raw rows at segment ends: every sum is an exact integer of
 // the rounded rows (order-free, reproducible).  Tiles of 32 features (8 words), LDS
 // [plane][bin][32] with the two-channel bin-major fill's rotated visits (any 16 consecutive
 // lanes hit 16 distinct features mod 16: distinct bank pairs whatever the bins), 8 lanes per
@@ -1969,7 +1971,7 @@ static __global__ __launch_bounds__(kPkkThreads) void fill_pkk_kernel(
             // every contribution of the segment is in the registers now: flush each plane's two
             // channels (stage the registers in the cells, then write the non-zero cells).  A segment
             // that lies wholly in this workgroup's range is this tile's only writer of its rows: its
-            // cells are stored (the level histogram starts zeroed); a segment shared with the
+            // cells are stored (the raw rows start zeroed); a segment shared with the
             // neighbouring range is added with global atomics
             const bool owned = pos == seg_lo && end == seg_end;
             long long* hd = hist + (size_t)slot * C * F * B;

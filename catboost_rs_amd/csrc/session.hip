@@ -1704,10 +1704,6 @@ int ctr_level_weights_dev(cbh_session* s, uint32_t level) {
     return CBH_OK;
 }
 
-// Every launch of one tree on the session stream, ending with the copies of its results
-// into pinned staging.  No host decision happens between launches (the split, partition
-// plan and leaf values stay on the device), so the sequence can be recorded once as a graph
-// and replayed for every later tree.
 // 64-bit LDS atomics a (row, feature) entry of the level's fill issues: one per channel (generic
 // and tiled exact fills), one (rounded packed and count-packed fills), one per plane of two
 // channels (packed multi-channel fills; the weight's plane left out at level 0 once it is cached).
@@ -1759,6 +1755,10 @@ int enqueue_prepare(cbh_session* s, const SampleParams& smp, bool use_host_sampl
     return s->stage_end();
 }
 
+// Every launch of one tree after its prepare on the session stream, ending with the kernel that writes
+// its results to pinned memory.  No host decision happens between launches (the split, partition
+// plan and leaf values stay on the device), so the sequence can be recorded once as a graph
+// and replayed for every later tree.
 template <int K>
 int enqueue_tree(cbh_session* s) {
     constexpr int C = K + 1;
